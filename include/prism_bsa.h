@@ -349,6 +349,50 @@ int prism_bsa_fwd_quad(const void* q, const void* k, const void* v, int BH, int6
                        const int32_t* quadmap, const int32_t* order, float sm_scale, void* o, float* lse,
                        int32_t* work_counter, hipStream_t stream);
 
+/* prism_bsa_fwd for launches of few pairs (no counterpart in the reference):
+ * one workgroup per query tile, the same outputs bit for bit.  ustart / ulen /
+ * ucols: the rows of prism_tile_lists, one per query tile (BH * Sq/64), in the
+ * entry format of prism_pair_union with the tile's own member bit (bit
+ * row % 2). */
+int prism_tile_lists(const int64_t* start, const int32_t* len, const int32_t* cols, int64_t rows, int64_t row_tiles,
+                     int64_t col_tiles, const uint64_t* tile_masks, int64_t ucap, int64_t* ustart, int32_t* ulen,
+                     int32_t* ucols, hipStream_t stream);
+int prism_bsa_fwd_tile(const void* q, const void* k, const void* v, int BH, int64_t Sq, int64_t Sk, int D,
+                       const uint64_t* tile_masks, const int64_t* ustart, const int32_t* ulen, const int32_t* ucols,
+                       float sm_scale, void* o, float* lse, hipStream_t stream);
+
+/* Split launches (no counterpart in the reference): prism_bsa_bwd_dq and
+ * prism_bsa_bwd_dkdv for launches whose pairs do not fill the GPU evenly.
+ * Pairs [0, whole) keep one work item each; every later pair is `splits`
+ * items, item i of which walks its listed tiles t with (t / 8) mod splits ==
+ * i; a second kernel adds the items' float32 results in item order:
+ * deterministic; the order of summation, and so the last bits, differ from the
+ * unsplit entry points'.  With n = whole + (pairs - whole) * splits items,
+ * ustart / ulen / ucols are prism_part_union's n rows (entries as
+ * prism_pair_union's) and order (or NULL) is a permutation of [0, n).
+ * prism_split_plan chooses whole and splits on the host for `heads` x
+ * pairs_per_head pairs (Sq/128 per head; for dK/dV Sk/128) whose lists hold up
+ * to max_entries entries (Sk/64; for dK/dV Sq/64); kernel: 1 dQ, 2 dK/dV.
+ * part_acc: workspace of (pairs - whole) * splits * 128 * D floats (dK/dV:
+ * twice that), 16-byte aligned; NULL when whole == pairs.  work_counter as for
+ * prism_bsa_fwd, not NULL.  The other arguments as for the unsplit entry
+ * points. */
+int prism_split_plan(int kernel, int64_t heads, int64_t pairs_per_head, int64_t max_entries, int D, int64_t* whole,
+                     int* splits);
+int prism_part_union(const int64_t* start, const int32_t* len, const int32_t* cols, int64_t rows, int64_t row_tiles,
+                     int64_t col_tiles, const int32_t* pairmap, const uint64_t* tile_masks, int64_t whole, int splits,
+                     int64_t ucap, int64_t* ustart, int32_t* ulen, int32_t* ucols, hipStream_t stream);
+int prism_bsa_bwd_dkdv_split(const void* q, const void* k, const void* v, const void* do_, const float* m2,
+                             const float* delta, int BH, int64_t Sq, int64_t Sk, int D, const uint8_t* kv_valid,
+                             const int64_t* ustart, const int32_t* ulen, const int32_t* ucols, const int32_t* pairmap,
+                             const int32_t* order, float sm_scale, void* dk, void* dv, int32_t* work_counter,
+                             int64_t whole, int splits, float* part_acc, hipStream_t stream);
+int prism_bsa_bwd_dq_split(const void* q, const void* k, const void* v, const void* do_, const float* m2,
+                           const float* delta, int BH, int64_t Sq, int64_t Sk, int D, const uint64_t* tile_masks,
+                           const int64_t* ustart, const int32_t* ulen, const int32_t* ucols, const int32_t* pairmap,
+                           const int32_t* order, float sm_scale, void* dq, int32_t* work_counter, int64_t whole,
+                           int splits, float* part_acc, hipStream_t stream);
+
 /* _attn_bwd_preprocess (common.py:110-127): delta[r] = sum_d o[r][d] * do[r][d]
  * over rows of bf16 [rows, D] tensors; fp32 out. */
 int prism_bwd_preprocess(const void* o, const void* do_, int64_t rows, int D, float* delta, hipStream_t stream);

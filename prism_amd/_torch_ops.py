@@ -210,3 +210,27 @@ def _register_fakes():
     @reg("prism::bsa_bwd_dq_quad")
     def _(q, k, v, do, m2, delta, tile_masks, ustart, ulen, ucols, quadmap, order, sm_scale):
         return _empty(q, q.shape, q.dtype)
+
+    @reg("prism::bsa_fwd_tile")
+    def _(q, k, v, tile_masks, ustart, ulen, ucols, sm_scale):
+        return _empty(q, q.shape, q.dtype), _empty(q, q.shape[:3], f32)
+
+    @reg("prism::bsa_bwd_dkdv_split")
+    def _(q, k, v, do, m2, delta, kv_valid, ustart, ulen, ucols, pairmap, order, sm_scale, whole, splits):
+        return _empty(k, k.shape, k.dtype), _empty(v, v.shape, v.dtype)
+
+    @reg("prism::bsa_bwd_dq_split")
+    def _(q, k, v, do, m2, delta, tile_masks, ustart, ulen, ucols, pairmap, order, sm_scale, whole, splits):
+        return _empty(q, q.shape, q.dtype)
+
+    @reg("prism::part_union")
+    def _(start, length, cols, row_tiles, col_tiles, pairmap, tile_masks, whole, splits):
+        items = whole + (start.numel() // 2 - whole) * splits
+        return (_empty(start, (items,), i64), _empty(start, (items,), i32),
+                _empty(start, (max(items * col_tiles, 1),), i32))
+
+    @reg("prism::tile_lists")
+    def _(start, length, cols, row_tiles, col_tiles, tile_masks):
+        rows = start.numel()
+        return (_empty(start, (rows,), i64), _empty(start, (rows,), i32),
+                _empty(start, (max(rows * col_tiles, 1),), i32))

@@ -84,6 +84,13 @@ def attn_fwd_bsa_varlen(q, k, v, sm_scale, block_indices, block_indices_lens, ch
     qstart, qlen, qcols = _lists_from_dense(block_indices, block_indices_lens)
     Ntq, Ntk = q.shape[2] // 64, k.shape[2] // 64
     tm = ops.tile_masks(ops._u8(kv_valid_mask))
+    pairs = q.shape[0] * q.shape[1] * Ntq // 2
+    if pairs <= ops.TILE_PAIRS:
+        return ops.bsa_fwd_tile(q, k, v, tm, ops.tile_lists(qstart, qlen, qcols, Ntq, tm, Ntk), sm_scale)
+    if pairs < ops.SPLIT_PAIRS:
+        qpair = ops.pair_tiles(qstart, qlen, qcols, Ntq, Ntk)
+        qunion = ops.pair_union(qstart, qlen, qcols, Ntq, tm, col_tiles=Ntk, pairmap=qpair)
+        return ops.bsa_fwd(q, k, v, tm, qunion, sm_scale, qpair, ops.items_order(qunion[1], 64))
     if ops.QUADS and Ntq % 4 == 0:
         # four query tiles per staged K / V tile (two overlap pairs of each
         # group of 8), the same outputs bit for bit
@@ -123,10 +130,19 @@ def attn_bwd_bsa_varlen(do, q, k, v, o, dq, dk, dv, sm_scale, lse, block_indices
     klists = ops.transpose_lists(qstart, qlen, qcols, B * H, Ntq, Ntk)
     kv = ops._u8(kv_valid_mask)
     tm = ops.tile_masks(kv)
-    qunion = ops.pair_union(qstart, qlen, qcols, Ntq, tm, col_tiles=Ntk)
-    kunion = ops.pair_union(*klists, Ntk, None, col_tiles=Ntq)
+    BH = B * H
+    qsplit, ksplit = ops.split_plan(1, BH, Ntq // 2, Ntk, D), ops.split_plan(2, BH, Ntk // 2, Ntq, D)
+    if qsplit[1] > 1:
+        qunion = ops.part_union(qstart, qlen, qcols, Ntq, *qsplit, tm, col_tiles=Ntk)
+    else:
+        qunion, qsplit = ops.pair_union(qstart, qlen, qcols, Ntq, tm, col_tiles=Ntk), None
+    if ksplit[1] > 1:
+        kunion = ops.part_union(*klists, Ntk, *ksplit, None, col_tiles=Ntq)
+    else:
+        kunion, ksplit = ops.pair_union(*klists, Ntk, None, col_tiles=Ntq), None
     m2 = ops.lse_to_m2(lse)
-    g_q, g_k, g_v = ops.bsa_bwd(q, k, v, do, m2, delta, kv, tm, qunion, kunion, sm_scale)
+    g_q, g_k, g_v = ops.bsa_bwd(q, k, v, do, m2, delta, kv, tm, qunion, kunion, sm_scale, q_split=qsplit,
+                                k_split=ksplit)
     dq.copy_(g_q)
     dk.copy_(g_k)
     dv.copy_(g_v)

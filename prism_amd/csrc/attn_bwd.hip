@@ -48,6 +48,7 @@
 
 #include "common.h"
 #include "mfma.h"
+#include "split.h"
 #include "tile_dma.h"
 #include "validate.h"
 
@@ -70,6 +71,7 @@ struct BwdArgs {
   uint16_t *dq, *dk, *dv;
   int total;                // pairs of the launch (BH * npairs)
   int* queue;               // work-queue counter (persistent launch), or null: one pair per workgroup
+  SplitArgs split;          // split launches only
 };
 
 constexpr float kLog2e = 1.4426950408889634f;
@@ -94,9 +96,11 @@ struct BwdTiles {
   static_assert(DKDV_LDS <= 160 * 1024 && DQ_LDS <= 160 * 1024, "LDS budget");
 };
 
-// one pair-union work list: the two key tiles of pair `logical`
-template <int D>
-__device__ __forceinline__ void bsa_bwd_dkdv_pair(const BwdArgs& a, uint8_t* smem, int logical) {
+// work list `item`: the two key tiles of pair `item`, or with SPLIT the pair
+// that split_item names (the dK and dV sums of a split pair's item go to its
+// workspace slot)
+template <int D, bool SPLIT>
+__device__ __forceinline__ void bsa_bwd_dkdv_pair(const BwdArgs& a, uint8_t* smem, int item) {
   using T = BwdTiles<D>;
   using RT = typename T::RT;
   constexpr int NS = D / 16, NDT = D / 32;
@@ -105,9 +109,10 @@ __device__ __forceinline__ void bsa_bwd_dkdv_pair(const BwdArgs& a, uint8_t* sme
   const int tid = opaque_thread_id(), lane = tid & 63, g = lane >> 5, l32 = lane & 31;
   const int w = (int)uniform_u32((uint32_t)tid >> 6);
   const int kh = w & 1, qh = (w >> 1) & 1, tk = w >> 2;
+  const int logical = SPLIT ? split_item(a.split.whole, a.split.splits, item).pair : item;
   const int bh = logical / a.npairs, pair = logical - bh * a.npairs;
-  const int32_t* U = a.ucols + a.ustart[logical];
-  const int n = a.ulen[logical];
+  const int32_t* U = a.ucols + a.ustart[item];
+  const int n = a.ulen[item];
   const int mybit = 1 << tk;
   const int64_t qoff = (int64_t)bh * a.Sq * D, koff = (int64_t)bh * a.Sk * D;
   const float* m2h = a.m2 + (int64_t)bh * a.Sq;
@@ -335,6 +340,20 @@ __device__ __forceinline__ void bsa_bwd_dkdv_pair(const BwdArgs& a, uint8_t* sme
         dk[dt][r] += red[((slot * 2 * NDT + dt) * 16 + r) * 64 + lane];
         dv[dt][r] += red[((slot * 2 * NDT + NDT + dt) * 16 + r) * 64 + lane];
       }
+      if constexpr (SPLIT) {
+        const int wslot = split_item(a.split.whole, a.split.splits, item).slot;
+        if (wslot >= 0) {
+          float4* pa = a.split.acc + ((int64_t)wslot * 4 + slot) * 2 * NDT * 256 + lane;
+#pragma unroll
+          for (int jj = 0; jj < 4; ++jj) {
+            pa[(dt * 4 + jj) * 64] =
+                make_float4(dk[dt][4 * jj], dk[dt][4 * jj + 1], dk[dt][4 * jj + 2], dk[dt][4 * jj + 3]);
+            pa[((NDT + dt) * 4 + jj) * 64] =
+                make_float4(dv[dt][4 * jj], dv[dt][4 * jj + 1], dv[dt][4 * jj + 2], dv[dt][4 * jj + 3]);
+          }
+          continue;
+        }
+      }
 #pragma unroll
       for (int jj = 0; jj < 4; ++jj) {
         uint2 o;
@@ -361,13 +380,15 @@ __global__ __launch_bounds__(512, 1) void bsa_bwd_dkdv_kernel(BwdArgs a) {
   for (int pid = a.queue ? work_queue_take(a.queue, a.total, &wq) : (int)blockIdx.x; pid >= 0;
        pid = a.queue ? work_queue_take(a.queue, a.total, &wq) : -1) {
     const BwdArgs ap = kernel_args<BwdArgs>();
-    bsa_bwd_dkdv_pair<D>(ap, smem, a.order ? a.order[pid] : xcd_group_remap<32>(pid, a.total));
+    bsa_bwd_dkdv_pair<D, false>(ap, smem, a.order ? a.order[pid] : xcd_group_remap<32>(pid, a.total));
   }
 }
 
-// one pair-union work list: the two query tiles of pair `logical`
-template <int D>
-__device__ __forceinline__ void bsa_bwd_dq_pair(const BwdArgs& a, uint8_t* smem, int logical) {
+// work list `item`: the two query tiles of pair `item`, or with SPLIT the pair
+// that split_item names (the dQ sums of a split pair's item go to its
+// workspace slot)
+template <int D, bool SPLIT>
+__device__ __forceinline__ void bsa_bwd_dq_pair(const BwdArgs& a, uint8_t* smem, int item) {
   using T = BwdTiles<D>;
   using RT = typename T::RT;
   constexpr int NS = D / 16, NDT = D / 32;
@@ -377,9 +398,10 @@ __device__ __forceinline__ void bsa_bwd_dq_pair(const BwdArgs& a, uint8_t* smem,
   const int tid = opaque_thread_id(), lane = tid & 63, g = lane >> 5, l32 = lane & 31;
   const int w = (int)uniform_u32((uint32_t)tid >> 6);
   const int qh = w & 1, tq = w >> 1;
+  const int logical = SPLIT ? split_item(a.split.whole, a.split.splits, item).pair : item;
   const int bh = logical / a.npairs, pair = logical - bh * a.npairs;
-  const int32_t* U = a.ucols + a.ustart[logical];
-  const int n = a.ulen[logical];
+  const int32_t* U = a.ucols + a.ustart[item];
+  const int n = a.ulen[item];
   const int mybit = 1 << tq;
   const int64_t qoff = (int64_t)bh * a.Sq * D, koff = (int64_t)bh * a.Sk * D;
   const float NINF = -__builtin_inff();
@@ -525,6 +547,19 @@ __device__ __forceinline__ void bsa_bwd_dq_pair(const BwdArgs& a, uint8_t* smem,
     __builtin_amdgcn_s_setprio(0);
   }
 
+  if constexpr (SPLIT) {
+    const int wslot = split_item(a.split.whole, a.split.splits, item).slot;
+    if (wslot >= 0) {
+      float4* pa = a.split.acc + ((int64_t)wslot * 4 + w) * NDT * 256 + lane;
+#pragma unroll
+      for (int dt = 0; dt < NDT; ++dt)
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj)
+          pa[(dt * 4 + jj) * 64] =
+              make_float4(dq[dt][4 * jj], dq[dt][4 * jj + 1], dq[dt][4 * jj + 2], dq[dt][4 * jj + 3]);
+      return;
+    }
+  }
   uint16_t* dqr = a.dq + qoff + qrow * D;
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt)
@@ -549,7 +584,73 @@ __global__ __launch_bounds__(256, 2) void bsa_bwd_dq_kernel(BwdArgs a) {
   for (int pid = a.queue ? work_queue_take(a.queue, a.total, &wq) : (int)blockIdx.x; pid >= 0;
        pid = a.queue ? work_queue_take(a.queue, a.total, &wq) : -1) {
     const BwdArgs ap = kernel_args<BwdArgs>();
-    bsa_bwd_dq_pair<D>(ap, smem, a.order ? a.order[pid] : xcd_group_remap<64>(pid, a.total));
+    bsa_bwd_dq_pair<D, false>(ap, smem, a.order ? a.order[pid] : xcd_group_remap<64>(pid, a.total));
+  }
+}
+
+// ------------------------------------------------------------ split lists
+// dK/dV and dQ over launches that do not fill the GPU evenly (split.h): one
+// work item per list of prism_part_union, the sums of a split pair's items
+// added in item order by bsa_bwd_merge_kernel.
+template <int D>
+__global__ __launch_bounds__(512, 1) void bsa_bwd_dkdv_split_kernel(BwdArgs a) {
+  __shared__ __align__(16) uint8_t smem[BwdTiles<D>::DKDV_LDS];
+  __shared__ WorkQueueState wq;
+  work_queue_init(&wq);
+  const int items = a.split.whole + (a.total - a.split.whole) * a.split.splits;
+  for (int b = work_queue_take(a.queue, items, &wq); b >= 0; b = work_queue_take(a.queue, items, &wq)) {
+    const BwdArgs ap = kernel_args<BwdArgs>();
+    bsa_bwd_dkdv_pair<D, true>(ap, smem, ap.order ? ap.order[b] : b);
+  }
+}
+
+template <int D>
+__global__ __launch_bounds__(256, 2) void bsa_bwd_dq_split_kernel(BwdArgs a) {
+  __shared__ __align__(16) uint8_t smem[kStagesDq * BwdTiles<D>::DQ_STAGE];
+  __shared__ WorkQueueState wq;
+  work_queue_init(&wq);
+  const int items = a.split.whole + (a.total - a.split.whole) * a.split.splits;
+  for (int b = work_queue_take(a.queue, items, &wq); b >= 0; b = work_queue_take(a.queue, items, &wq)) {
+    const BwdArgs ap = kernel_args<BwdArgs>();
+    bsa_bwd_dq_pair<D, true>(ap, smem, ap.order ? ap.order[b] : b);
+  }
+}
+
+// one workgroup per split pair and 32-column block: thread = (row half, lane)
+// of the attention kernel's accumulators.  KV: blocks 0 .. NDT - 1 are dK,
+// NDT .. 2 NDT - 1 dV, rows the pair's keys; else dQ, rows its queries.
+template <int D, bool KV>
+__global__ __launch_bounds__(256) void bsa_bwd_merge_kernel(BwdArgs a) {
+  constexpr int NDT = D / 32, NB = KV ? 2 * NDT : NDT;
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, l32 = lane & 31, w = tid >> 6;
+  const int i = (int)blockIdx.x, blk = (int)blockIdx.y, S = a.split.splits;
+  const int logical = a.split.whole + i;
+  const int bh = logical / a.npairs, pair = logical - bh * a.npairs;
+  const int slot2 = 2 * pair + (w >> 1);  // (accumulator group w: 32-row half w & 1 of tile w >> 1)
+  const int tile = a.pairmap ? a.pairmap[(int64_t)bh * 2 * a.npairs + slot2] : slot2;
+  const int64_t row = (int64_t)bh * (KV ? a.Sk : a.Sq) + (int64_t)tile * 64 + 32 * (w & 1) + l32;
+  const float4* pa = a.split.acc + (((int64_t)i * S * 4 + w) * NB + blk) * 256 + lane;
+  float4 acc[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) acc[j] = pa[j * 64];
+  for (int p = 1; p < S; ++p)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float4 x = pa[(int64_t)p * 4 * NB * 256 + j * 64];
+      acc[j].x += x.x;
+      acc[j].y += x.y;
+      acc[j].z += x.z;
+      acc[j].w += x.w;
+    }
+  const bool is_dv = KV && blk >= NDT;
+  const float sc = is_dv ? 1.0f : a.sm_scale;
+  uint16_t* out = (KV ? (is_dv ? a.dv : a.dk) : a.dq) + row * D + 32 * (blk % NDT) + 4 * g;
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    uint2 o;
+    o.x = pack_bf16(acc[j].x * sc, acc[j].y * sc);
+    o.y = pack_bf16(acc[j].z * sc, acc[j].w * sc);
+    *reinterpret_cast<uint2*>(out + 8 * j) = o;
   }
 }
 
@@ -798,6 +899,16 @@ int check_common(const void* q, const void* k, int BH, int64_t Sq, int64_t Sk, i
 }
 
 
+// workgroups of the split kernels that the device holds at once
+int dq_slots(int D) {
+  return D == 128 ? resident_workgroups<bsa_bwd_dq_split_kernel<128>>(256)
+                  : resident_workgroups<bsa_bwd_dq_split_kernel<64>>(256);
+}
+int dkdv_slots(int D) {
+  return D == 128 ? resident_workgroups<bsa_bwd_dkdv_split_kernel<128>>(512)
+                  : resident_workgroups<bsa_bwd_dkdv_split_kernel<64>>(512);
+}
+
 }  // namespace
 
 extern "C" {
@@ -874,6 +985,102 @@ int prism_bsa_bwd_dq(const void* q, const void* k, const void* v, const void* do
   if (D == 128) bsa_bwd_dq_kernel<128><<<blocks, 256, 0, stream>>>(a);
   else bsa_bwd_dq_kernel<64><<<blocks, 256, 0, stream>>>(a);
   PRISM_LAUNCH_CHECK("prism_bsa_bwd_dq");
+  return PRISM_OK;
+}
+
+int prism_split_plan(int kernel, int64_t heads, int64_t pairs_per_head, int64_t max_entries, int D, int64_t* whole,
+                     int* splits) {
+  PRISM_REQUIRE(whole && splits, "prism_split_plan: null pointer");
+  PRISM_REQUIRE(kernel == 1 || kernel == 2, "prism_split_plan: kernel %d unknown (1 dQ, 2 dK/dV)", kernel);
+  PRISM_REQUIRE(D == 64 || D == 128, "prism_split_plan: head_dim %d unsupported (64, 128)", D);
+  PRISM_REQUIRE(heads >= 1 && pairs_per_head >= 1 && heads < (1ll << 31) / pairs_per_head && max_entries >= 1,
+                "prism_split_plan: bad sizes");
+  split_plan(heads, pairs_per_head, max_entries, kernel == 2 ? dkdv_slots(D) : dq_slots(D), whole, splits);
+  return PRISM_OK;
+}
+
+int prism_bsa_bwd_dkdv_split(const void* q, const void* k, const void* v, const void* do_, const float* m2,
+                             const float* delta, int BH, int64_t Sq, int64_t Sk, int D, const uint8_t* kv_valid,
+                             const int64_t* ustart, const int32_t* ulen, const int32_t* ucols, const int32_t* pairmap,
+                             const int32_t* order, float sm_scale, void* dk, void* dv, int32_t* work_counter,
+                             int64_t whole, int splits, float* part_acc, hipStream_t stream) {
+  int rc = check_common(q, k, BH, Sq, Sk, D, "prism_bsa_bwd_dkdv_split");
+  if (rc) return rc;
+  PRISM_REQUIRE(v && do_ && m2 && delta && ustart && ulen && ucols && dk && dv && work_counter,
+                "prism_bsa_bwd_dkdv_split: null pointer");
+  const int64_t total = (int64_t)BH * (Sk / 128);
+  rc = split_check("prism_bsa_bwd_dkdv_split", total, whole, splits, part_acc);
+  if (rc) return rc;
+  const int64_t items = whole + (total - whole) * splits;
+  if (prism_debug_enabled()) {
+    PRISM_DEBUG_CHECK(prism_debug_check_lists("prism_bsa_bwd_dkdv_split", ustart, ulen, ucols, items, Sq / 64, 1,
+                                              nullptr, stream));
+    PRISM_DEBUG_CHECK(
+        prism_debug_check_maps("prism_bsa_bwd_dkdv_split", pairmap, BH, Sk / 64, order, items, stream));
+  }
+  BwdArgs a = {};
+  a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v; a.do_ = (const uint16_t*)do_;
+  a.m2 = m2; a.delta = delta; a.kv_valid = kv_valid;
+  a.ustart = ustart; a.ulen = ulen; a.ucols = ucols; a.pairmap = pairmap; a.order = order; a.Sq = Sq; a.Sk = Sk;
+  a.npairs = (int)(Sk / 128);
+  a.sm_scale = sm_scale; a.scale_log2 = sm_scale * kLog2e; a.dk = (uint16_t*)dk; a.dv = (uint16_t*)dv;
+  a.total = (int)total;
+  a.queue = work_counter;
+  a.split = SplitArgs{(int)whole, splits, (float4*)part_acc};
+  zero_counter_kernel<<<1, kQueueLanes, 0, stream>>>(a.queue);
+  const int64_t res = dkdv_slots(D);
+  const unsigned blocks = (unsigned)(res < items ? res : items);
+  const dim3 merge((unsigned)(total - whole), (unsigned)(2 * D / 32));
+  if (D == 128) {
+    bsa_bwd_dkdv_split_kernel<128><<<blocks, 512, 0, stream>>>(a);
+    if (merge.x) bsa_bwd_merge_kernel<128, true><<<merge, 256, 0, stream>>>(a);
+  } else {
+    bsa_bwd_dkdv_split_kernel<64><<<blocks, 512, 0, stream>>>(a);
+    if (merge.x) bsa_bwd_merge_kernel<64, true><<<merge, 256, 0, stream>>>(a);
+  }
+  PRISM_LAUNCH_CHECK("prism_bsa_bwd_dkdv_split");
+  return PRISM_OK;
+}
+
+int prism_bsa_bwd_dq_split(const void* q, const void* k, const void* v, const void* do_, const float* m2,
+                           const float* delta, int BH, int64_t Sq, int64_t Sk, int D, const uint64_t* tile_masks,
+                           const int64_t* ustart, const int32_t* ulen, const int32_t* ucols, const int32_t* pairmap,
+                           const int32_t* order, float sm_scale, void* dq, int32_t* work_counter, int64_t whole,
+                           int splits, float* part_acc, hipStream_t stream) {
+  int rc = check_common(q, k, BH, Sq, Sk, D, "prism_bsa_bwd_dq_split");
+  if (rc) return rc;
+  PRISM_REQUIRE(v && do_ && m2 && delta && ustart && ulen && ucols && dq && work_counter,
+                "prism_bsa_bwd_dq_split: null pointer");
+  const int64_t total = (int64_t)BH * (Sq / 128);
+  rc = split_check("prism_bsa_bwd_dq_split", total, whole, splits, part_acc);
+  if (rc) return rc;
+  const int64_t items = whole + (total - whole) * splits;
+  if (prism_debug_enabled()) {
+    PRISM_DEBUG_CHECK(prism_debug_check_lists("prism_bsa_bwd_dq_split", ustart, ulen, ucols, items, Sk / 64, 1,
+                                              tile_masks, stream));
+    PRISM_DEBUG_CHECK(prism_debug_check_maps("prism_bsa_bwd_dq_split", pairmap, BH, Sq / 64, order, items, stream));
+  }
+  BwdArgs a = {};
+  a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v; a.do_ = (const uint16_t*)do_;
+  a.m2 = m2; a.delta = delta; a.tmask = tile_masks;
+  a.ustart = ustart; a.ulen = ulen; a.ucols = ucols; a.pairmap = pairmap; a.order = order; a.Sq = Sq; a.Sk = Sk;
+  a.npairs = (int)(Sq / 128);
+  a.sm_scale = sm_scale; a.scale_log2 = sm_scale * kLog2e; a.dq = (uint16_t*)dq;
+  a.total = (int)total;
+  a.queue = work_counter;
+  a.split = SplitArgs{(int)whole, splits, (float4*)part_acc};
+  zero_counter_kernel<<<1, kQueueLanes, 0, stream>>>(a.queue);
+  const int64_t res = dq_slots(D);
+  const unsigned blocks = (unsigned)(res < items ? res : items);
+  const dim3 merge((unsigned)(total - whole), (unsigned)(D / 32));
+  if (D == 128) {
+    bsa_bwd_dq_split_kernel<128><<<blocks, 256, 0, stream>>>(a);
+    if (merge.x) bsa_bwd_merge_kernel<128, false><<<merge, 256, 0, stream>>>(a);
+  } else {
+    bsa_bwd_dq_split_kernel<64><<<blocks, 256, 0, stream>>>(a);
+    if (merge.x) bsa_bwd_merge_kernel<64, false><<<merge, 256, 0, stream>>>(a);
+  }
+  PRISM_LAUNCH_CHECK("prism_bsa_bwd_dq_split");
   return PRISM_OK;
 }
 

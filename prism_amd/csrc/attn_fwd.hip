@@ -63,7 +63,8 @@ struct FwdArgs {
   int* queue;              // work-queue counter (persistent launch), or null: one pair per workgroup
 };
 
-constexpr int kStages = 2;  // two workgroups per CU: 2 x 2 stages of K and V fill the LDS
+constexpr int kStages = 2;      // two workgroups per CU: 2 x 2 stages of K and V fill the LDS
+constexpr int kStagesTile = 4;  // one workgroup per CU
 
 template <int D>
 struct FwdTiles {
@@ -73,44 +74,51 @@ struct FwdTiles {
   static_assert(STAGE_KB % 2 == 0, "stage must split evenly over 2 waves");
 };
 
-// one pair-union work list: the two query tiles of pair `logical`
-template <int D>
-__device__ __forceinline__ void bsa_fwd_pair(const FwdArgs& a, uint8_t* smem, int logical) {
+// work list `item`: the two query tiles of pair `item`; with TILE, query tile
+// item & 1 of pair item / 2 alone: its waves take the math, the other tile's
+// two waves issue the copies
+template <int D, bool TILE>
+__device__ __forceinline__ void bsa_fwd_pair(const FwdArgs& a, uint8_t* smem, int item) {
   using T = FwdTiles<D>;
   using RT = typename T::RT;
   constexpr int NS = D / 16;   // MFMA k-steps over d
   constexpr int NDT = D / 32;  // 32-row d blocks of O^T
+  constexpr int NST = TILE ? kStagesTile : kStages;
 
   const int tid = opaque_thread_id(), lane = tid & 63, g = lane >> 5, l32 = lane & 31;
   const int w = (int)uniform_u32((uint32_t)tid >> 6);
+  const int logical = TILE ? item >> 1 : item;
   const int bh = logical / a.npairs, pair = logical - bh * a.npairs;
-  const int32_t* U = a.ucols + a.ustart[logical];
-  const int n = a.ulen[logical];
+  const int32_t* U = a.ucols + a.ustart[item];
+  const int n = a.ulen[item];
   const int mybit = 1 << (w >> 1);
+  const bool mine = !TILE || (w >> 1) == (item & 1);  // this wave takes math
+  const bool copies = TILE ? !mine : w < 2;           // this wave issues copies
 
   const uint16_t* Qh = a.q + (int64_t)bh * a.Sq * D;
   const uint16_t* Kh = a.k + (int64_t)bh * a.Sk * D;
   const uint16_t* Vh = a.v + (int64_t)bh * a.Sk * D;
   const float NINF = -__builtin_inff();
 
-  // DMA plan: waves 0 and 1 issue KB-instructions w, w + 2, ... of each
-  // stage (K then V); waves 2 and 3 issue none.  A wave stalls while the
-  // CU's address path takes its copy instructions, so the two waves that
-  // issue none start their MFMAs right after the barrier (-1% against four
-  // waves issuing ten each, A/B on one box).  Instruction i + 4m of a tile
-  // reads 4096 m bytes past instruction i, so two lane offsets serve all.
+  // DMA plan: two waves (0 and 1, with TILE the idle tile's) issue
+  // KB-instructions w % 2, w % 2 + 2, ... of each stage (K then V).  A wave
+  // stalls while the CU's address path takes its copy instructions, so the
+  // two waves that issue none start their MFMAs right after the barrier (-1%
+  // against four waves issuing ten each, A/B on one box).  Instruction i + 4m
+  // of a tile reads 4096 m bytes past instruction i, so two lane offsets
+  // serve all.
   constexpr int SL2 = T::STAGE_KB / 2, NOFF = RT::KB / 4;
   static_assert(RT::KB % 4 == 0, "tile splits into fours");
   const uint32_t soff0 = RT::src_offset(w & 1, lane), soff1 = RT::src_offset((w & 1) + 2, lane);
   const uint32_t lds0 = lds_addr(smem);
   auto issue = [&](int kt, int st) {
-    if (w >= 2) return;
+    if (!copies) return;
     const char* kb = (const char*)uniform_ptr(Kh + (int64_t)kt * 64 * D);
     const char* vb = (const char*)uniform_ptr(Vh + (int64_t)kt * 64 * D);
     const uint32_t base = lds0 + (uint32_t)(st * T::STAGE);
 #pragma unroll
     for (int s = 0; s < SL2; ++s) {
-      const int i = w + 2 * s;                  // instruction of the stage
+      const int i = (w & 1) + 2 * s;            // instruction of the stage
       const int t = i < RT::KB ? i : i - RT::KB;  // instruction of its tile
       dma_b128((s & 1) ? soff1 : soff0, (i < RT::KB ? kb : vb) + 4096 * ((t >> 2) % NOFF), base + (uint32_t)i * 1024u);
     }
@@ -120,10 +128,10 @@ __device__ __forceinline__ void bsa_fwd_pair(const FwdArgs& a, uint8_t* smem, in
   TrOperand vop;
   vop.init<RT>(0, lane);
 
-  EntryRing<kStages> ring;
+  EntryRing<NST> ring;
   ring.init(U, n);
 #pragma unroll
-  for (int k = 0; k + 1 < kStages; ++k)
+  for (int k = 0; k + 1 < NST; ++k)
     if (k < n) issue(ring.e[k] >> 3, k);
 
   const int slot2 = 2 * pair + (w >> 1);
@@ -142,14 +150,14 @@ __device__ __forceinline__ void bsa_fwd_pair(const FwdArgs& a, uint8_t* smem, in
 
   int st = 0;  // stage of entry j
   for (int j = 0; j < n; ++j) {
-    const int e = ring.e[0], enext = ring.e[kStages - 1];
+    const int e = ring.e[0], enext = ring.e[NST - 1];
     ring.advance(U, n, j);
-    stage_wait<kStages, SL2>(n - 1 - j);
+    stage_wait<NST, SL2>(n - 1 - j);
     __syncthreads();
-    if (j + kStages - 1 < n) issue(enext >> 3, stage_ahead<kStages>(st));
+    if (j + NST - 1 < n) issue(enext >> 3, stage_ahead<NST>(st));
     const uint8_t* sK = smem + st * T::STAGE;
-    st = st + 1 == kStages ? 0 : st + 1;
-    if (!(e & mybit)) continue;
+    st = st + 1 == NST ? 0 : st + 1;
+    if (!mine || !(e & mybit)) continue;
 
     const uint8_t* sV = sK + RT::BYTES;
     // S^T[key][q] = K Q^T, two 32-key halves as interleaved MFMA chains; the
@@ -249,6 +257,7 @@ __device__ __forceinline__ void bsa_fwd_pair(const FwdArgs& a, uint8_t* smem, in
     __builtin_amdgcn_s_setprio(0);
   }
 
+  if (!mine) return;
   const float inv = 1.0f / l;
   uint16_t* Oq = a.o + ((int64_t)bh * a.Sq + qrow) * D;
 #pragma unroll
@@ -522,8 +531,24 @@ __global__ __launch_bounds__(256, 2) void bsa_fwd_kernel(FwdArgs a) {
   for (int pid = a.queue ? work_queue_take(a.queue, a.total, &wq) : (int)blockIdx.x; pid >= 0;
        pid = a.queue ? work_queue_take(a.queue, a.total, &wq) : -1) {
     const FwdArgs ap = kernel_args<FwdArgs>();
-    bsa_fwd_pair<D>(ap, smem, a.order ? a.order[pid] : xcd_group_remap<64>(pid, a.total));
+    bsa_fwd_pair<D, false>(ap, smem, a.order ? a.order[pid] : xcd_group_remap<64>(pid, a.total));
   }
+}
+
+// ------------------------------------------------------------ single tiles
+// Launches of at most half as many pairs as the GPU has CUs: a workgroup per
+// query tile instead of per pair, so twice as many CUs work and a tile walks
+// its own list instead of the pair's union.  Its other two waves have no math
+// and issue the copies, three entries ahead (four stages: with two workgroups
+// per pair's worth of LDS gone, the copy latency of a lone workgroup is what
+// bounds the pair kernel here).  Every row's arithmetic is the pair kernel's.
+// Measured: 160 tiles of 860 entries (80 pairs of 1,613) 1,692 -> 1,028 us, 128
+// tiles of 10 entries (D = 64) 25 -> 13 us; 320 tiles take two rounds and lose
+// (1,695 -> 2,086 us), so launches stop at one tile per CU.
+template <int D>
+__global__ __launch_bounds__(256, 1) void bsa_fwd_tile_kernel(FwdArgs a) {
+  __shared__ __align__(16) uint8_t smem[kStagesTile * FwdTiles<D>::STAGE];
+  bsa_fwd_pair<D, true>(a, smem, (int)blockIdx.x);
 }
 
 }  // namespace
@@ -562,6 +587,31 @@ int prism_bsa_fwd(const void* q, const void* k, const void* v, int BH, int64_t S
   if (D == 128) bsa_fwd_kernel<128><<<blocks, 256, 0, stream>>>(a);
   else bsa_fwd_kernel<64><<<blocks, 256, 0, stream>>>(a);
   PRISM_LAUNCH_CHECK("prism_bsa_fwd");
+  return PRISM_OK;
+}
+
+int prism_bsa_fwd_tile(const void* q, const void* k, const void* v, int BH, int64_t Sq, int64_t Sk, int D,
+                       const uint64_t* tile_masks, const int64_t* ustart, const int32_t* ulen, const int32_t* ucols,
+                       float sm_scale, void* o, float* lse, hipStream_t stream) {
+  PRISM_REQUIRE(q && k && v && ustart && ulen && ucols && o && lse, "prism_bsa_fwd_tile: null pointer");
+  PRISM_REQUIRE(D == 64 || D == 128, "prism_bsa_fwd_tile: head_dim %d unsupported (64, 128)", D);
+  PRISM_REQUIRE(Sq > 0 && Sq % 128 == 0 && Sk > 0 && Sk % 128 == 0,
+                "prism_bsa_fwd_tile: Sq and Sk must be positive multiples of 128");
+  PRISM_REQUIRE(BH >= 1 && (int64_t)BH * (Sq / 64) < (1ll << 31), "prism_bsa_fwd_tile: grid too large");
+  const int64_t tiles = (int64_t)BH * (Sq / 64);
+  if (prism_debug_enabled())
+    PRISM_DEBUG_CHECK(
+        prism_debug_check_lists("prism_bsa_fwd_tile", ustart, ulen, ucols, tiles, Sk / 64, 1, tile_masks, stream));
+  FwdArgs a = {};
+  a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v; a.tmask = tile_masks;
+  a.ustart = ustart; a.ulen = ulen; a.ucols = ucols; a.Sq = Sq; a.Sk = Sk;
+  a.npairs = (int)(Sq / 128);
+  a.scale_log2 = sm_scale * 1.4426950408889634f;
+  a.o = (uint16_t*)o; a.lse = lse;
+  a.total = (int)(tiles / 2);
+  if (D == 128) bsa_fwd_tile_kernel<128><<<(unsigned)tiles, 256, 0, stream>>>(a);
+  else bsa_fwd_tile_kernel<64><<<(unsigned)tiles, 256, 0, stream>>>(a);
+  PRISM_LAUNCH_CHECK("prism_bsa_fwd_tile");
   return PRISM_OK;
 }
 

@@ -20,28 +20,35 @@
 // prism_lists_csr_offsets / prism_lists_csr_fill turn any (start, len, cols)
 // lists into compact CSR (int32 offsets, entries stored once, O(nnz) memory).
 #include "common.h"
+#include "split.h"
 #include "validate.h"
 
 namespace {
 
 constexpr int kUnionWin = 8192;  // tiles per LDS bitmap window (256 words)
 
-// one 256-thread workgroup per group of R rows (R = 2: a pair, R = 4: a quad);
+// one 256-thread workgroup per group of R rows (R = 1: a tile, as an entry list
+// of its pair; R = 2: a pair, R = 4: a quad);
 // the group's rows are R p .. R p + R - 1 of the head, or pairmap[R p + k]
 // (row indices inside the head).  Entries: tile << (R + 1) | partial << R |
 // member bits (bit k: row k lists the tile).
-template <int R>
+// SPLIT (R = 2): row b is work item b of a split launch (split.h): a whole
+// pair, or the entries of a pair whose tile t has (t / 8) mod splits equal to
+// the item's number within its pair.
+template <int R, bool SPLIT>
 __global__ __launch_bounds__(256) void pair_union_kernel(const int64_t* __restrict__ start,
                                                     const int32_t* __restrict__ len,
                                                     const int32_t* __restrict__ cols, int64_t Nr, int64_t Nc,
                                                     const int32_t* __restrict__ pairmap,
                                                     const uint64_t* __restrict__ tile_masks, int64_t ucap,
-                                                    int64_t* __restrict__ ustart, int32_t* __restrict__ ulen,
-                                                    int32_t* __restrict__ ucols) {
+                                                    int whole, int splits, int64_t* __restrict__ ustart,
+                                                    int32_t* __restrict__ ulen, int32_t* __restrict__ ucols) {
   __shared__ uint32_t bm[R][kUnionWin / 32];
   __shared__ uint32_t wtot[4];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  const int64_t p = blockIdx.x;
+  const int64_t row = blockIdx.x;
+  const SplitItem item = SPLIT ? split_item(whole, splits, (int)row) : SplitItem{(int)row, -1};
+  const int64_t p = item.pair;
   const int64_t head0 = (R * p) / Nr * Nr;
   const int32_t* L[R];
   int nl[R];
@@ -52,7 +59,7 @@ __global__ __launch_bounds__(256) void pair_union_kernel(const int64_t* __restri
     nl[k] = len[r];
   }
   // list entries index column tiles inside one head (0 .. Nc-1), as does tile_masks
-  int32_t* out = ucols + p * ucap;
+  int32_t* out = ucols + row * ucap;
   int count = 0;
   for (int64_t w0 = 0; w0 < Nc; w0 += kUnionWin) {
 #pragma unroll
@@ -71,6 +78,14 @@ __global__ __launch_bounds__(256) void pair_union_kernel(const int64_t* __restri
       mb[k] = bm[k][tid];
       u |= mb[k];
     }
+    if (SPLIT && item.slot >= 0) {
+      // byte i of the word: tiles of group (w0 + 32 tid) / 8 + i
+      const int g0 = (int)(w0 >> 3) + 4 * tid, part = item.slot % splits;
+      uint32_t keep = 0u;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) keep |= (g0 + i) % splits == part ? 0xffu << (8 * i) : 0u;
+      u &= keep;
+    }
     const uint32_t c = __popc(u);
     const uint32_t incl = wave_incl_scan_u32(c, lane);
     if (lane == 63) wtot[w] = incl;
@@ -87,18 +102,20 @@ __global__ __launch_bounds__(256) void pair_union_kernel(const int64_t* __restri
       const int bit = __ffs(u) - 1;
       u &= u - 1;
       const int64_t tile = w0 + 32 * tid + bit;
-      int e = (int)(tile << (R + 1));
+      // (R = 1: the pair's entry format with the row's own member bit)
+      constexpr int MB = R == 1 ? 2 : R;
+      int e = (int)(tile << (MB + 1));
 #pragma unroll
-      for (int k = 0; k < R; ++k) e |= (int)(((mb[k] >> bit) & 1u) << k);
-      if (tile_masks && tile_masks[tile] != ~0ull) e |= 1 << R;
+      for (int k = 0; k < R; ++k) e |= (int)(((mb[k] >> bit) & 1u) << (R == 1 ? (int)(row & 1) : k));
+      if (tile_masks && tile_masks[tile] != ~0ull) e |= 1 << MB;
       out[pos++] = e;
     }
     count += (int)total;
     __syncthreads();
   }
   if (tid == 0) {
-    ustart[p] = p * ucap;
-    ulen[p] = count;
+    ustart[row] = row * ucap;
+    ulen[row] = count;
   }
 }
 
@@ -357,9 +374,55 @@ int prism_pair_union(const int64_t* start, const int32_t* len, const int32_t* co
     PRISM_DEBUG_CHECK(prism_debug_check_maps("prism_pair_union", pairmap, rows / row_tiles, row_tiles, nullptr, 0,
                                              stream));
   }
-  pair_union_kernel<2><<<(unsigned)pairs, 256, 0, stream>>>(start, len, cols, row_tiles, col_tiles, pairmap, tile_masks,
-                                                             ucap, ustart, ulen, ucols);
+  pair_union_kernel<2, false><<<(unsigned)pairs, 256, 0, stream>>>(start, len, cols, row_tiles, col_tiles, pairmap,
+                                                                    tile_masks, ucap, 0, 1, ustart, ulen, ucols);
   PRISM_LAUNCH_CHECK("prism_pair_union");
+  return PRISM_OK;
+}
+
+int prism_part_union(const int64_t* start, const int32_t* len, const int32_t* cols, int64_t rows, int64_t row_tiles,
+                     int64_t col_tiles, const int32_t* pairmap, const uint64_t* tile_masks, int64_t whole, int splits,
+                     int64_t ucap, int64_t* ustart, int32_t* ulen, int32_t* ucols, hipStream_t stream) {
+  PRISM_REQUIRE(start && len && cols && ustart && ulen && ucols, "prism_part_union: null pointer");
+  PRISM_REQUIRE(rows >= 0 && rows % 2 == 0, "prism_part_union: rows must be even (pairs of tiles)");
+  PRISM_REQUIRE(row_tiles > 0 && row_tiles % 2 == 0 && rows % row_tiles == 0,
+                "prism_part_union: rows must be a multiple of an even row_tiles (tiles per head)");
+  PRISM_REQUIRE(col_tiles > 0 && col_tiles < (1ll << 28), "prism_part_union: col_tiles out of range");
+  PRISM_REQUIRE(ucap >= col_tiles, "prism_part_union: ucap must be >= col_tiles");
+  const int64_t pairs = rows / 2;
+  if (pairs == 0) return PRISM_OK;
+  const int rc = split_check("prism_part_union", pairs, whole, splits, ucols);
+  if (rc) return rc;
+  const int64_t items = whole + (pairs - whole) * splits;
+  if (prism_debug_enabled()) {
+    PRISM_DEBUG_CHECK(prism_debug_check_lists("prism_part_union", start, len, cols, rows, col_tiles, 0, nullptr,
+                                              stream));
+    PRISM_DEBUG_CHECK(prism_debug_check_maps("prism_part_union", pairmap, rows / row_tiles, row_tiles, nullptr, 0,
+                                             stream));
+  }
+  pair_union_kernel<2, true><<<(unsigned)items, 256, 0, stream>>>(start, len, cols, row_tiles, col_tiles, pairmap,
+                                                                   tile_masks, ucap, (int)whole, splits, ustart, ulen,
+                                                                   ucols);
+  PRISM_LAUNCH_CHECK("prism_part_union");
+  return PRISM_OK;
+}
+
+int prism_tile_lists(const int64_t* start, const int32_t* len, const int32_t* cols, int64_t rows, int64_t row_tiles,
+                     int64_t col_tiles, const uint64_t* tile_masks, int64_t ucap, int64_t* ustart, int32_t* ulen,
+                     int32_t* ucols, hipStream_t stream) {
+  PRISM_REQUIRE(start && len && cols && ustart && ulen && ucols, "prism_tile_lists: null pointer");
+  PRISM_REQUIRE(rows >= 0 && row_tiles > 0 && row_tiles % 2 == 0 && rows % row_tiles == 0,
+                "prism_tile_lists: rows must be a multiple of an even row_tiles (tiles per head)");
+  PRISM_REQUIRE(col_tiles > 0 && col_tiles < (1ll << 28), "prism_tile_lists: col_tiles out of range");
+  PRISM_REQUIRE(ucap >= col_tiles, "prism_tile_lists: ucap must be >= col_tiles");
+  if (rows == 0) return PRISM_OK;
+  PRISM_REQUIRE(rows < (1ll << 31), "prism_tile_lists: too many tiles");
+  if (prism_debug_enabled())
+    PRISM_DEBUG_CHECK(prism_debug_check_lists("prism_tile_lists", start, len, cols, rows, col_tiles, 0, nullptr,
+                                              stream));
+  pair_union_kernel<1, false><<<(unsigned)rows, 256, 0, stream>>>(start, len, cols, row_tiles, col_tiles, nullptr,
+                                                                   tile_masks, ucap, 0, 1, ustart, ulen, ucols);
+  PRISM_LAUNCH_CHECK("prism_tile_lists");
   return PRISM_OK;
 }
 
@@ -381,8 +444,8 @@ int prism_quad_union(const int64_t* start, const int32_t* len, const int32_t* co
     PRISM_DEBUG_CHECK(prism_debug_check_maps("prism_quad_union", pairmap, rows / row_tiles, row_tiles, nullptr, 0,
                                              stream));
   }
-  pair_union_kernel<4><<<(unsigned)quads, 256, 0, stream>>>(start, len, cols, row_tiles, col_tiles, pairmap, tile_masks,
-                                                              ucap, ustart, ulen, ucols);
+  pair_union_kernel<4, false><<<(unsigned)quads, 256, 0, stream>>>(start, len, cols, row_tiles, col_tiles, pairmap,
+                                                                    tile_masks, ucap, 0, 1, ustart, ulen, ucols);
   PRISM_LAUNCH_CHECK("prism_quad_union");
   return PRISM_OK;
 }

@@ -462,6 +462,47 @@ std::tuple<Tensor, Tensor, Tensor> quad_union(const Tensor& s_, const Tensor& l_
   return {ustart, ulen, ucols};
 }
 
+std::tuple<Tensor, Tensor, Tensor> part_union(const Tensor& s_, const Tensor& l_, const Tensor& c_, int64_t row_tiles,
+                                              int64_t col_tiles, const OptT& pairmap_, const OptT& masks_, int64_t whole,
+                                              int64_t splits) {
+  check_lists(s_, l_, c_);
+  on_gpu(pairmap_, "pairmap");
+  on_gpu(masks_, "tile_masks");
+  check_dtype(pairmap_, at::kInt, "pairmap");
+  check_dtype(masks_, at::kLong, "tile_masks");
+  const c10::DeviceGuard guard(s_.device());
+  const Tensor s = s_.contiguous(), l = l_.contiguous(), c = c_.contiguous();
+  const OptT pairmap = cont(pairmap_), masks = cont(masks_);
+  const int64_t rows = s.numel(), pairs = rows / 2;
+  TORCH_CHECK_VALUE(whole >= 0 && whole <= pairs && splits >= 1 && splits <= 64, "part_union: bad split");
+  const int64_t items = whole + (pairs - whole) * splits;
+  Tensor ustart = at::empty({items}, opts(s, at::kLong));
+  Tensor ulen = at::empty({items}, opts(s, at::kInt));
+  Tensor ucols = at::empty({std::max<int64_t>(items * col_tiles, 1)}, opts(s, at::kInt));
+  PRISM_TORCH_CALL(prism_part_union, s.data_ptr<int64_t>(), l.data_ptr<int32_t>(), c.data_ptr<int32_t>(), rows,
+                   row_tiles, col_tiles, (const int32_t*)p(pairmap), (const uint64_t*)p(masks), whole, (int)splits, col_tiles,
+                   ustart.data_ptr<int64_t>(), ulen.data_ptr<int32_t>(), ucols.data_ptr<int32_t>(), stream_of(s));
+  return {ustart, ulen, ucols};
+}
+
+std::tuple<Tensor, Tensor, Tensor> tile_lists(const Tensor& s_, const Tensor& l_, const Tensor& c_, int64_t row_tiles,
+                                              int64_t col_tiles, const OptT& masks_) {
+  check_lists(s_, l_, c_);
+  on_gpu(masks_, "tile_masks");
+  check_dtype(masks_, at::kLong, "tile_masks");
+  const c10::DeviceGuard guard(s_.device());
+  const Tensor s = s_.contiguous(), l = l_.contiguous(), c = c_.contiguous();
+  const OptT masks = cont(masks_);
+  const int64_t rows = s.numel();
+  Tensor ustart = at::empty({rows}, opts(s, at::kLong));
+  Tensor ulen = at::empty({rows}, opts(s, at::kInt));
+  Tensor ucols = at::empty({std::max<int64_t>(rows * col_tiles, 1)}, opts(s, at::kInt));
+  PRISM_TORCH_CALL(prism_tile_lists, s.data_ptr<int64_t>(), l.data_ptr<int32_t>(), c.data_ptr<int32_t>(), rows,
+                   row_tiles, col_tiles, (const uint64_t*)p(masks), col_tiles, ustart.data_ptr<int64_t>(),
+                   ulen.data_ptr<int32_t>(), ucols.data_ptr<int32_t>(), stream_of(s));
+  return {ustart, ulen, ucols};
+}
+
 // CSR entry buffer of nnz entries, with at least one element: lists that
 // hold no entry at all (top-k of int((1 - s) N) = 0 blocks) still get a
 // valid pointer for the attention entry points, which take none as null
@@ -583,6 +624,25 @@ void check_union(const Tensor& us, const Tensor& ul, const Tensor& uc) { check_l
 // launch call returns
 Tensor work_counter(const Tensor& like) { return at::empty({8}, opts(like, at::kInt)); }
 
+// workspace of the (pairs - whole) * splits items of a split launch,
+// `floats` each
+struct SplitSpace {
+  Tensor acc;
+  SplitSpace(int64_t pairs, int64_t whole, int64_t splits, int64_t floats, const Tensor& like) {
+    TORCH_CHECK_VALUE(whole >= 0 && whole <= pairs && splits >= 1 && splits <= 64, "prism: bad split of ", pairs,
+                      " pairs (whole ", whole, ", splits ", splits, ")");
+    const int64_t n = (pairs - whole) * splits;
+    if (n > 0) acc = at::empty({n, floats}, opts(like, at::kFloat));
+  }
+  float* ptr() const { return acc.defined() ? acc.data_ptr<float>() : nullptr; }
+};
+
+// a split launch's lists hold one row per item
+void check_items(const Tensor& ul, int64_t pairs, int64_t whole, int64_t splits) {
+  TORCH_CHECK_VALUE(ul.numel() == whole + (pairs - whole) * splits, "prism: ", ul.numel(), " lists for ", pairs,
+                    " pairs (whole ", whole, ", splits ", splits, ")");
+}
+
 std::tuple<Tensor, Tensor> bsa_fwd(const Tensor& q_, const Tensor& k_, const Tensor& v_, const OptT& masks_,
                                    const Tensor& us_, const Tensor& ul_, const Tensor& uc_, const OptT& pairmap_,
                                    const OptT& order_, double sm_scale) {
@@ -601,6 +661,24 @@ std::tuple<Tensor, Tensor> bsa_fwd(const Tensor& q_, const Tensor& k_, const Ten
                    (const uint64_t*)p(masks), us.data_ptr<int64_t>(), ul.data_ptr<int32_t>(), uc.data_ptr<int32_t>(),
                    (const int32_t*)p(pairmap), (const int32_t*)p(order), (float)sm_scale, o.data_ptr(),
                    lse.data_ptr<float>(), work_counter(q).data_ptr<int32_t>(), stream_of(q));
+  return {o, lse};
+}
+
+std::tuple<Tensor, Tensor> bsa_fwd_tile(const Tensor& q_, const Tensor& k_, const Tensor& v_, const OptT& masks_,
+                                        const Tensor& us_, const Tensor& ul_, const Tensor& uc_, double sm_scale) {
+  const AttnShape s = attn_shape(q_, k_, v_);
+  check_union(us_, ul_, uc_);
+  on_gpu(masks_, "tile_masks");
+  const c10::DeviceGuard guard(q_.device());
+  const Tensor q = q_.contiguous(), k = k_.contiguous(), v = v_.contiguous();
+  const Tensor us = us_.contiguous(), ul = ul_.contiguous(), uc = uc_.contiguous();
+  const OptT masks = cont(masks_);
+  check_items(ul, s.B * s.H * (s.Sq / 64), s.B * s.H * (s.Sq / 64), 1);
+  Tensor o = at::empty_like(q);
+  Tensor lse = at::empty({s.B, s.H, s.Sq}, opts(q, at::kFloat));
+  PRISM_TORCH_CALL(prism_bsa_fwd_tile, q.data_ptr(), k.data_ptr(), v.data_ptr(), (int)(s.B * s.H), s.Sq, s.Sk,
+                   (int)s.D, (const uint64_t*)p(masks), us.data_ptr<int64_t>(), ul.data_ptr<int32_t>(),
+                   uc.data_ptr<int32_t>(), (float)sm_scale, o.data_ptr(), lse.data_ptr<float>(), stream_of(q));
   return {o, lse};
 }
 
@@ -671,10 +749,47 @@ std::tuple<Tensor, Tensor> bsa_bwd_dkdv(const Tensor& q_, const Tensor& k_, cons
   return {dk, dv};
 }
 
-// dQ over pair unions (quad = false) or quad unions (quad = true)
+std::tuple<Tensor, Tensor> bsa_bwd_dkdv_split(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& do_,
+                                        const Tensor& m2_, const Tensor& delta_, const OptT& kv_valid_,
+                                        const Tensor& us_, const Tensor& ul_, const Tensor& uc_, const OptT& pairmap_,
+                                        const OptT& order_, double sm_scale, int64_t whole,
+                                              int64_t splits) {
+  const AttnShape s = attn_shape(q_, k_, v_);
+  check_union(us_, ul_, uc_);
+  on_gpu(do_, "do");
+  on_gpu(m2_, "m2");
+  on_gpu(delta_, "delta");
+  on_gpu(kv_valid_, "kv_valid");
+  on_gpu(pairmap_, "pairmap");
+  on_gpu(order_, "order");
+  check_dtype(do_, at::kBFloat16, "do");
+  check_dtype(m2_, at::kFloat, "m2");
+  check_dtype(delta_, at::kFloat, "delta");
+  check_dtype(kv_valid_, at::kByte, "kv_valid");
+  TORCH_CHECK_VALUE(do_.sizes() == q_.sizes(), "bsa_bwd_dkdv_split: do must have q's shape");
+  const c10::DeviceGuard guard(q_.device());
+  const Tensor q = q_.contiguous(), k = k_.contiguous(), v = v_.contiguous(), d = do_.contiguous();
+  const Tensor m2 = m2_.contiguous(), delta = delta_.contiguous();
+  const Tensor us = us_.contiguous(), ul = ul_.contiguous(), uc = uc_.contiguous();
+  const OptT kv = cont(kv_valid_), pairmap = cont(pairmap_), order = cont(order_);
+  const int64_t pairs = s.B * s.H * (s.Sk / 128);
+  const SplitSpace sp(pairs, whole, splits, 2 * 128 * s.D, q);
+  check_items(ul, pairs, whole, splits);
+  Tensor dk = at::empty_like(k), dv = at::empty_like(v);
+  PRISM_TORCH_CALL(prism_bsa_bwd_dkdv_split, q.data_ptr(), k.data_ptr(), v.data_ptr(), d.data_ptr(), m2.data_ptr<float>(),
+                   delta.data_ptr<float>(), (int)(s.B * s.H), s.Sq, s.Sk, (int)s.D, (const uint8_t*)p(kv),
+                   us.data_ptr<int64_t>(), ul.data_ptr<int32_t>(), uc.data_ptr<int32_t>(), (const int32_t*)p(pairmap),
+                   (const int32_t*)p(order), (float)sm_scale, dk.data_ptr(), dv.data_ptr(),
+                   work_counter(q).data_ptr<int32_t>(), whole, (int)splits, sp.ptr(), stream_of(q));
+  return {dk, dv};
+}
+
+// dQ over pair unions, over pair unions with split lists where they pay, or
+// over quad unions
+enum class DqKind { pair, split, quad };
 Tensor bsa_bwd_dq_any(const Tensor& q_, const Tensor& k_, const Tensor& v_, const Tensor& do_, const Tensor& m2_,
                       const Tensor& delta_, const OptT& masks_, const Tensor& us_, const Tensor& ul_, const Tensor& uc_,
-                      const OptT& pairmap_, const OptT& order_, double sm_scale, bool quad) {
+                      const OptT& pairmap_, const OptT& order_, double sm_scale, DqKind kind, int64_t whole = 0, int64_t splits = 1) {
   const AttnShape s = attn_shape(q_, k_, v_);
   check_union(us_, ul_, uc_);
   on_gpu(do_, "do");
@@ -693,7 +808,19 @@ Tensor bsa_bwd_dq_any(const Tensor& q_, const Tensor& k_, const Tensor& v_, cons
   const Tensor us = us_.contiguous(), ul = ul_.contiguous(), uc = uc_.contiguous();
   const OptT masks = cont(masks_), pairmap = cont(pairmap_), order = cont(order_);
   Tensor dq = at::empty_like(q);
-  auto fn = quad ? &prism_bsa_bwd_dq_quad : &prism_bsa_bwd_dq;
+  if (kind == DqKind::split) {
+    const int64_t pairs = s.B * s.H * (s.Sq / 128);
+    const SplitSpace sp(pairs, whole, splits, 128 * s.D, q);
+    check_items(ul, pairs, whole, splits);
+    PRISM_TORCH_CALL(prism_bsa_bwd_dq_split, q.data_ptr(), k.data_ptr(), v.data_ptr(), d.data_ptr(),
+                     m2.data_ptr<float>(), delta.data_ptr<float>(), (int)(s.B * s.H), s.Sq, s.Sk, (int)s.D,
+                     (const uint64_t*)p(masks), us.data_ptr<int64_t>(), ul.data_ptr<int32_t>(),
+                     uc.data_ptr<int32_t>(), (const int32_t*)p(pairmap), (const int32_t*)p(order), (float)sm_scale,
+                     dq.data_ptr(), work_counter(q).data_ptr<int32_t>(), whole, (int)splits, sp.ptr(),
+                     stream_of(q));
+    return dq;
+  }
+  auto fn = kind == DqKind::quad ? &prism_bsa_bwd_dq_quad : &prism_bsa_bwd_dq;
   PRISM_TORCH_CALL(fn, q.data_ptr(), k.data_ptr(), v.data_ptr(), d.data_ptr(), m2.data_ptr<float>(),
                    delta.data_ptr<float>(), (int)(s.B * s.H), s.Sq, s.Sk, (int)s.D, (const uint64_t*)p(masks),
                    us.data_ptr<int64_t>(), ul.data_ptr<int32_t>(), uc.data_ptr<int32_t>(), (const int32_t*)p(pairmap),
@@ -704,13 +831,20 @@ Tensor bsa_bwd_dq_any(const Tensor& q_, const Tensor& k_, const Tensor& v_, cons
 Tensor bsa_bwd_dq(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& d, const Tensor& m2,
                   const Tensor& delta, const OptT& masks, const Tensor& us, const Tensor& ul, const Tensor& uc,
                   const OptT& pairmap, const OptT& order, double sm_scale) {
-  return bsa_bwd_dq_any(q, k, v, d, m2, delta, masks, us, ul, uc, pairmap, order, sm_scale, false);
+  return bsa_bwd_dq_any(q, k, v, d, m2, delta, masks, us, ul, uc, pairmap, order, sm_scale, DqKind::pair);
+}
+
+Tensor bsa_bwd_dq_split(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& d, const Tensor& m2,
+                        const Tensor& delta, const OptT& masks, const Tensor& us, const Tensor& ul, const Tensor& uc,
+                        const OptT& pairmap, const OptT& order, double sm_scale, int64_t whole, int64_t splits) {
+  return bsa_bwd_dq_any(q, k, v, d, m2, delta, masks, us, ul, uc, pairmap, order, sm_scale, DqKind::split, whole,
+                        splits);
 }
 
 Tensor bsa_bwd_dq_quad(const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& d, const Tensor& m2,
                        const Tensor& delta, const OptT& masks, const Tensor& us, const Tensor& ul, const Tensor& uc,
                        const OptT& quadmap, const OptT& order, double sm_scale) {
-  return bsa_bwd_dq_any(q, k, v, d, m2, delta, masks, us, ul, uc, quadmap, order, sm_scale, true);
+  return bsa_bwd_dq_any(q, k, v, d, m2, delta, masks, us, ul, uc, quadmap, order, sm_scale, DqKind::quad);
 }
 
 }  // namespace
@@ -760,6 +894,18 @@ TORCH_LIBRARY(prism, m) {
         "Tensor ustart, Tensor ulen, Tensor ucols, Tensor? pairmap, Tensor? order, float sm_scale) -> Tensor");
   m.def("bsa_bwd_dq_quad(Tensor q, Tensor k, Tensor v, Tensor do, Tensor m2, Tensor delta, Tensor? tile_masks, "
         "Tensor ustart, Tensor ulen, Tensor ucols, Tensor? quadmap, Tensor? order, float sm_scale) -> Tensor");
+  m.def("part_union(Tensor start, Tensor len, Tensor cols, int row_tiles, int col_tiles, Tensor? pairmap, "
+        "Tensor? tile_masks, int whole, int splits) -> (Tensor, Tensor, Tensor)");
+  m.def("tile_lists(Tensor start, Tensor len, Tensor cols, int row_tiles, int col_tiles, Tensor? tile_masks) "
+        "-> (Tensor, Tensor, Tensor)");
+  m.def("bsa_fwd_tile(Tensor q, Tensor k, Tensor v, Tensor? tile_masks, Tensor ustart, Tensor ulen, Tensor ucols, "
+        "float sm_scale) -> (Tensor, Tensor)");
+  m.def("bsa_bwd_dkdv_split(Tensor q, Tensor k, Tensor v, Tensor do, Tensor m2, Tensor delta, Tensor? kv_valid, "
+        "Tensor ustart, Tensor ulen, Tensor ucols, Tensor? pairmap, Tensor? order, float sm_scale, "
+        "int whole, int splits) -> (Tensor, Tensor)");
+  m.def("bsa_bwd_dq_split(Tensor q, Tensor k, Tensor v, Tensor do, Tensor m2, Tensor delta, Tensor? tile_masks, "
+        "Tensor ustart, Tensor ulen, Tensor ucols, Tensor? pairmap, Tensor? order, float sm_scale, "
+        "int whole, int splits) -> Tensor");
 }
 
 // GPU tensors of the ROCm build dispatch under torch's CUDA key
@@ -796,4 +942,9 @@ TORCH_LIBRARY_IMPL(prism, CUDA, m) {
   m.impl("bsa_bwd_dkdv", &bsa_bwd_dkdv);
   m.impl("bsa_bwd_dq", &bsa_bwd_dq);
   m.impl("bsa_bwd_dq_quad", &bsa_bwd_dq_quad);
+  m.impl("part_union", &part_union);
+  m.impl("tile_lists", &tile_lists);
+  m.impl("bsa_fwd_tile", &bsa_fwd_tile);
+  m.impl("bsa_bwd_dkdv_split", &bsa_bwd_dkdv_split);
+  m.impl("bsa_bwd_dq_split", &bsa_bwd_dq_split);
 }

@@ -25,6 +25,7 @@ import torch
 
 from . import ops
 from .dynamic_block_shape import ALL_CANDIDATE_SHAPES, ZONE_SIZE, _gradient_and_shapes
+from .worklists import WorkLists
 
 _TILE = 64  # kernel tile (dynamic_block_attention.py:15)
 
@@ -48,7 +49,7 @@ def _build_block_tile_maps(shape_ids, ZT, ZH, ZW, device):
 
 
 # ------------------------------------------------------------------ selection (steps 3-5)
-class _Plan:
+class _Plan(WorkLists):
     """Everything the attention kernels need for one call, built under no_grad."""
 
     def __init__(self, q, k, v, grid, shape_ids, valid_mask, sparsity, cdf_threshold, sm_scale,
@@ -80,116 +81,9 @@ class _Plan:
         self.qstart, self.qlen = ops.tile_rows(sel["ntiles"], lay.block_id_of_tile, B * H, lay.Nt, lay.N_b,
                                                sel["tcap"], self.tile_count if skip else None)
         self.qcols = sel["tiles"].view(-1)
-        # compact lists: the two pair unions the backward keeps are stored as
-        # CSR, O(nnz) memory instead of pairs x Nt (settle(); one host read of
-        # both nnz, made while the forward kernel runs); same entries in the
-        # same order, so identical results
-        self.compact = compact_lists
-        self._settled = False
-        # pair unions of the per-query-tile key lists (forward, dQ) and the key
-        # validity words of padded key tiles
-        self.tmasks = ops.tile_masks(self.kv_valid) if masked else None
-        # pair the query tiles of each zone by list overlap (fewest idle wave slots)
-        self.qpair = ops.pair_tiles(self.qstart, self.qlen, self.qcols, lay.Nt)
-        self.qunion = ops.pair_union(self.qstart, self.qlen, self.qcols, lay.Nt, self.tmasks, pairmap=self.qpair)
-        self._csr = ops.DeferredCompaction(3) if compact_lists else None
-        if compact_lists:
-            self._csr.add(0, self.qunion)
-        # launch order of the forward and dQ kernels (the last workgroups ids
-        # take the longest lists first: the launch does not end on a long one)
-        self.qorder = ops.pair_order(self.qunion[1], 64)
-        # quad unions (two pairs of a zone per workgroup: four query tiles per
-        # staged K / V tile), which the forward and dQ kernels walk instead of
-        # the pair unions when ops.QUADS is set (same results, bit for bit)
-        self.qquad = self.qquad_order = self.qquadmap = None
-        # dq_quads: dQ walks them too (by default on this path), so the
-        # backward keeps them
-        self.quads = ops.QUADS and lay.Nt % 4 == 0
-        self.dq_quads = self.quads and ops.DQ_QUADS is not False
-        if self.quads:
-            self.qquadmap = self.qpair
-            self.qquad = ops.quad_union(self.qstart, self.qlen, self.qcols, lay.Nt, self.tmasks,
-                                        pairmap=self.qquadmap)
-            if compact_lists and self.dq_quads:
-                self._csr.add(2, self.qquad)
-            self.qquad_order = ops.pair_order(self.qquad[1], 32)
-        self.klists = None
-        self.kpair = None
-        self.kunion = None
-        self.korder = None
-        self.keys_ready = None  # event of a key-list build on the side stream
-
-    def build_key_lists_side(self):
-        """build_key_lists on the side stream, after the work queued so far on
-        the current stream."""
-        if self.kunion is not None:
-            return
-        _, self.keys_ready = ops.side_launch(
-            self.qcols.device, self.build_key_lists, reads=(self.qstart, self.qlen, self.qcols),
-            produces=lambda _: (*self.klists, self.kpair, *self.kunion, self.korder,
-                                self._csr.offsets[1] if self._csr is not None else None))
-
-    def join_side(self):
-        """Make the current stream wait for a side-stream key-list build (the
-        stream fork is joined where it was opened, so a captured or
-        backward-less forward leaves no dangling dependency)."""
-        if self.keys_ready is not None:
-            torch.cuda.current_stream().wait_event(self.keys_ready)
-            self.keys_ready = None
-
-    def build_key_lists(self):
-        """Per-key-tile query lists, their pairing, unions and launch order
-        (the dK/dV side), built on first use."""
-        self.join_side()
-        if self.kunion is not None:
-            return
-        Nt = self.lay.Nt
-        self.klists = ops.transpose_lists(self.qstart, self.qlen, self.qcols, self.B * self.H, Nt)
-        self.kpair = ops.pair_tiles(*self.klists, Nt)
-        self.kunion = ops.pair_union(*self.klists, Nt, pairmap=self.kpair)
-        self.korder = ops.pair_order(self.kunion[1], 32)
-        if self._csr is not None:
-            self._csr.add(1, self.kunion)
-
-    def settle(self):
-        """Keep only what the backward reads: the query-side and key-side pair
-        unions, and the quad unions when dQ walks them (compact CSR when the
-        plan is compact, with one batched host read of their nnz), pairings
-        and launch orders.  The per-tile lists (1.0 GB query-side and 0.66 GB
-        key-side at config 4) and the forward-only quad unions are released."""
-        if self._settled:
-            return
-        self.build_key_lists()
-        if self._csr is not None:
-            lists = [self.qunion, self.kunion] + ([self.qquad] if self.dq_quads else [])
-            done = self._csr.finish(lists)
-            self.qunion, self.kunion = done[:2]
-            if self.dq_quads:
-                self.qquad = done[2]
-            self._csr = None
-        if not self.dq_quads:  # the forward's only: released once it is queued
-            self.qquad = self.qquad_order = None
-        self.qcols = None
-        self.klists = None
-        self.sel = {key: val for key, val in self.sel.items() if key != "tiles"}
-        self._settled = True
-
-    def list_bytes(self) -> int:
-        """Bytes of the work lists the plan holds."""
-        ts = [*self.qunion, self.qstart, self.qlen]
-        if self.qquad is not None:
-            ts += list(self.qquad)
-        if self.qcols is not None:
-            ts.append(self.qcols)
-        if self.kunion is not None:
-            ts += list(self.kunion)
-        if self.klists is not None:
-            ts += list(self.klists)
-        return sum(t.numel() * t.element_size() for t in ts)
-
-    def sum_lens(self) -> int:
-        """Executed (query tile, key tile) pairs (host sync)."""
-        return int(self.qlen.sum().item())
+        # key validity words of padded key tiles, and the work lists
+        tmasks = ops.tile_masks(self.kv_valid) if masked else None
+        self._build_query_lists(B * H, lay.Nt, lay.Nt, D, tmasks, compact_lists, ops.DQ_QUADS is not False)
 
 
 class _DynBSA(torch.autograd.Function):
@@ -199,22 +93,7 @@ class _DynBSA(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, plan: _Plan, sm_scale: float):
-        grads = any(ctx.needs_input_grad[:3])
-        if grads:
-            # the backward's lists, beside the forward kernel (or before it)
-            if ops.OVERLAP_SIDE_WORK:
-                plan.build_key_lists_side()
-            else:
-                plan.build_key_lists()
-        if plan.qquad is not None:
-            o_re, lse = ops.bsa_fwd_quad(plan.q_re, plan.k_re, plan.v_re, plan.tmasks, plan.qquad, sm_scale,
-                                         plan.qquadmap, plan.qquad_order)
-        else:
-            o_re, lse = ops.bsa_fwd(plan.q_re, plan.k_re, plan.v_re, plan.tmasks, plan.qunion, sm_scale, plan.qpair,
-                                    plan.qorder)
-        plan.join_side()  # queued after the forward kernel: the key lists still run beside it
-        if grads:
-            plan.settle()  # release the per-tile lists; compact the unions while the forward runs
+        o_re, lse = plan.attend(sm_scale, any(ctx.needs_input_grad[:3]))
         ctx.plan = plan
         ctx.sm_scale = sm_scale
         ctx.in_dtypes = (q.dtype, k.dtype, v.dtype)
@@ -228,8 +107,6 @@ class _DynBSA(torch.autograd.Function):
         lay = plan.lay
         gd = ops.gather_pool(do.contiguous(), lay, None, rows=True, dot_with=o_re)
         do_re, delta = gd["rows"], gd["rowdot"]
-        plan.build_key_lists()
-        m2 = ops.lse_to_m2(lse)
         tq, tk, tv = ctx.in_dtypes
         side = {}
 
@@ -240,12 +117,7 @@ class _DynBSA(torch.autograd.Function):
                     dk_re.device, lambda: (ops.scatter_rows(dk_re, lay, tk), ops.scatter_rows(dv_re, lay, tv)),
                     reads=(dk_re, dv_re), produces=lambda out: out)
 
-        quads = plan.dq_quads
-        dq_re, dk_re, dv_re = ops.bsa_bwd(plan.q_re, plan.k_re, plan.v_re, do_re, m2, delta, plan.kv_valid,
-                                          plan.tmasks, plan.qquad if quads else plan.qunion, plan.kunion,
-                                          ctx.sm_scale, plan.qquadmap if quads else plan.qpair, plan.kpair,
-                                          plan.qquad_order if quads else plan.qorder, plan.korder,
-                                          after_dkdv=scatter_dkdv, q_quads=quads)
+        dq_re, dk_re, dv_re = plan.attend_backward(do_re, lse, delta, ctx.sm_scale, scatter_dkdv)
         dq = ops.scatter_rows(dq_re, lay, tq)
         if "dkdv" in side:
             (dk, dv), done = side["dkdv"]

@@ -9,6 +9,7 @@ where the kernels need it.
 from __future__ import annotations
 
 import contextlib
+import ctypes
 import os
 from typing import Dict, List, Optional, Tuple
 
@@ -457,11 +458,13 @@ class DeferredCompaction:
         self.offsets[i], self.events[i] = off, ev
 
     def finish(self, lists_seq):
-        """lists_seq[i]: the lists added as i (slots never added are left out)."""
-        for ev in self.events[:len(lists_seq)]:
-            ev.synchronize()
+        """lists_seq[i]: the lists added as i; others come back as they are."""
+        for ev in self.events:
+            if ev is not None:
+                ev.synchronize()
         nnz = self.host.tolist()
-        return [(*csr_lists(self.offsets[i]), csr_fill(*lists, self.offsets[i], nnz[i]))
+        return [lists if self.offsets[i] is None else
+                (*csr_lists(self.offsets[i]), csr_fill(*lists, self.offsets[i], nnz[i]))
                 for i, lists in enumerate(lists_seq)]
 
 
@@ -585,6 +588,62 @@ def bsa_fwd(q, k, v, tmasks, qunion, sm_scale: float, qpair: Optional[torch.Tens
     return _op("bsa_fwd", q, k, v, tmasks, ustart, ulen, ucols, qpair, qorder, float(sm_scale))
 
 
+# Query-side launches of fewer pairs than SPLIT_PAIRS (eight rounds of the 512
+# workgroups that the pair forward and dQ kernels keep resident) walk pairs, dQ
+# and dK/dV with split lists where they pay; forward launches of at most
+# TILE_PAIRS (one tile per CU) walk single tiles.
+SPLIT_PAIRS = 4096
+TILE_PAIRS = 128
+# A side of a few rounds keeps up to this much of dense lists to the backward:
+# compact ones would cost a host read of their size and launches of their own.
+KEEP_DENSE_BYTES = 64 << 20
+
+
+def split_plan(kernel: int, heads: int, pairs_per_head: int, max_entries: int, D: int) -> Tuple[int, int]:
+    """(whole, splits) of a split launch (prism_split_plan; kernel 1 dQ, 2
+    dK/dV): pairs below whole keep one work item, every later pair is
+    cut into splits items."""
+    whole, splits = ctypes.c_int64(), ctypes.c_int32()
+    _lib.call("prism_split_plan", int(kernel), int(heads), int(pairs_per_head), int(max_entries), int(D),
+              ctypes.byref(whole), ctypes.byref(splits))
+    return whole.value, splits.value
+
+
+def part_union(start: torch.Tensor, length: torch.Tensor, cols: torch.Tensor, Nt: int, whole: int, splits: int,
+               tmasks: Optional[torch.Tensor] = None, col_tiles: Optional[int] = None,
+               pairmap: Optional[torch.Tensor] = None):
+    """pair_union with one row per work item of a split launch: the unions of
+    the pairs below whole, then splits rows for every later pair, row i with
+    the tiles t of its union with (t / 8) mod splits == i."""
+    _cuda(start, length, cols, tmasks, pairmap)
+    return _op("part_union", start, length, cols, int(Nt), int(Nt if col_tiles is None else col_tiles), pairmap, tmasks,
+               int(whole), int(splits))
+
+
+def items_order(ulen: torch.Tensor, group: int) -> Optional[torch.Tensor]:
+    """Launch order of an attention launch (group: 64 for the forward and dQ,
+    32 for dK/dV), longest lists first in its last quarter; None when all of
+    its work items run at once."""
+    return pair_order(ulen, group) if ulen.numel() > 8 * group else None
+
+
+def tile_lists(start: torch.Tensor, length: torch.Tensor, cols: torch.Tensor, Nt: int,
+               tmasks: Optional[torch.Tensor] = None, col_tiles: Optional[int] = None):
+    """Per-tile lists as the entries of bsa_fwd_tile: one row per tile, in
+    pair_union's format with the tile's own member bit (bit row % 2)."""
+    _cuda(start, length, cols, tmasks)
+    return _op("tile_lists", start, length, cols, int(Nt), int(Nt if col_tiles is None else col_tiles), tmasks)
+
+
+def bsa_fwd_tile(q, k, v, tmasks, lists, sm_scale: float):
+    """bsa_fwd over tile_lists rows, one workgroup per query tile (the same o
+    and lse, bit for bit): for launches of few pairs (TILE_PAIRS)."""
+    _cuda(q, k, v, tmasks)
+    q, k, v = _bf16(q, "q"), _bf16(k, "k"), _bf16(v, "v")
+    _attn_shapes(q, k, v)
+    return _op("bsa_fwd_tile", q, k, v, tmasks, *lists, float(sm_scale))
+
+
 def bsa_fwd_quad(q, k, v, tmasks, quadunion, sm_scale: float, quadmap: Optional[torch.Tensor] = None,
                  qorder: Optional[torch.Tensor] = None):
     """bsa_fwd over quad unions (quad_union of the per-query-tile key lists with
@@ -665,22 +724,24 @@ def side_launch(device: torch.device, fn, reads=(), produces=None):
 def bsa_bwd(q, k, v, do, m2, delta, kv_valid, tmasks, qunion, kunion, sm_scale: float,
             qpair: Optional[torch.Tensor] = None, kpair: Optional[torch.Tensor] = None,
             qorder: Optional[torch.Tensor] = None, korder: Optional[torch.Tensor] = None, after_dkdv=None,
-            q_quads: bool = False):
+            q_quads: bool = False, q_split: Optional[Tuple[int, int]] = None,
+            k_split: Optional[Tuple[int, int]] = None):
     """Backward over tile-order bf16 tensors; qunion / kunion = pair unions of
     the per-query-tile key lists and of the per-key-tile query lists, built
     with the pairings qpair / kpair (None: neighbouring tiles).  With q_quads,
     qunion is the quad_union of the per-query-tile lists (quadmap qpair,
     launch order qorder over quads) and dQ runs over quads (bit-identical).
     Returns dq, dk, dv (bf16, tile order).  after_dkdv(dk, dv), if given, is
-    called between the dK/dV and the dQ launches."""
+    called between the dK/dV and the dQ launches.  q_split / k_split
+    (whole, splits): qunion / kunion are the part_union of a split launch."""
     _cuda(q, k, v, do, m2, delta, kv_valid, tmasks, qpair, kpair, qorder, korder)
     q, k, v, do = _bf16(q, "q"), _bf16(k, "k"), _bf16(v, "v"), _bf16(do, "do")
     B, H, Sq, Sk, D = _attn_shapes(q, k, v)
     if do.shape != q.shape:
         raise ValueError("do must have q's shape")
     def dkdv():
-        return _op("bsa_bwd_dkdv", q, k, v, do, m2, delta, kv_valid, kunion[0], kunion[1], kunion[2], kpair, korder,
-                   float(sm_scale))
+        args = (q, k, v, do, m2, delta, kv_valid, kunion[0], kunion[1], kunion[2], kpair, korder, float(sm_scale))
+        return _op("bsa_bwd_dkdv", *args) if k_split is None else _op("bsa_bwd_dkdv_split", *args, *k_split)
 
     main = torch.cuda.current_stream()
     if BWD_CONCURRENT:
@@ -697,8 +758,11 @@ def bsa_bwd(q, k, v, do, m2, delta, kv_valid, tmasks, qunion, kunion, sm_scale: 
         dk, dv = dkdv()
     if after_dkdv is not None:
         after_dkdv(dk, dv)
-    dq = _op("bsa_bwd_dq_quad" if q_quads else "bsa_bwd_dq", q, k, v, do, m2, delta, tmasks, qunion[0], qunion[1],
-             qunion[2], qpair, qorder, float(sm_scale))
+    args = (q, k, v, do, m2, delta, tmasks, qunion[0], qunion[1], qunion[2], qpair, qorder, float(sm_scale))
+    if q_split is not None:
+        dq = _op("bsa_bwd_dq_split", *args, *q_split)
+    else:
+        dq = _op("bsa_bwd_dq_quad" if q_quads else "bsa_bwd_dq", *args)
     if BWD_CONCURRENT:
         main.wait_stream(side)
     return dq, dk, dv

@@ -36,9 +36,10 @@ from typing import Optional, Sequence
 import torch
 
 from . import ops
+from .worklists import WorkLists
 
 
-class _ChunkPlan:
+class _ChunkPlan(WorkLists):
     """Rearranged rows, selection and work lists of one call (built under no_grad)."""
 
     def __init__(self, q, k, v, lq: ops.ChunkLayout, lk: ops.ChunkLayout, q_valid, k_valid, sparsity,
@@ -71,95 +72,8 @@ class _ChunkPlan:
         self.qstart, self.qlen = ops.tile_rows(sel["ntiles"], lq.block_id_of_tile, BH, lq.Nt, lq.N_b, sel["tcap"],
                                                qcount)
         self.qcols = sel["tiles"].view(-1)
-        # compact lists: the pair unions the backward keeps as CSR, O(nnz)
-        # memory (settle(); one host read of both nnz; same entries)
-        self.compact = compact_lists
-        self._settled = False
-        self.tmasks = ops.tile_masks(self.kv_valid) if k_masked else None
-        self.qpair = ops.pair_tiles(self.qstart, self.qlen, self.qcols, lq.Nt, lk.Nt)
-        self.qunion = ops.pair_union(self.qstart, self.qlen, self.qcols, lq.Nt, self.tmasks, col_tiles=lk.Nt,
-                                     pairmap=self.qpair)
-        self._csr = ops.DeferredCompaction(3) if compact_lists else None
-        if compact_lists:
-            self._csr.add(0, self.qunion)
-        # launch order of the forward and dQ kernels (longest lists last-dispatched first)
-        self.qorder = ops.pair_order(self.qunion[1], 64)
-        # quad unions (two pairs per workgroup), which the forward and dQ
-        # kernels walk instead of the pair unions when ops.QUADS is set (same
-        # results, bit for bit)
-        self.qquad = self.qquad_order = self.qquadmap = None
-        # dq_quads: dQ walks them too (only when ops.DQ_QUADS forces it on
-        # these paths, whose quads leave more slots idle), so the backward
-        # keeps them
-        self.quads = ops.QUADS and lq.Nt % 4 == 0
-        self.dq_quads = self.quads and ops.DQ_QUADS is True
-        if self.quads:
-            self.qquadmap = self.qpair
-            self.qquad = ops.quad_union(self.qstart, self.qlen, self.qcols, lq.Nt, self.tmasks, col_tiles=lk.Nt,
-                                        pairmap=self.qquadmap)
-            if compact_lists and self.dq_quads:
-                self._csr.add(2, self.qquad)
-            self.qquad_order = ops.pair_order(self.qquad[1], 32)
-        self.klists = None
-        self.kpair = None
-        self.kunion = None
-        self.korder = None
-        self.keys_ready = None  # event of a key-list build on the side stream
-
-    def key_lists_side(self):
-        """key_lists on the side stream, after the work queued so far on the
-        current stream."""
-        if self.kunion is not None:
-            return
-        _, self.keys_ready = ops.side_launch(
-            self.qcols.device, self.key_lists, reads=(self.qstart, self.qlen, self.qcols),
-            produces=lambda _: (*self.klists, self.kpair, *self.kunion, self.korder,
-                                self._csr.offsets[1] if self._csr is not None else None))
-
-    def join_side(self):
-        """Make the current stream wait for a side-stream key-list build (the
-        fork is joined in the forward that opened it)."""
-        if getattr(self, "keys_ready", None) is not None:
-            torch.cuda.current_stream().wait_event(self.keys_ready)
-            self.keys_ready = None
-
-    def key_lists(self):
-        self.join_side()
-        if self.kunion is None:
-            self.klists = ops.transpose_lists(self.qstart, self.qlen, self.qcols, self.B * self.H, self.lq.Nt,
-                                              self.lk.Nt)
-            self.kpair = ops.pair_tiles(*self.klists, self.lk.Nt, self.lq.Nt)
-            self.kunion = ops.pair_union(*self.klists, self.lk.Nt, None, col_tiles=self.lq.Nt, pairmap=self.kpair)
-            self.korder = ops.pair_order(self.kunion[1], 32)
-            if self._csr is not None:
-                self._csr.add(1, self.kunion)
-        return self.kunion
-
-    def settle(self):
-        """Keep only what the backward reads: the pair unions, and the quad
-        unions when dQ walks them (compact CSR when the plan is compact, one
-        batched host read of their nnz), pairings and launch orders; the
-        per-tile lists and the forward-only quad unions are released."""
-        if self._settled:
-            return
-        self.key_lists()
-        if self._csr is not None:
-            lists = [self.qunion, self.kunion] + ([self.qquad] if self.dq_quads else [])
-            done = self._csr.finish(lists)
-            self.qunion, self.kunion = done[:2]
-            if self.dq_quads:
-                self.qquad = done[2]
-            self._csr = None
-        if not self.dq_quads:  # the forward's only: released once it is queued
-            self.qquad = self.qquad_order = None
-        self.qcols = None
-        self.klists = None
-        self.sel = {key: val for key, val in self.sel.items() if key != "tiles"}
-        self._settled = True
-
-    def sum_lens(self) -> int:
-        """Executed (query tile, key tile) pairs (host sync)."""
-        return int(self.qlen.sum().item())
+        tmasks = ops.tile_masks(self.kv_valid) if k_masked else None
+        self._build_query_lists(BH, lq.Nt, lk.Nt, D, tmasks, compact_lists, ops.DQ_QUADS is True)
 
 
 class _ChunkBSA(torch.autograd.Function):
@@ -169,22 +83,7 @@ class _ChunkBSA(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, q, k, v, plan: _ChunkPlan, sm_scale: float):
-        grads = any(ctx.needs_input_grad[:3])
-        if grads:
-            # the backward's lists, beside the forward kernel (or before it)
-            if ops.OVERLAP_SIDE_WORK:
-                plan.key_lists_side()
-            else:
-                plan.key_lists()
-        if plan.qquad is not None:
-            o_re, lse = ops.bsa_fwd_quad(plan.q_re, plan.k_re, plan.v_re, plan.tmasks, plan.qquad, sm_scale,
-                                         plan.qquadmap, plan.qquad_order)
-        else:
-            o_re, lse = ops.bsa_fwd(plan.q_re, plan.k_re, plan.v_re, plan.tmasks, plan.qunion, sm_scale, plan.qpair,
-                                    plan.qorder)
-        plan.join_side()  # queued after the forward kernel: the key lists still run beside it
-        if grads:
-            plan.settle()  # release the per-tile lists; compact the unions while the forward runs
+        o_re, lse = plan.attend(sm_scale, any(ctx.needs_input_grad[:3]))
         ctx.plan = plan
         ctx.sm_scale = sm_scale
         ctx.in_dtypes = (q.dtype, k.dtype, v.dtype)
@@ -196,8 +95,6 @@ class _ChunkBSA(torch.autograd.Function):
         plan: _ChunkPlan = ctx.plan
         o_re, lse = ctx.saved_tensors
         gd = ops.chunk_gather_pool(do.contiguous(), plan.lq, None, rows=True, dot_with=o_re)
-        kunion = plan.key_lists()
-        m2 = ops.lse_to_m2(lse)
         tq, tk, tv = ctx.in_dtypes
         side = {}
 
@@ -209,12 +106,7 @@ class _ChunkBSA(torch.autograd.Function):
                     lambda: (ops.chunk_scatter_rows(dk_re, plan.lk, tk), ops.chunk_scatter_rows(dv_re, plan.lk, tv)),
                     reads=(dk_re, dv_re), produces=lambda out: out)
 
-        quads = plan.dq_quads
-        dq_re, dk_re, dv_re = ops.bsa_bwd(plan.q_re, plan.k_re, plan.v_re, gd["rows"], m2, gd["rowdot"],
-                                          plan.kv_valid, plan.tmasks, plan.qquad if quads else plan.qunion, kunion,
-                                          ctx.sm_scale, plan.qquadmap if quads else plan.qpair, plan.kpair,
-                                          plan.qquad_order if quads else plan.qorder, plan.korder,
-                                          after_dkdv=scatter_dkdv, q_quads=quads)
+        dq_re, dk_re, dv_re = plan.attend_backward(gd["rows"], lse, gd["rowdot"], ctx.sm_scale, scatter_dkdv)
         dq = ops.chunk_scatter_rows(dq_re, plan.lq, tq)
         if "dkdv" in side:
             (dk, dv), done = side["dkdv"]

@@ -1,0 +1,134 @@
+"""Launches of few pairs: prism_bsa_fwd_tile over prism_tile_lists rows (one
+workgroup per query tile, the pair forward's bits), prism_part_union and the
+split dQ / dK/dV launches over it.
+
+Lists of 0 to 6 entries around the copy pipeline's depth, tile counts that are
+not multiples of the groups of 8 or of the 32-bit bitmap words, a list range of
+more than one bitmap window (8,192 tiles), rows without a list, key masks,
+split launches with and without whole pairs."""
+import math
+
+import numpy as np
+import pytest
+import torch
+
+from tests.test_gpu_parity import bits_equal, host, say
+from tests.test_gpu_torch_ops import UTILS
+
+pytestmark = pytest.mark.gpu
+
+
+def make(seed, BH, Ntq, Ntk, D, longest, masked):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    rng = np.random.default_rng(seed)
+    t = lambda n: torch.randn((1, BH, n * 64, D), device="cuda", generator=g).to(torch.bfloat16)
+    q, do, k, v = t(Ntq), t(Ntq), t(Ntk), t(Ntk)
+    lens = rng.integers(0, min(longest, Ntk) + 1, BH * Ntq).astype(np.int32)
+    lens[: min(7, lens.size)] = np.minimum(np.arange(min(7, lens.size)), Ntk)
+    cols = np.concatenate([np.sort(rng.choice(Ntk, n, replace=False)) for n in lens] + [np.zeros(1)]).astype(np.int32)
+    start = (np.cumsum(lens) - lens).astype(np.int64)
+    dev = lambda a: torch.from_numpy(a).to("cuda")
+    valid = torch.rand((Ntk * 64,), device="cuda", generator=g) < 0.8 if masked else None
+    return q, k, v, do, (dev(start), dev(lens), dev(cols)), valid
+
+
+@pytest.mark.parametrize("shape", [(1, 2, 2, 64, 2, False), (3, 6, 10, 64, 6, True), (2, 10, 40, 128, 40, True),
+                                   (1, 4, 8202, 64, 60, False)], ids=str)
+def test_tile_forward_equals_pair_forward(shape):
+    from prism_amd import ops
+    BH, Ntq, Ntk, D, longest, masked = shape
+    say("tile forward", shape)
+    q, k, v, _, lists, valid = make(1, BH, Ntq, Ntk, D, longest, masked)
+    tm, sm = ops.tile_masks(valid), 1.0 / math.sqrt(D)
+    rows = ops.tile_lists(*lists, Ntq, tm, Ntk)
+    st, ln, cl = (host(t) for t in rows)
+    s0, l0, c0 = (host(t) for t in lists)
+    full = None if tm is None else host(tm) == -1
+    for r in range(BH * Ntq):
+        t = c0[s0[r]: s0[r] + l0[r]]
+        part = np.zeros_like(t) if full is None else (~full[t]).astype(np.int32)
+        assert np.array_equal(cl[st[r]: st[r] + ln[r]], t << 3 | part << 2 | 1 << (r % 2)), r
+    o1, l1 = ops.bsa_fwd(q, k, v, tm, ops.pair_union(*lists, Ntq, tm, col_tiles=Ntk), sm)
+    o2, l2 = ops.bsa_fwd_tile(q, k, v, tm, rows, sm)
+    assert bits_equal(host(o1), host(o2)) and bits_equal(host(l1), host(l2))
+
+
+# (whole, splits): every pair split, some, none
+@pytest.mark.parametrize("shape", [(1, 2, 2, 64, 2, False, 0, 2), (3, 6, 10, 64, 6, True, 3, 3),
+                                   (2, 10, 40, 128, 40, True, 4, 5), (2, 16, 24, 128, 24, False, 16, 1),
+                                   (1, 4, 8202, 64, 60, False, 0, 16)], ids=str)
+def test_split_backward(shape):
+    from prism_amd import ops
+    BH, Ntq, Ntk, D, longest, masked, whole, splits = shape
+    say("split backward", shape)
+    q, k, v, do, lists, valid = make(2, BH, Ntq, Ntk, D, longest, masked)
+    tm, sm = ops.tile_masks(valid), 1.0 / math.sqrt(D)
+    kv = None if valid is None else valid.to(torch.uint8)
+    klists = ops.transpose_lists(*lists, BH, Ntq, Ntk)
+    qpair, kpair = ops.pair_tiles(*lists, Ntq, Ntk), ops.pair_tiles(*klists, Ntk, Ntq)
+    qun = ops.pair_union(*lists, Ntq, tm, col_tiles=Ntk, pairmap=qpair)
+    kun = ops.pair_union(*klists, Ntk, None, col_tiles=Ntq, pairmap=kpair)
+    kwhole = min(whole, BH * Ntk // 2)
+    qit = ops.part_union(*lists, Ntq, whole, splits, tm, col_tiles=Ntk, pairmap=qpair)
+    kit = ops.part_union(*klists, Ntk, kwhole, splits, None, col_tiles=Ntq, pairmap=kpair)
+    for un, it, w in ((qun, qit, whole), (kun, kit, kwhole)):
+        us, ul, uc = (host(t) for t in un)
+        s, n, c = (host(t) for t in it)
+        assert n.size == w + (ul.size - w) * splits
+        for i in range(n.size):
+            p, part = (i, -1) if i < w else (w + (i - w) // splits, (i - w) % splits)
+            e = uc[us[p]: us[p] + ul[p]]
+            assert np.array_equal(c[s[i]: s[i] + n[i]], e if part < 0 else e[(e >> 6) % splits == part]), i
+    o, lse = ops.bsa_fwd(q, k, v, tm, qun, sm, qpair)
+    m2, delta = ops.lse_to_m2(lse), ops.bwd_preprocess(o, do)
+    ref = ops.bsa_bwd(q, k, v, do, m2, delta, kv, tm, qun, kun, sm, qpair, kpair)
+    order = lambda u: torch.randperm(u[1].numel(), device="cuda").int()
+    one = (order(qit), order(kit))
+    got = [ops.bsa_bwd(q, k, v, do, m2, delta, kv, tm, qit, kit, sm, qpair, kpair, *od, q_split=(whole, splits),
+                       k_split=(kwhole, splits)) for od in (one, (None, None))]
+    for name, a, b, c in zip(("dq", "dk", "dv"), ref, *got):
+        assert bits_equal(host(b), host(c)), name  # the launch order changes nothing
+        # the same float32 products in another order of summation, rounded to
+        # bf16 once: at most one bf16 step (2^-7 of the value) apart, plus the
+        # float32 rounding of at most 60 x 64 terms, well below 2^-10 of the
+        # tensor's root mean square
+        x, y = a.float(), b.float()
+        assert bool(((x - y).abs() <= 2.0 ** -7 * x.abs() + 2.0 ** -10 * x.pow(2).mean().sqrt()).all()), name
+        if splits == 1:
+            assert bits_equal(host(a), host(b)), name
+
+
+def test_split_plan_covers_the_gpu():
+    """split_plan cuts only launches of a few rounds over long lists, at a
+    group boundary, and never makes more items than it has workgroups for
+    eight rounds."""
+    from prism_amd import ops
+    for kernel in (1, 2):
+        for heads, per_head in ((1, 1), (5, 16), (3, 720), (1, 37), (24, 2000)):
+            for entries in (32, 511, 512, 6900):
+                whole, splits = ops.split_plan(kernel, heads, per_head, entries, 128)
+                pairs = heads * per_head
+                assert 0 <= whole <= pairs and 1 <= splits <= 16
+                assert (whole == pairs) == (splits == 1)
+                assert splits == 1 or (entries >= 512 and (whole % per_head) % 4 == 0)
+                assert whole + (pairs - whole) * splits <= max(pairs, 8 * 512)
+
+
+def test_operators_opcheck():
+    from prism_amd import ops
+    q, k, v, do, lists, _ = make(3, 1, 4, 6, 64, 6, False)
+    P = torch.ops.prism
+
+    def chk(op, args):
+        torch.library.opcheck(op.default, args, test_utils=UTILS)
+
+    rows = ops.tile_lists(*lists, 4, None, 6)
+    chk(P.tile_lists, (*lists, 4, 6, None))
+    chk(P.bsa_fwd_tile, (q, k, v, None, *rows, 0.125))
+    items = ops.part_union(*lists, 4, 1, 2, None, col_tiles=6)
+    chk(P.part_union, (*lists, 4, 6, None, None, 1, 2))
+    o, lse = ops.bsa_fwd_tile(q, k, v, None, rows, 0.125)
+    m2, delta = ops.lse_to_m2(lse), ops.bwd_preprocess(o, do)
+    chk(P.bsa_bwd_dq_split, (q, k, v, do, m2, delta, None, *items, None, None, 0.125, 1, 2))
+    kit = ops.part_union(*ops.transpose_lists(*lists, 1, 4, 6), 6, 1, 2, None, col_tiles=4)
+    chk(P.bsa_bwd_dkdv_split, (q, k, v, do, m2, delta, None, *kit, None, None, 0.125, 1, 2))
