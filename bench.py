@@ -684,6 +684,8 @@ def main():
     attn = {"prism_bsa_fwd": (4 * fl, 4 * fl), "prism_bsa_bwd_dkdv": (8 * fl, 8 * fl),
             "prism_bsa_bwd_dq": (2 * fl, 6 * fl)}
     attn.update({n + "_quad": attn[n] for n in ("prism_bsa_fwd", "prism_bsa_bwd_dq")})
+    attn.update({n + s: attn[n] for n, s in (("prism_bsa_fwd", "_either"), ("prism_bsa_fwd", "_tile"),
+                                             ("prism_bsa_bwd_dq", "_split"), ("prism_bsa_bwd_dkdv", "_split"))})
     X = B * H * Sp * D * 2   # one bf16 [B,H,S_p,D] tile-order tensor (zone grid)
     Xin = B * H * S * D * 2  # one bf16 [B,H,S,D] THW tensor (input grid)
     nnz_tiles = int(plan.sel["ntiles"].sum().item())
@@ -1057,6 +1059,8 @@ def run_uniform(args, inp):
     attn = {"prism_bsa_fwd": (4 * fl, 4 * fl), "prism_bsa_bwd_dkdv": (8 * fl, 8 * fl),
             "prism_bsa_bwd_dq": (2 * fl, 6 * fl)}
     attn.update({n + "_quad": attn[n] for n in ("prism_bsa_fwd", "prism_bsa_bwd_dq")})
+    attn.update({n + s: attn[n] for n, s in (("prism_bsa_fwd", "_either"), ("prism_bsa_fwd", "_tile"),
+                                             ("prism_bsa_bwd_dq", "_split"), ("prism_bsa_bwd_dkdv", "_split"))})
     X_in, X_rows = B * H * S * D * 2, B * H * lq.rows * D * 2
     hbm = {"prism_chunk_gather_pool": (4 * (X_in + X_rows) + X_rows) / 4,  # q, k, v, dO (+ O for delta)
            "prism_chunk_scatter_rows": X_rows + X_in,

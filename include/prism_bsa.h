@@ -297,6 +297,16 @@ int prism_pair_tiles(const int64_t* start, const int32_t* len, const int32_t* co
  * counterpart in the reference (its launch order is the hardware's). */
 int prism_pair_order(const int32_t* ulen, int64_t n, int G, int64_t tail, int32_t* order, hipStream_t stream);
 
+/* Launch order of an attention kernel over n work lists: every run of seg
+ * consecutive lists (seg <= 16384; a head's, say), longest first (then the
+ * lower list), the runs one after the other.  With chunk > 1, inside a run each
+ * 8 * chunk consecutive ranks are dealt to the 8 XCDs in runs of chunk (launch
+ * position b runs on XCD b mod 8), in reverse every second time.  total (one
+ * int64 on the device, or NULL) = the sum of ulen.  Changes no result.  No
+ * counterpart in the reference. */
+int prism_launch_order(const int32_t* ulen, int64_t n, int64_t seg, int chunk, int32_t* order, int64_t* total,
+                       hipStream_t stream);
+
 /* Key validity per 64-token tile (the reference's kv_valid_mask,
  * bsa_interface.py:328-385, flash_attn_bsa_varlen_mask.py:263-295) packed as
  * masks[t] bit j = valid[64 t + j] != 0.  valid: [Nt*64] uint8 tile order. */
@@ -348,6 +358,20 @@ int prism_bsa_fwd_quad(const void* q, const void* k, const void* v, int BH, int6
                        const uint64_t* tile_masks, const int64_t* ustart, const int32_t* ulen, const int32_t* ucols,
                        const int32_t* quadmap, const int32_t* order, float sm_scale, void* o, float* lse,
                        int32_t* work_counter, hipStream_t stream);
+
+/* prism_bsa_fwd or prism_bsa_fwd_quad, whichever the lists favour (no
+ * counterpart in the reference; the same outputs bit for bit either way): p_*
+ * are the pair unions, q_* the quad unions of the same lists, both built with
+ * pairmap, with their launch orders and, on the device, the sums of their
+ * lengths (prism_launch_order).  Both kernels are launched and one of them
+ * returns at once: the quads run where 2 * *p_total >= 3 * *q_total.
+ * work_counter: 16 int32, not NULL. */
+int prism_bsa_fwd_either(const void* q, const void* k, const void* v, int BH, int64_t Sq, int64_t Sk, int D,
+                         const uint64_t* tile_masks, const int64_t* p_ustart, const int32_t* p_ulen,
+                         const int32_t* p_ucols, const int32_t* p_order, const int64_t* p_total,
+                         const int64_t* q_ustart, const int32_t* q_ulen, const int32_t* q_ucols,
+                         const int32_t* q_order, const int64_t* q_total, const int32_t* pairmap, float sm_scale,
+                         void* o, float* lse, int32_t* work_counter, hipStream_t stream);
 
 /* prism_bsa_fwd for launches of few pairs (no counterpart in the reference):
  * one workgroup per query tile, the same outputs bit for bit.  ustart / ulen /

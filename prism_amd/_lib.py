@@ -53,6 +53,8 @@ SIGNATURES = {
     "prism_bsa_bwd_dkdv": [P, P, P, P, P, P, I32, I64, I64, I32, P, P, P, P, P, P, F32, P, P, P, P],
     "prism_bsa_bwd_dq": [P, P, P, P, P, P, I32, I64, I64, I32, P, P, P, P, P, P, F32, P, P, P],
     "prism_bsa_bwd_dq_quad": [P, P, P, P, P, P, I32, I64, I64, I32, P, P, P, P, P, P, F32, P, P, P],
+    "prism_launch_order": [P, I64, I64, I32, P, P, P],
+    "prism_bsa_fwd_either": [P, P, P, I32, I64, I64, I32, P, P, P, P, P, P, P, P, P, P, P, P, F32, P, P, P, P],
     "prism_split_plan": [I32, I64, I64, I64, I32, P, P],
     "prism_part_union": [P, P, P, I64, I64, I64, P, P, I64, I32, I64, P, P, P, P],
     "prism_tile_lists": [P, P, P, I64, I64, I64, P, I64, P, P, P, P],

@@ -234,3 +234,12 @@ def _register_fakes():
         rows = start.numel()
         return (_empty(start, (rows,), i64), _empty(start, (rows,), i32),
                 _empty(start, (max(rows * col_tiles, 1),), i32))
+
+    @reg("prism::launch_order")
+    def _(ulen, seg, chunk):
+        return _empty(ulen, (ulen.numel(),), i32), _empty(ulen, (1,), i64)
+
+    @reg("prism::bsa_fwd_either")
+    def _(q, k, v, tile_masks, pustart, pulen, pucols, porder, ptotal, qustart, qulen, qucols, qorder, qtotal, pairmap,
+          sm_scale):
+        return _empty(q, q.shape, q.dtype), _empty(q, q.shape[:3], f32)

@@ -61,7 +61,14 @@ struct FwdArgs {
   float* lse;              // [BH, Sq] natural log
   int total;               // pairs of the launch (BH * npairs)
   int* queue;              // work-queue counter (persistent launch), or null: one pair per workgroup
+  const int64_t *p_total, *q_total;  // prism_bsa_fwd_either: entries of the pair and quad unions, else null
 };
+
+// Whether a launch of prism_bsa_fwd_either walks quads.  Quads stage fewer
+// tiles but idle the waves whose tile does not list one.  Pair entries over
+// quad entries, and the forward on pairs and quads (ms): 1.20: 47.6, 51.8;
+// 1.39: 25.9, 26.9; 1.65: 51.6, 49.0; 1.72: 63.0, 60.6.
+__device__ __forceinline__ bool walks_quads(const FwdArgs& a) { return 2 * *a.p_total >= 3 * *a.q_total; }
 
 constexpr int kStages = 2;      // two workgroups per CU: 2 x 2 stages of K and V fill the LDS
 constexpr int kStagesTile = 4;  // one workgroup per CU
@@ -511,6 +518,7 @@ template <int D>
 __global__ __launch_bounds__(512, 1) void bsa_fwd_quad_kernel(FwdArgs a) {
   __shared__ __align__(16) uint8_t smem[kStagesQuad * FwdTiles<D>::STAGE];
   __shared__ WorkQueueState wq;
+  if (a.p_total && !walks_quads(a)) return;
   work_queue_init(&wq);
   for (int pid = a.queue ? work_queue_take(a.queue, a.total, &wq) : (int)blockIdx.x; pid >= 0;
        pid = a.queue ? work_queue_take(a.queue, a.total, &wq) : -1) {
@@ -527,6 +535,7 @@ template <int D>
 __global__ __launch_bounds__(256, 2) void bsa_fwd_kernel(FwdArgs a) {
   __shared__ __align__(16) uint8_t smem[kStages * FwdTiles<D>::STAGE];
   __shared__ WorkQueueState wq;
+  if (a.p_total && walks_quads(a)) return;
   work_queue_init(&wq);
   for (int pid = a.queue ? work_queue_take(a.queue, a.total, &wq) : (int)blockIdx.x; pid >= 0;
        pid = a.queue ? work_queue_take(a.queue, a.total, &wq) : -1) {
@@ -572,7 +581,7 @@ int prism_bsa_fwd(const void* q, const void* k, const void* v, int BH, int64_t S
     PRISM_DEBUG_CHECK(prism_debug_check_maps("prism_bsa_fwd", pairmap, BH, Sq / 64, order, (int64_t)BH * (Sq / 128),
                                              stream));
   }
-  FwdArgs a;
+  FwdArgs a = {};
   a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v; a.tmask = tile_masks;
   a.ustart = ustart; a.ulen = ulen; a.ucols = ucols; a.pairmap = pairmap; a.order = order; a.Sq = Sq; a.Sk = Sk;
   a.npairs = (int)(Sq / 128);
@@ -587,6 +596,56 @@ int prism_bsa_fwd(const void* q, const void* k, const void* v, int BH, int64_t S
   if (D == 128) bsa_fwd_kernel<128><<<blocks, 256, 0, stream>>>(a);
   else bsa_fwd_kernel<64><<<blocks, 256, 0, stream>>>(a);
   PRISM_LAUNCH_CHECK("prism_bsa_fwd");
+  return PRISM_OK;
+}
+
+int prism_bsa_fwd_either(const void* q, const void* k, const void* v, int BH, int64_t Sq, int64_t Sk, int D,
+                         const uint64_t* tile_masks, const int64_t* p_ustart, const int32_t* p_ulen,
+                         const int32_t* p_ucols, const int32_t* p_order, const int64_t* p_total,
+                         const int64_t* q_ustart, const int32_t* q_ulen, const int32_t* q_ucols,
+                         const int32_t* q_order, const int64_t* q_total, const int32_t* pairmap, float sm_scale,
+                         void* o, float* lse, int32_t* work_counter, hipStream_t stream) {
+  PRISM_REQUIRE(q && k && v && p_ustart && p_ulen && p_ucols && p_total && q_ustart && q_ulen && q_ucols && q_total &&
+                    o && lse && work_counter,
+                "prism_bsa_fwd_either: null pointer");
+  PRISM_REQUIRE(D == 64 || D == 128, "prism_bsa_fwd_either: head_dim %d unsupported (64, 128)", D);
+  PRISM_REQUIRE(Sq > 0 && Sq % 256 == 0 && Sk > 0 && Sk % 128 == 0,
+                "prism_bsa_fwd_either: Sq must be a positive multiple of 256, Sk of 128");
+  PRISM_REQUIRE(BH >= 1 && (int64_t)BH * (Sq / 128) < (1ll << 31), "prism_bsa_fwd_either: grid too large");
+  const int64_t pairs = (int64_t)BH * (Sq / 128);
+  if (prism_debug_enabled()) {
+    PRISM_DEBUG_CHECK(prism_debug_check_lists("prism_bsa_fwd_either", p_ustart, p_ulen, p_ucols, pairs, Sk / 64, 1,
+                                              tile_masks, stream));
+    PRISM_DEBUG_CHECK(prism_debug_check_lists("prism_bsa_fwd_either", q_ustart, q_ulen, q_ucols, pairs / 2, Sk / 64, 2,
+                                              tile_masks, stream));
+    PRISM_DEBUG_CHECK(prism_debug_check_maps("prism_bsa_fwd_either", pairmap, BH, Sq / 64, p_order, pairs, stream));
+    PRISM_DEBUG_CHECK(prism_debug_check_maps("prism_bsa_fwd_either", nullptr, BH, Sq / 64, q_order, pairs / 2, stream));
+  }
+  FwdArgs a = {};
+  a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v; a.tmask = tile_masks;
+  a.pairmap = pairmap; a.Sq = Sq; a.Sk = Sk;
+  a.scale_log2 = sm_scale * 1.4426950408889634f;
+  a.o = (uint16_t*)o; a.lse = lse;
+  a.p_total = p_total; a.q_total = q_total;
+  FwdArgs b = a;
+  a.ustart = p_ustart; a.ulen = p_ulen; a.ucols = p_ucols; a.order = p_order;
+  a.npairs = (int)(Sq / 128);
+  a.total = (int)pairs;
+  a.queue = work_counter;
+  b.ustart = q_ustart; b.ulen = q_ulen; b.ucols = q_ucols; b.order = q_order;
+  b.npairs = (int)(Sq / 256);
+  b.total = (int)(pairs / 2);
+  b.queue = work_counter + kQueueLanes;
+  zero_counter_kernel<<<1, 2 * kQueueLanes, 0, stream>>>(work_counter);
+  auto grid = [](int res, int total) { return (unsigned)(res < total ? res : total); };
+  if (D == 128) {
+    bsa_fwd_quad_kernel<128><<<grid(resident_workgroups<bsa_fwd_quad_kernel<128>>(512), b.total), 512, 0, stream>>>(b);
+    bsa_fwd_kernel<128><<<grid(resident_workgroups<bsa_fwd_kernel<128>>(256), a.total), 256, 0, stream>>>(a);
+  } else {
+    bsa_fwd_quad_kernel<64><<<grid(resident_workgroups<bsa_fwd_quad_kernel<64>>(512), b.total), 512, 0, stream>>>(b);
+    bsa_fwd_kernel<64><<<grid(resident_workgroups<bsa_fwd_kernel<64>>(256), a.total), 256, 0, stream>>>(a);
+  }
+  PRISM_LAUNCH_CHECK("prism_bsa_fwd_either");
   return PRISM_OK;
 }
 
@@ -631,7 +690,7 @@ int prism_bsa_fwd_quad(const void* q, const void* k, const void* v, int BH, int6
     PRISM_DEBUG_CHECK(prism_debug_check_maps("prism_bsa_fwd_quad", quadmap, BH, Sq / 64, order,
                                              (int64_t)BH * (Sq / 256), stream));
   }
-  FwdArgs a;
+  FwdArgs a = {};
   a.q = (const uint16_t*)q; a.k = (const uint16_t*)k; a.v = (const uint16_t*)v; a.tmask = tile_masks;
   a.ustart = ustart; a.ulen = ulen; a.ucols = ucols; a.pairmap = quadmap; a.order = order; a.Sq = Sq; a.Sk = Sk;
   a.npairs = (int)(Sq / 256);  // quads per head

@@ -277,6 +277,105 @@ __global__ __launch_bounds__(1024) void pair_order_kernel(const int32_t* __restr
   for (int i = threadIdx.x; i < T; i += blockDim.x) order[k + i] = (int32_t)(key[i] & 0xffffffffu);
 }
 
+// ------------------------------------------------------------------ head order
+// Launch order of the attention launches: every run of `seg` consecutive lists
+// (a head's) longest first, the runs one after the other.  Workgroups that run
+// at the same time then walk lists of nearly one length of one head, so they
+// cross its key tiles at nearly one pace and meet in the L2, and no long list
+// starts late.  Against pair_order_kernel's order (only the launch's last
+// quarter sorted), 302,400 tokens, 5 heads: pair forward 54.0 -> 51.7 ms, dQ
+// 58.0 -> 55.5, quad forward 52.5 -> 51.8; 171,360 tokens, 3 heads: 12.4 ->
+// 11.4, 13.9 -> 13.2, 12.7 -> 11.4 ms.  Sorting all heads together takes
+// another 7% off dQ there but costs 10% and more once the heads' K and V
+// outgrow the Infinity Cache (the caller picks seg).
+// With chunk > 1, runs of `chunk` consecutive ranks go to one XCD (launch
+// position b runs on XCD b mod 8), every second round of XCDs in reverse so
+// that no XCD gets all the long lists: the workgroups of one L2 then walk
+// lists of one length (pair forward, 302,400 tokens: 51.7 -> 47.6 ms; dQ and
+// the quad forward lose 2%, dK/dV gains nothing, so only the pair forward
+// asks for it).
+// One workgroup sorts a run: a bitonic network over EPT keys per thread in
+// registers (thread t holds positions t EPT ..), whose steps of less than a
+// wave's reach use lane shuffles and only the rest LDS and barriers (4,096
+// lists: 10 of 78 steps; 20 us against 35 with every step in LDS).
+constexpr int kSegMax = 16384;  // lists per run
+
+template <int EPT>
+__global__ __launch_bounds__(1024) void launch_order_kernel(const int32_t* __restrict__ ulen, int n, int seg,
+                                                            int chunk, int32_t* __restrict__ order,
+                                                            int64_t* __restrict__ total) {
+  __shared__ uint32_t xch[1024 * EPT];
+  __shared__ int64_t wsum[16];
+  const int tid = threadIdx.x, base = (int)blockIdx.x * seg, m = min(seg, n - base);
+  if (total && blockIdx.x == 0) {
+    int64_t t = 0;
+    for (int i = tid; i < n; i += 1024) t += ulen[i];
+    t = (int64_t)wave_sum_u64((uint64_t)t);
+    if ((tid & 63) == 0) wsum[tid >> 6] = t;
+    __syncthreads();
+    if (tid == 0) {
+      t = 0;
+      for (int i = 0; i < 16; ++i) t += wsum[i];
+      *total = t;
+    }
+  }
+  // (2^18 - 1 - length) << 14 | list: ascending = longest first, then lower list
+  uint32_t key[EPT];
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) {
+    const int i = tid * EPT + e;
+    key[e] = i < m ? (0x3ffffu - (uint32_t)min(ulen[base + i], 0x3ffff)) << 14 | (uint32_t)i : 0xffffffffu;
+  }
+  for (int size = 2; size <= 1024 * EPT; size <<= 1)
+    for (int stride = size >> 1; stride > 0; stride >>= 1) {
+      if (stride >= EPT) {
+        // partners hold the same slot e of thread tid ^ (stride / EPT)
+        uint32_t other[EPT];
+        const int ts = stride / EPT;
+        if (ts < 64) {
+#pragma unroll
+          for (int e = 0; e < EPT; ++e) other[e] = (uint32_t)__shfl_xor((int)key[e], ts, 64);
+        } else {
+          __syncthreads();
+#pragma unroll
+          for (int e = 0; e < EPT; ++e) xch[e * 1024 + tid] = key[e];
+          __syncthreads();
+#pragma unroll
+          for (int e = 0; e < EPT; ++e) other[e] = xch[e * 1024 + (tid ^ ts)];
+        }
+        // (size > stride >= EPT: one direction for all of the thread's slots)
+        const bool low = ((tid & ts) == 0) == ((tid * EPT & size) == 0);
+#pragma unroll
+        for (int e = 0; e < EPT; ++e) key[e] = low ? min(key[e], other[e]) : max(key[e], other[e]);
+      } else {
+#pragma unroll
+        for (int st = EPT / 2; st > 0; st >>= 1)
+          if (st == stride) {
+#pragma unroll
+            for (int e = 0; e < EPT; ++e)
+              if ((e & st) == 0) {
+                const bool up = ((tid * EPT + e) & size) == 0;
+                const uint32_t x = key[e], y = key[e | st];
+                key[e] = up ? min(x, y) : max(x, y);
+                key[e | st] = up ? max(x, y) : min(x, y);
+              }
+          }
+      }
+    }
+  const int round = 8 * chunk, full = m / round * round;
+#pragma unroll
+  for (int e = 0; e < EPT; ++e) {
+    const int r = tid * EPT + e;
+    if (r >= m) continue;
+    int b = r;
+    if (chunk > 1 && r < full) {
+      const int c = r / round, x = (r % round) / chunk;
+      b = c * round + 8 * (r % chunk) + ((c & 1) ? 7 - x : x);
+    }
+    order[base + b] = base + (int)(key[e] & 0x3fffu);
+  }
+}
+
 // ------------------------------------------------------------------ compact CSR
 // offsets[r] = sum of len[0..r) as int32, *total = the int64 sum (so the
 // caller can reject a total past int32).  One workgroup: thread t sums a
@@ -495,6 +594,24 @@ int prism_pair_order(const int32_t* ulen, int64_t n, int G, int64_t tail, int32_
   const unsigned blocks = (unsigned)(head > 0 ? (head + 1023) / 1024 : 1);
   pair_order_kernel<<<blocks < 1 ? 1 : blocks, 1024, 0, stream>>>(ulen, (int)n, G, (int)tail, P2, order);
   PRISM_LAUNCH_CHECK("prism_pair_order");
+  return PRISM_OK;
+}
+
+int prism_launch_order(const int32_t* ulen, int64_t n, int64_t seg, int chunk, int32_t* order, int64_t* total,
+                       hipStream_t stream) {
+  PRISM_REQUIRE(ulen && order, "prism_launch_order: null pointer");
+  PRISM_REQUIRE(n >= 1 && n < (1ll << 31), "prism_launch_order: n out of range");
+  PRISM_REQUIRE(seg >= 1 && seg <= kSegMax, "prism_launch_order: seg must be in [1, %d]", kSegMax);
+  PRISM_REQUIRE(chunk >= 1 && chunk <= 1024, "prism_launch_order: chunk must be in [1, 1024]");
+  if (seg > n) seg = n;
+  const unsigned g = (unsigned)((n + seg - 1) / seg);
+  const int N = (int)n, S = (int)seg;
+  if (seg <= 1024) launch_order_kernel<1><<<g, 1024, 0, stream>>>(ulen, N, S, chunk, order, total);
+  else if (seg <= 2048) launch_order_kernel<2><<<g, 1024, 0, stream>>>(ulen, N, S, chunk, order, total);
+  else if (seg <= 4096) launch_order_kernel<4><<<g, 1024, 0, stream>>>(ulen, N, S, chunk, order, total);
+  else if (seg <= 8192) launch_order_kernel<8><<<g, 1024, 0, stream>>>(ulen, N, S, chunk, order, total);
+  else launch_order_kernel<16><<<g, 1024, 0, stream>>>(ulen, N, S, chunk, order, total);
+  PRISM_LAUNCH_CHECK("prism_launch_order");
   return PRISM_OK;
 }
 

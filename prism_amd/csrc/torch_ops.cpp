@@ -567,6 +567,17 @@ Tensor lists_csr_fill(const Tensor& s_, const Tensor& l_, const Tensor& c_, cons
   return out;
 }
 
+std::tuple<Tensor, Tensor> launch_order(const Tensor& ulen_, int64_t seg, int64_t chunk) {
+  on_gpu(ulen_, "ulen");
+  check_dtype(ulen_, at::kInt, "ulen");
+  const c10::DeviceGuard guard(ulen_.device());
+  const Tensor ulen = ulen_.contiguous();
+  Tensor order = at::empty({ulen.numel()}, opts(ulen, at::kInt)), total = at::empty({1}, opts(ulen, at::kLong));
+  PRISM_TORCH_CALL(prism_launch_order, ulen.data_ptr<int32_t>(), ulen.numel(), seg, (int)chunk,
+                   order.data_ptr<int32_t>(), total.data_ptr<int64_t>(), stream_of(ulen));
+  return {order, total};
+}
+
 Tensor pair_order(const Tensor& ulen_, int64_t group, int64_t tail) {
   on_gpu(ulen_, "ulen");
   check_dtype(ulen_, at::kInt, "ulen");
@@ -661,6 +672,39 @@ std::tuple<Tensor, Tensor> bsa_fwd(const Tensor& q_, const Tensor& k_, const Ten
                    (const uint64_t*)p(masks), us.data_ptr<int64_t>(), ul.data_ptr<int32_t>(), uc.data_ptr<int32_t>(),
                    (const int32_t*)p(pairmap), (const int32_t*)p(order), (float)sm_scale, o.data_ptr(),
                    lse.data_ptr<float>(), work_counter(q).data_ptr<int32_t>(), stream_of(q));
+  return {o, lse};
+}
+
+std::tuple<Tensor, Tensor> bsa_fwd_either(const Tensor& q_, const Tensor& k_, const Tensor& v_, const OptT& masks_,
+                                          const Tensor& pus_, const Tensor& pul_, const Tensor& puc_,
+                                          const OptT& porder_, const Tensor& ptotal, const Tensor& qus_,
+                                          const Tensor& qul_, const Tensor& quc_, const OptT& qorder_,
+                                          const Tensor& qtotal, const OptT& pairmap_, double sm_scale) {
+  const AttnShape s = attn_shape(q_, k_, v_);
+  check_union(pus_, pul_, puc_);
+  check_union(qus_, qul_, quc_);
+  on_gpu(masks_, "tile_masks");
+  on_gpu(pairmap_, "pairmap");
+  on_gpu(porder_, "porder");
+  on_gpu(qorder_, "qorder");
+  on_gpu(ptotal, "ptotal");
+  on_gpu(qtotal, "qtotal");
+  check_dtype(ptotal, at::kLong, "ptotal");
+  check_dtype(qtotal, at::kLong, "qtotal");
+  const c10::DeviceGuard guard(q_.device());
+  const Tensor q = q_.contiguous(), k = k_.contiguous(), v = v_.contiguous();
+  const Tensor pus = pus_.contiguous(), pul = pul_.contiguous(), puc = puc_.contiguous();
+  const Tensor qus = qus_.contiguous(), qul = qul_.contiguous(), quc = quc_.contiguous();
+  const OptT masks = cont(masks_), pairmap = cont(pairmap_), porder = cont(porder_), qorder = cont(qorder_);
+  Tensor o = at::empty_like(q);
+  Tensor lse = at::empty({s.B, s.H, s.Sq}, opts(q, at::kFloat));
+  Tensor counter = at::empty({16}, opts(q, at::kInt));
+  PRISM_TORCH_CALL(prism_bsa_fwd_either, q.data_ptr(), k.data_ptr(), v.data_ptr(), (int)(s.B * s.H), s.Sq, s.Sk,
+                   (int)s.D, (const uint64_t*)p(masks), pus.data_ptr<int64_t>(), pul.data_ptr<int32_t>(),
+                   puc.data_ptr<int32_t>(), (const int32_t*)p(porder), ptotal.data_ptr<int64_t>(),
+                   qus.data_ptr<int64_t>(), qul.data_ptr<int32_t>(), quc.data_ptr<int32_t>(),
+                   (const int32_t*)p(qorder), qtotal.data_ptr<int64_t>(), (const int32_t*)p(pairmap), (float)sm_scale,
+                   o.data_ptr(), lse.data_ptr<float>(), counter.data_ptr<int32_t>(), stream_of(q));
   return {o, lse};
 }
 
@@ -898,6 +942,10 @@ TORCH_LIBRARY(prism, m) {
         "Tensor? tile_masks, int whole, int splits) -> (Tensor, Tensor, Tensor)");
   m.def("tile_lists(Tensor start, Tensor len, Tensor cols, int row_tiles, int col_tiles, Tensor? tile_masks) "
         "-> (Tensor, Tensor, Tensor)");
+  m.def("launch_order(Tensor ulen, int seg, int chunk) -> (Tensor, Tensor)");
+  m.def("bsa_fwd_either(Tensor q, Tensor k, Tensor v, Tensor? tile_masks, Tensor pustart, Tensor pulen, Tensor pucols, "
+        "Tensor? porder, Tensor ptotal, Tensor qustart, Tensor qulen, Tensor qucols, Tensor? qorder, Tensor qtotal, "
+        "Tensor? pairmap, float sm_scale) -> (Tensor, Tensor)");
   m.def("bsa_fwd_tile(Tensor q, Tensor k, Tensor v, Tensor? tile_masks, Tensor ustart, Tensor ulen, Tensor ucols, "
         "float sm_scale) -> (Tensor, Tensor)");
   m.def("bsa_bwd_dkdv_split(Tensor q, Tensor k, Tensor v, Tensor do, Tensor m2, Tensor delta, Tensor? kv_valid, "
@@ -944,6 +992,8 @@ TORCH_LIBRARY_IMPL(prism, CUDA, m) {
   m.impl("bsa_bwd_dq_quad", &bsa_bwd_dq_quad);
   m.impl("part_union", &part_union);
   m.impl("tile_lists", &tile_lists);
+  m.impl("launch_order", &launch_order);
+  m.impl("bsa_fwd_either", &bsa_fwd_either);
   m.impl("bsa_fwd_tile", &bsa_fwd_tile);
   m.impl("bsa_bwd_dkdv_split", &bsa_bwd_dkdv_split);
   m.impl("bsa_bwd_dq_split", &bsa_bwd_dq_split);

@@ -457,15 +457,24 @@ class DeferredCompaction:
         ev.record()
         self.offsets[i], self.events[i] = off, ev
 
-    def finish(self, lists_seq):
-        """lists_seq[i]: the lists added as i; others come back as they are."""
+    def sizes(self):
+        """Entries of every list added (waits for the copies; slots never
+        added hold nothing meaningful)."""
         for ev in self.events:
             if ev is not None:
                 ev.synchronize()
-        nnz = self.host.tolist()
-        return [lists if self.offsets[i] is None else
-                (*csr_lists(self.offsets[i]), csr_fill(*lists, self.offsets[i], nnz[i]))
-                for i, lists in enumerate(lists_seq)]
+        return self.host.tolist()
+
+    def fill(self, i: int, lists):
+        """CSR form of the lists added as i; lists never added come back as
+        they are."""
+        if self.offsets[i] is None:
+            return lists
+        return (*csr_lists(self.offsets[i]), csr_fill(*lists, self.offsets[i], self.sizes()[i]))
+
+    def finish(self, lists_seq):
+        """fill of every list: lists_seq[i] was added as i."""
+        return [self.fill(i, lists) for i, lists in enumerate(lists_seq)]
 
 
 def csr_lists(offsets: torch.Tensor):
@@ -620,11 +629,44 @@ def part_union(start: torch.Tensor, length: torch.Tensor, cols: torch.Tensor, Nt
                int(whole), int(splits))
 
 
-def items_order(ulen: torch.Tensor, group: int) -> Optional[torch.Tensor]:
-    """Launch order of an attention launch (group: 64 for the forward and dQ,
-    32 for dK/dV), longest lists first in its last quarter; None when all of
-    its work items run at once."""
-    return pair_order(ulen, group) if ulen.numel() > 8 * group else None
+def launch_order(ulen: torch.Tensor, heads: int, cache_bytes: int, chunk: int = 1):
+    """(order int32 [n], total int64 [1]) of an attention launch over the lists
+    of `heads` heads: each head's lists longest first, or all heads' together
+    when the operands they read (cache_bytes) fit the Infinity Cache; total is
+    the sum of the lengths (prism_launch_order)."""
+    _cuda(ulen)
+    n = ulen.numel()
+    seg = n if n <= SEGMENT_MAX and cache_bytes <= CACHE_BYTES else -(-n // heads)
+    if seg > SEGMENT_MAX:
+        seg = -(-seg // -(-seg // SEGMENT_MAX))
+    return _op("launch_order", ulen, int(seg), int(chunk))
+
+
+# ranks per XCD run of the pair forward's launch order
+FWD_CHUNK = 64
+SEGMENT_MAX = 16384
+# 256 MB of Infinity Cache; the launches' padded tiles are never read, so a
+# little more than that may pass (171,360 tokens of 3 heads, 318 MB with the
+# padding and 263 without, gain from one sorted run)
+CACHE_BYTES = 320 << 20
+
+
+def items_order(ulen: torch.Tensor, group: int, heads: int = 1, cache_bytes: int = 0,
+                chunk: int = 1) -> Optional[torch.Tensor]:
+    """launch_order of an attention launch (group: 64 for the forward and dQ,
+    32 for dK/dV); None when all of its work items run at once."""
+    return launch_order(ulen, heads, cache_bytes, chunk)[0] if ulen.numel() > 8 * group else None
+
+
+def bsa_fwd_either(q, k, v, tmasks, pairs, porder, ptotal, quads, qorder, qtotal, sm_scale: float, qpair=None):
+    """bsa_fwd over pair unions or bsa_fwd_quad over quad unions of the same
+    lists, decided on the device by the sums of their lengths (the same o and
+    lse, bit for bit)."""
+    _cuda(q, k, v, tmasks, qpair)
+    q, k, v = _bf16(q, "q"), _bf16(k, "k"), _bf16(v, "v")
+    _attn_shapes(q, k, v)
+    return _op("bsa_fwd_either", q, k, v, tmasks, *pairs, porder, ptotal, *quads, qorder, qtotal, qpair,
+               float(sm_scale))
 
 
 def tile_lists(start: torch.Tensor, length: torch.Tensor, cols: torch.Tensor, Nt: int,
@@ -686,15 +728,17 @@ OVERLAP_DKDV_SCATTER = False
 
 # The forward over quad unions (bsa_fwd_quad: four query tiles per staged K /
 # V tile, bit-identical to bsa_fwd) when the query tiles per head are a
-# multiple of 4; PRISM_QUADS=0 keeps the pair kernel.  dQ over the same quad
-# unions (bsa_bwd_dq_quad, bit-identical to bsa_bwd_dq; the plan then keeps
-# them for the backward): DQ_QUADS None (the default) takes it on the
-# dynamic-shape path and not on the uniform and cross paths; True / False
-# (PRISM_DQ_QUADS=1 / 0) force it either way.  The quads stage 42% fewer
-# tile bytes but leave more wave slots idle (24% against 8% for pairs at
-# config 4): forward 52.5 -> 49.7 ms there, dQ 59.6 -> 59.1 ms; on the
-# uniform path (35% idle) forward 56.1-57.0 -> 52.1 ms but dQ 60.6-60.7 ->
-# 61.5 ms.
+# multiple of 4, the launch has eight rounds of pairs and the lists favour it
+# (bsa_fwd_either); PRISM_QUADS=0 keeps the pair kernel.  dQ over the same
+# quad unions (bsa_bwd_dq_quad, bit-identical to bsa_bwd_dq; the plan then
+# keeps them for the backward): DQ_QUADS None (the default) takes it on the
+# dynamic-shape path where the pair unions hold at least DQ_QUAD_RATIO times
+# the quad unions' entries (known on the host when a compact plan settles),
+# and not on the uniform and cross paths; True / False (PRISM_DQ_QUADS=1 / 0)
+# force it on launches of eight rounds.  Pair over quad entries, dQ on pairs
+# and quads (ms): 1.20: 55.5, 62.3; 1.39: 31.9, 33.2; 1.65: 60.6, 60.9; 1.72:
+# 79.2, 76.8.
+DQ_QUAD_RATIO = 1.68
 QUADS = os.environ.get("PRISM_QUADS", "1") not in ("", "0")
 _dq_env = os.environ.get("PRISM_DQ_QUADS", "")
 DQ_QUADS: Optional[bool] = None if _dq_env == "" else _dq_env != "0"

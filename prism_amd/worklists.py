@@ -68,8 +68,13 @@ class _Side:
         """Launch order over pairs or items."""
         key = "items" if lists is self._items else "pairs"
         if key not in self._orders:
-            self._orders[key] = ops.items_order(lists[1], self.group)
+            self._orders[key] = ops.items_order(lists[1], self.group, self.BH, self.cache_bytes)
         return self._orders[key]
+
+    @property
+    def cache_bytes(self):
+        """bf16 operand rows that the lists index (K and V, or Q and dO)."""
+        return self.BH * self.cols * 64 * self.D * 4
 
 
 class WorkLists:
@@ -78,7 +83,7 @@ class WorkLists:
 
     A query side of fewer than eight rounds of workgroups walks pairs (its
     forward single tiles when there are few), whatever the quad switches say; a
-    larger one walks quads where they allow it."""
+    larger one walks pairs or quads, as the switches and the lists say."""
 
     def _build_query_lists(self, BH, Ntq, Ntk, D, tmasks, compact, dq_quads):
         self._BH, self._Ntq, self._Ntk, self._D = BH, Ntq, Ntk, D
@@ -95,11 +100,11 @@ class WorkLists:
         # staged K / V tile); quads: the call may walk them, dq_quads: dQ too
         self.quads = ops.QUADS and Ntq % 4 == 0
         self.dq_quads = self.quads and dq_quads
-        self._qquad = self._qquad_order = None
+        self._qquad = self._qquad_order = self._qquad_total = None
         self._shown = {}
         if self.quads and not self._q.small:
             self._qquad = self._query_quads()
-            self._qquad_order = ops.pair_order(self._qquad[1], 32)
+            self._qquad_order, self._qquad_total = ops.launch_order(self._qquad[1], BH, self._q.cache_bytes)
         self.klists = None
         self.keys_ready = None  # event of a key-list build on the side stream
 
@@ -229,9 +234,15 @@ class WorkLists:
             return
         self.build_key_lists()
         self._start_compaction()
+        if self.dq_quads and not self._q.small and ops.DQ_QUADS is None:
+            sizes = None if self._csr is None else self._csr.sizes()
+            self.dq_quads = sizes is not None and sizes[0] >= ops.DQ_QUAD_RATIO * sizes[2]
+        if not self.dq_quads and not self._q.small:
+            self._qquad = None
         if self._csr is not None:
-            self._q._pairs, self._k._pairs, self._qquad = self._csr.finish(
-                [self._q._pairs, self._k._pairs, self._qquad])
+            self._q._pairs, self._k._pairs = self._csr.finish([self._q._pairs, self._k._pairs])
+            if self._qquad is not None:
+                self._qquad = self._csr.fill(2, self._qquad)
             self._csr = None
         if not self.dq_quads or self._q.small:  # not walked by the backward
             self._qquad = self._qquad_order = None
@@ -276,7 +287,9 @@ class WorkLists:
         if self._few:
             out = ops.bsa_fwd_tile(*qkv, ops.tile_lists(*q.source, self._Ntq, self.tmasks, self._Ntk), sm_scale)
         elif self.quads and not q.small:
-            out = ops.bsa_fwd_quad(*qkv, self._qquad, sm_scale, q.pairmap, self._qquad_order)
+            order, total = ops.launch_order(q.pairs[1], self._BH, q.cache_bytes, ops.FWD_CHUNK)
+            out = ops.bsa_fwd_either(*qkv, q.pairs, order, total, self._qquad, self._qquad_order, self._qquad_total,
+                                     sm_scale, q.pairmap)
         else:
             out = ops.bsa_fwd(*qkv, q.pairs, sm_scale, q.pairmap, q.order(q.pairs))
         self.join_side()  # queued after the forward kernel: the key lists still run beside it

@@ -132,3 +132,71 @@ def test_operators_opcheck():
     chk(P.bsa_bwd_dq_split, (q, k, v, do, m2, delta, None, *items, None, None, 0.125, 1, 2))
     kit = ops.part_union(*ops.transpose_lists(*lists, 1, 4, 6), 6, 1, 2, None, col_tiles=4)
     chk(P.bsa_bwd_dkdv_split, (q, k, v, do, m2, delta, None, *kit, None, None, 0.125, 1, 2))
+
+
+@pytest.mark.parametrize("heads,per_head", [(1, 1), (3, 7), (2, 1024), (5, 1025), (2, 2600), (1, 5000), (1, 16384),
+                                            (2, 16500)], ids=str)
+def test_launch_order(heads, per_head):
+    """Each run longest first, then the lower list; total the sum; chunked
+    orders the same ranks dealt to the XCDs; lengths past the sort key's
+    range still give a permutation."""
+    from prism_amd import ops
+    n = heads * per_head
+    rng = np.random.default_rng(n)
+    u = rng.integers(0, 40, n).astype(np.int32)
+    ulen = torch.from_numpy(u).to("cuda")
+    say("launch order", (heads, per_head))
+    seg = -(-per_head // -(-per_head // 16384))
+    runs = [np.arange(b, min(b + seg, n)) for b in range(0, n, seg)]
+    want = np.concatenate([r[np.argsort(-u[r], kind="stable")] for r in runs])
+    order, total = ops.launch_order(ulen, heads, 1 << 40)
+    assert np.array_equal(host(order), want) and int(total) == int(u.sum())
+    chunked = host(ops.launch_order(ulen, heads, 1 << 40, 4)[0])
+    for r in runs:
+        ranks, got = want[r], chunked[r]
+        for c in range(len(r) // 32):
+            for x in range(8):
+                seg_x = 7 - x if c & 1 else x
+                assert np.array_equal(got[32 * c + x: 32 * c + 32: 8], ranks[32 * c + 4 * seg_x: 32 * c + 4 * seg_x + 4])
+        tail = len(r) // 32 * 32
+        assert np.array_equal(got[tail:], ranks[tail:])
+    if n <= 16384:
+        assert np.array_equal(host(ops.launch_order(ulen, heads, 0)[0]), np.argsort(-u, kind="stable"))
+    big = ops.launch_order(ulen * 100000, heads, 1 << 40)[0]
+    assert np.array_equal(np.sort(host(big)), np.arange(n))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("shared", [True, False])
+def test_fwd_either_walks_one(D, shared):
+    """The device's choice (quads when the tiles of a quad share their lists,
+    pairs when they do not) changes no bit; the kernel not chosen writes
+    nothing."""
+    from prism_amd import ops
+    BH, Nt, W = 2, 16, 5
+    say("fwd either", D, shared)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    q, k, v = (torch.randn((1, BH, Nt * 64, D), device="cuda", generator=g).to(torch.bfloat16) for _ in range(3))
+    rng = np.random.default_rng(5)
+    rows = [np.sort(rng.choice(Nt, W, replace=False)) for _ in range(BH * Nt)]
+    if shared:
+        rows = [rows[r // 8] for r in range(BH * Nt)]
+    dev = lambda a, t: torch.from_numpy(np.ascontiguousarray(a)).to("cuda", t)
+    lists = (dev(np.arange(BH * Nt) * W, torch.int64), dev(np.full(BH * Nt, W), torch.int32),
+             dev(np.concatenate(rows), torch.int32))
+    pm = ops.pair_tiles(*lists, Nt)
+    pairs, quads = ops.pair_union(*lists, Nt, pairmap=pm), ops.quad_union(*lists, Nt, pairmap=pm)
+    po, pt = ops.launch_order(pairs[1], BH, 0)
+    qo, qt = ops.launch_order(quads[1], BH, 0)
+    assert (2 * int(pt) >= 3 * int(qt)) == shared
+    want = ops.bsa_fwd(q, k, v, None, pairs, 0.1, pm)
+    got = ops.bsa_fwd_either(q, k, v, None, pairs, po, pt, quads, qo, qt, 0.1, pm)
+    assert all(bits_equal(host(a), host(b)) for a, b in zip(want, got))
+    # the choice is the totals': the other way round on the same lists
+    zero = torch.zeros_like(pt)
+    for a, b in ((zero, qt), (pt, zero)):
+        got = ops.bsa_fwd_either(q, k, v, None, pairs, None, a, quads, None, b, 0.1, pm)
+        assert all(bits_equal(host(x), host(y)) for x, y in zip(want, got))
+    torch.library.opcheck(torch.ops.prism.launch_order.default, (pairs[1], 8, 1), test_utils=UTILS)
+    torch.library.opcheck(torch.ops.prism.bsa_fwd_either.default,
+                          (q, k, v, None, *pairs, po, pt, *quads, qo, qt, pm, 0.1), test_utils=UTILS)
