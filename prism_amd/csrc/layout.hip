@@ -96,28 +96,57 @@ struct GatherArgs {
   float* rowdot;             // [B,H,S_out] fp32, or null
 };
 
-// Rearranged row r (0..511) of work unit u -> source token, for the two
-// layouts.  token() is -1 for a padding row (no source token); a block is
-// bsz consecutive rows starting at a multiple of bsz.
-//
+// Rearranged rows of work unit u (512 rows) -> source tokens, for the two
+// layouts.  The rows go by groups of 64 (a block has 64 or 128 rows, so a group
+// lies in one block): group() finds the block's origin once, with scalar
+// arithmetic, and token(o) of the group's row o is shifts and masks (every
+// extent of a block is a power of two: their product is 64 or 128); it is -1
+// for a padding row (no source token).  (With the block found by divisions
+// for every row, the gathers and scatters of 14,040 tokens x 5 heads took 45
+// and 40 us.)
+struct BlockRows {
+  int T, H, W;         // input grid
+  int lb, lh, lw;      // log2 of the block's rows, h extent and w extent
+  int t0, h0, w0, o0;  // the group's block origin, and its first row in the block
+  __device__ __forceinline__ int64_t token(int o) const {
+    const int off = o0 + o;
+    const int t = t0 + (off >> (lh + lw)), h = h0 + ((off >> lw) & ((1 << lh) - 1)), w = w0 + (off & ((1 << lw) - 1));
+    return t >= T || h >= H || w >= W ? -1 : ((int64_t)t * H + h) * W + w;
+  }
+};
+
 // ZoneMap: the dynamic layout.  Unit = zone z (512 rows); its blocks have the
-// zone's candidate shape (local_of_rearr) and are numbered from block_offset[z].
+// zone's candidate shape (blocks t-major, then h, then w, as local_of_rearr)
+// and are numbered from block_offset[z].
 struct ZoneMap {
   const int64_t* shape_ids;
   const int32_t* block_offset;
   int ZH, ZW;
   GridBox box;  // input grid (tokens outside it are padding)
-  int z, c, bsz, boff;
+  int z, bsz, boff, lt;
+  BlockRows g;
   __device__ __forceinline__ void init(int unit) {
     z = unit;
-    c = (int)shape_ids[z];
-    bsz = kCand[c][0] * kCand[c][1] * kCand[c][2];
+    const int c = (int)shape_ids[z];
+    lt = __builtin_ctz(kCand[c][0]);
+    g.lh = __builtin_ctz(kCand[c][1]);
+    g.lw = __builtin_ctz(kCand[c][2]);
+    g.lb = lt + g.lh + g.lw;
+    g.T = box.T; g.H = box.H; g.W = box.W;
+    bsz = 1 << g.lb;
     boff = block_offset ? block_offset[z] : 0;  // (the scatter needs no block numbers)
   }
   __device__ __forceinline__ int64_t row(int r) const { return (int64_t)z * 512 + r; }
   __device__ __forceinline__ bool live(int) const { return true; }
-  __device__ __forceinline__ int64_t token(int r) const { return token_in(z, local_of_rearr(c, r), ZH, ZW, box); }
-  __device__ __forceinline__ int64_t block(int r) const { return boff + r / bsz; }
+  __device__ __forceinline__ void group(int r) {
+    const int blk = r >> g.lb, nw = 3 - g.lw, nh = 3 - g.lh;  // (log2 of the zone's blocks along w and h)
+    const int zt = z / (ZH * ZW), zh = (z / ZW) % ZH, zw = z % ZW;
+    g.t0 = 8 * zt + ((blk >> (nw + nh)) << lt);
+    g.h0 = 8 * zh + (((blk >> nw) & ((1 << nh) - 1)) << g.lh);
+    g.w0 = 8 * zw + ((blk & ((1 << nw) - 1)) << g.lw);
+    g.o0 = r & (bsz - 1);
+  }
+  __device__ __forceinline__ int64_t block(int r) const { return boff + (r >> g.lb); }
 };
 
 // ChunkMap: the uniform 3-D chunk layout (rearrange_THW_to_3d_block,
@@ -128,33 +157,28 @@ struct ZoneMap {
 // flash_attn_bsa_cross, bsa_interface.py:1263-1273, 1318-1331) and rows past
 // Tp Hp Wp (tile-pair alignment) are padding.  Unit = 512 consecutive rows.
 struct ChunkMap {
-  int T, Hg, Wg;    // input grid
   int ct, ch, cw;   // chunk shape
   int Nh, Nw;       // chunks along padded h, w
   int64_t Sp;       // Tp Hp Wp
   int64_t S_out;    // rows per head (>= Sp)
   int bsz;          // ct ch cw
   int64_t base;
+  BlockRows g;      // T, H, W, lb, lh, lw set by the host
   __device__ __forceinline__ void init(int unit) { base = (int64_t)unit * 512; }
   __device__ __forceinline__ int64_t row(int r) const { return base + r; }
   __device__ __forceinline__ bool live(int r) const { return base + r < S_out; }
-  __device__ __forceinline__ int64_t token(int r) const {
+  __device__ __forceinline__ void group(int r) {
     const int64_t p = base + r;
-    if (p >= Sp) return -1;
-    const int64_t n = p / bsz;
-    const int off = (int)(p - n * bsz);
-    const int64_t nt = n / ((int64_t)Nh * Nw);
-    const int nh = (int)((n / Nw) % Nh), nw = (int)(n % Nw);
-    const int it = off / (ch * cw), ih = (off / cw) % ch, iw = off % cw;
-    const int64_t t = nt * ct + it;
-    const int h = nh * ch + ih, w = nw * cw + iw;
-    if (t >= T || h >= Hg || w >= Wg) return -1;
-    return (t * Hg + h) * Wg + w;
+    const uint32_t n = (uint32_t)(p >> g.lb), u = n / (uint32_t)Nw;  // (chunk_map bounds the chunks by 2^31)
+    g.t0 = p < Sp ? (int)(u / (uint32_t)Nh) * ct : g.T;  // (rows past Tp Hp Wp: no token)
+    g.h0 = (int)(u % (uint32_t)Nh) * ch;
+    g.w0 = (int)(n % (uint32_t)Nw) * cw;
+    g.o0 = (int)p & (bsz - 1);
   }
-  __device__ __forceinline__ int64_t block(int r) const { return (base + r) / bsz; }
+  __device__ __forceinline__ int64_t block(int r) const { return (base + r) >> g.lb; }
 };
 
-constexpr int kGatherThreads = 256;  // 4 waves, 128 rearranged rows each
+constexpr int kGatherThreads = 256;  // 4 waves
 
 // 8 channels of one row as floats (16 bytes of bf16 or 32 bytes of fp32)
 template <typename T>
@@ -174,149 +198,186 @@ __device__ __forceinline__ void load8(const T* p, float* x) {
   }
 }
 
-// grid (units, B*H).  Wave w covers rearranged rows [128 w, 128 w + 128) of
-// unit u (blocks of 64 or 128 rows: one or two whole blocks, two tiles).  A
-// lane moves 8 channels (16 bytes of bf16): D / 8 lanes per row, 64 / (D / 8)
-// rows per wave instruction, NB instructions in flight (fewer registers, more
-// waves per SIMD beat more loads per wave here).  Block means: row group g
-// (rows o of the block with o mod RPI = g, RPI = 512 / D) is summed in fp32
-// in row order from +0 by the lanes that load it, and the block sum is
-// ((p_0 + p_1) + ...) + p_{RPI-1}, formed by the first group's lanes when the
-// block is complete; padding rows are written as zeros, are invalid, and
-// belong to no block when they lie past the last block.
-template <int D, typename T, typename Map, bool POOL>
+// grid (units x 128 / RPW, B*H).  A wave covers RPW rearranged rows of its unit
+// (blocks of 64 or 128 rows).  A lane moves 8 channels (16 bytes of bf16): D / 8
+// lanes per row, 64 / (D / 8) rows per wave instruction, NB instructions in
+// flight.  Block means: row group g (rows o of the block with o mod RPI = g,
+// RPI = 512 / D) is summed in fp32 in row order from +0 by the lanes that load
+// it, and the block sum is ((p_0 + p_1) + ...) + p_{RPI-1}, formed by the first
+// group's lanes when the block is complete; padding rows are written as zeros,
+// are invalid, and belong to no block when they lie past the last block.
+// RPW = 128: a wave sums its one or two whole blocks, batch by batch.  RPW = 64
+// (launches of few workgroups): one batch per wave; of a block of 128 rows the
+// second wave takes over the first one's sums through LDS and goes on in row
+// order.
+template <int D, typename T, typename Map, bool POOL, int NB, int RPW>
 __global__ __launch_bounds__(kGatherThreads) void gather_pool_kernel(GatherArgs a, Map m) {
   constexpr int LPR = D / 8;     // lanes per row
   constexpr int RPI = 64 / LPR;  // rows per wave instruction
-  // wave instructions in flight: with pooling 2 (2: 0.256 ms, 4: 0.283, 8:
-  // 0.326 averaged over the step's launches at C4), without it 4
-  constexpr int NB = POOL ? 2 : 4;
   constexpr int RB = RPI * NB;   // rows per batch (inside one block and one tile)
-  static_assert(64 % RB == 0, "batches must not straddle tiles");
+  constexpr bool HALF = POOL && RPW == 64;
+  static_assert(64 % RB == 0 && RPW % RB == 0, "batches must not straddle tiles");
+  static_assert(!POOL || RPW == 128 || RB == 64, "pooling waves of 64 rows take them in one batch");
+  constexpr int SUBS = 128 / RPW;  // workgroups per unit
+  __shared__ float sAcc[HALF ? 4 : 1][8][HALF ? 64 : 1];
+  __shared__ int sCnt[4];
   const int bh = blockIdx.y;
-  const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int sub = lane / LPR, cl = lane % LPR, c8 = cl * 8;
-  m.init(blockIdx.x);
-  if (!m.live(wid * 128)) return;  // rows per head are a multiple of 128
+  m.init(blockIdx.x / SUBS);
+  const int r0 = (int)(blockIdx.x % SUBS) * 4 * RPW + wid * RPW;  // this wave's first row in the unit
+  const bool live = m.live(r0);                                   // rows per head are a multiple of 128
+  if (!HALF && !live) return;
   const bool first_bh = bh == 0;
   const T* x = reinterpret_cast<const T*>(a.x) + (int64_t)bh * a.S_in * D + c8;
   const int64_t rowbase = (int64_t)bh * a.S_out;
 
   float acc[8];
-  int cnt = 0, tcnt = 0;  // (meaningful in the first row group)
+  int cnt = 0, tcnt = 0;
 #pragma unroll
   for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
+  // the sums of this lane's row group of the block that ends at row rlast -> its mean
+  auto finish_block = [&](int rlast) {
+    const int64_t blk = m.block(rlast);
+    if (blk >= a.N_b) return;
+    if (a.block_mean) {
+      float sum[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sum[j] = acc[j];
+#pragma unroll
+      for (int g = 1; g < RPI; ++g)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) sum[j] = sum[j] + __shfl(acc[j], g * LPR + cl, 64);
+      if (sub == 0) {
+        const float den = (float)(cnt > 0 ? cnt : 1);
+        float* dst = a.block_mean + ((int64_t)bh * a.N_b + blk) * D + c8;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) dst[j] = sum[j] / den;
+      }
+    }
+    if (first_bh && lane == 0 && a.block_count) a.block_count[blk] = cnt;
+  };
 
-  for (int o0 = 0; o0 < 128; o0 += RB) {
+  for (int o0 = 0; o0 < RPW; o0 += RB) {
     float xv[NB][8];
     bool ok[NB];
     int64_t grow[NB];
+    if (live) {
+      if (RPW < 128 || (o0 & 63) == 0) m.group((r0 + o0) & ~63);
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int r = wid * 128 + o0 + b * RPI + sub;
-      const int64_t tok = m.token(r);
-      grow[b] = m.row(r);
-      ok[b] = tok >= 0 && (a.valid ? (a.valid[tok] != 0) : true);
-      if (tok >= 0) {
-        load8<T>(x + tok * D, xv[b]);
-      } else {
+      for (int b = 0; b < NB; ++b) {
+        const int r = r0 + o0 + b * RPI + sub;
+        const int64_t tok = m.g.token(r & 63);
+        grow[b] = m.row(r);
+        ok[b] = tok >= 0 && (a.valid ? (a.valid[tok] != 0) : true);
+        if (tok >= 0) {
+          load8<T>(x + tok * D, xv[b]);
+        } else {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) xv[b][j] = 0.0f;
+          for (int j = 0; j < 8; ++j) xv[b][j] = 0.0f;
+        }
       }
-    }
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      if (a.out_rows) {
-        uint4 u;
-        u.x = (uint32_t)f2bf(xv[b][0]) | ((uint32_t)f2bf(xv[b][1]) << 16);
-        u.y = (uint32_t)f2bf(xv[b][2]) | ((uint32_t)f2bf(xv[b][3]) << 16);
-        u.z = (uint32_t)f2bf(xv[b][4]) | ((uint32_t)f2bf(xv[b][5]) << 16);
-        u.w = (uint32_t)f2bf(xv[b][6]) | ((uint32_t)f2bf(xv[b][7]) << 16);
-        *reinterpret_cast<uint4*>(a.out_rows + (rowbase + grow[b]) * D + c8) = u;
+      for (int b = 0; b < NB; ++b) {
+        if (a.out_rows) {
+          uint4 u;
+          u.x = (uint32_t)f2bf(xv[b][0]) | ((uint32_t)f2bf(xv[b][1]) << 16);
+          u.y = (uint32_t)f2bf(xv[b][2]) | ((uint32_t)f2bf(xv[b][3]) << 16);
+          u.z = (uint32_t)f2bf(xv[b][4]) | ((uint32_t)f2bf(xv[b][5]) << 16);
+          u.w = (uint32_t)f2bf(xv[b][6]) | ((uint32_t)f2bf(xv[b][7]) << 16);
+          *reinterpret_cast<uint4*>(a.out_rows + (rowbase + grow[b]) * D + c8) = u;
+        }
+        if (a.rowdot) {
+          float y[8];
+          load8<uint16_t>(a.dot_with + (rowbase + grow[b]) * D + c8, y);
+          float part = 0.0f;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) part = __builtin_fmaf(xv[b][j], y[j], part);
+#pragma unroll
+          for (int off = LPR / 2; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
+          if (cl == 0) a.rowdot[rowbase + grow[b]] = part;
+        }
+        if (first_bh && cl == 0 && a.valid_re) a.valid_re[grow[b]] = ok[b] ? 1 : 0;
       }
-      if (a.rowdot) {
-        float y[8];
-        load8<uint16_t>(a.dot_with + (rowbase + grow[b]) * D + c8, y);
-        float part = 0.0f;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) part = __builtin_fmaf(xv[b][j], y[j], part);
-#pragma unroll
-        for (int off = LPR / 2; off >= 1; off >>= 1) part += __shfl_xor(part, off, 64);
-        if (cl == 0) a.rowdot[rowbase + grow[b]] = part;
-      }
-      if (first_bh && cl == 0 && a.valid_re) a.valid_re[grow[b]] = ok[b] ? 1 : 0;
     }
     if (POOL) {
       // this lane's row of each instruction, in row order within its group;
       // valid rows counted from one ballot per instruction (a lane per row)
       constexpr uint64_t kRowLead = LPR == 16 ? 0x0001000100010001ull : 0x0101010101010101ull;
+      auto add = [&] {
 #pragma unroll
-      for (int b = 0; b < NB; ++b) {
+        for (int b = 0; b < NB; ++b) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[j] = ok[b] ? acc[j] + xv[b][j] : acc[j];
-        const int nv = __popcll(__ballot(ok[b]) & kRowLead);
-        cnt += nv;
-        tcnt += nv;
-      }
-      const int rlast = wid * 128 + o0 + RB - 1;
-      if ((rlast + 1) % m.bsz == 0) {  // block complete
-        const int64_t blk = m.block(rlast);
-        if (blk < a.N_b) {
-          if (a.block_mean) {
-            float sum[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) sum[j] = acc[j];
-#pragma unroll
-            for (int g = 1; g < RPI; ++g)
-#pragma unroll
-              for (int j = 0; j < 8; ++j) sum[j] = sum[j] + __shfl(acc[j], g * LPR + cl, 64);
-            if (sub == 0) {
-              const float den = (float)(cnt > 0 ? cnt : 1);
-              float* dst = a.block_mean + ((int64_t)bh * a.N_b + blk) * D + c8;
-#pragma unroll
-              for (int j = 0; j < 8; ++j) dst[j] = sum[j] / den;
-            }
-          }
-          if (first_bh && lane == 0 && a.block_count) a.block_count[blk] = cnt;
+          for (int j = 0; j < 8; ++j) acc[j] = ok[b] ? acc[j] + xv[b][j] : acc[j];
+          const int nv = __popcll(__ballot(ok[b]) & kRowLead);
+          cnt += nv;
+          tcnt += nv;
         }
-        cnt = 0;
+      };
+      if constexpr (HALF) {
+        const bool whole = m.bsz == 64, second = !whole && (r0 & 64);
+        if (live && !second) add();
+        if (live && !whole && !second) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
-      }
-      if ((rlast + 1) % 64 == 0) {  // tile complete
-        if (first_bh && lane == 0 && a.tile_count) a.tile_count[m.row(rlast) >> 6] = tcnt;
-        tcnt = 0;
+          for (int j = 0; j < 8; ++j) sAcc[wid][j][lane] = acc[j];
+          if (lane == 0) sCnt[wid] = cnt;
+        }
+        __syncthreads();
+        if (!live) return;
+        if (second) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) acc[j] = sAcc[wid - 1][j][lane];
+          cnt = sCnt[wid - 1];
+          add();
+        }
+        if (whole || second) finish_block(r0 + 63);
+        if (first_bh && lane == 0 && a.tile_count) a.tile_count[m.row(r0) >> 6] = tcnt;
+      } else {
+        add();
+        const int rlast = r0 + o0 + RB - 1;
+        if ((rlast + 1) % m.bsz == 0) {  // block complete
+          finish_block(rlast);
+          cnt = 0;
+#pragma unroll
+          for (int j = 0; j < 8; ++j) acc[j] = 0.0f;
+        }
+        if ((rlast + 1) % 64 == 0) {  // tile complete
+          if (first_bh && lane == 0 && a.tile_count) a.tile_count[m.row(rlast) >> 6] = tcnt;
+          tcnt = 0;
+        }
       }
     }
   }
 }
 
-// grid (units, B*H): tile-order bf16 rows (S_out per head) -> THW rows of
-// dtype TO (S_in per head); padding rows are dropped.  Each lane moves 16
-// bytes (8 channels): a wave instruction covers 64 / (D / 8) rows, and NB
-// instructions are in flight per wave.
-template <int D, typename TO, typename Map>
+// grid (units x 128 / RPW, B*H): tile-order bf16 rows (S_out per head) -> THW
+// rows of dtype TO (S_in per head); padding rows are dropped.  Each lane moves
+// 16 bytes (8 channels): a wave instruction covers 64 / (D / 8) rows, NB
+// instructions are in flight per wave, and a wave takes RPW rows.
+template <int D, typename TO, typename Map, int NB, int RPW>
 __global__ __launch_bounds__(kGatherThreads) void scatter_rows_kernel(const uint16_t* __restrict__ in, int64_t S_in,
                                                                       int64_t S_out, Map m, TO* __restrict__ out) {
   constexpr int LPR = D / 8;     // lanes per row
   constexpr int RPI = 64 / LPR;  // rows per wave instruction
-  constexpr int NB = 4;          // wave instructions in flight
   constexpr int RB = RPI * NB;   // rows per batch
-  static_assert(128 % RB == 0, "a wave's 128 rows split into whole batches");
+  static_assert(64 % RB == 0 && RPW % RB == 0, "batches must not straddle blocks");
   const int bh = blockIdx.y;
-  const int wid = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int sub = lane / LPR, c8 = (lane % LPR) * 8;
-  m.init(blockIdx.x);
-  if (!m.live(wid * 128)) return;
+  constexpr int SUBS = 128 / RPW;  // workgroups per unit
+  m.init(blockIdx.x / SUBS);
+  const int r0 = (int)(blockIdx.x % SUBS) * 4 * RPW + wid * RPW;
+  if (!m.live(r0)) return;
   const uint16_t* inh = in + (int64_t)bh * S_out * D + c8;
   TO* outh = out + (int64_t)bh * S_in * D + c8;
-  for (int o0 = 0; o0 < 128; o0 += RB) {
+  for (int o0 = 0; o0 < RPW; o0 += RB) {
     uint4 v[NB];
     int64_t tok[NB];
+    if (RPW < 128 || (o0 & 63) == 0) m.group((r0 + o0) & ~63);
 #pragma unroll
     for (int b = 0; b < NB; ++b) {
-      const int r = wid * 128 + o0 + b * RPI + sub;
-      tok[b] = m.token(r);
+      const int r = r0 + o0 + b * RPI + sub;
+      tok[b] = m.g.token(r & 63);
       if (tok[b] >= 0) v[b] = *reinterpret_cast<const uint4*>(inh + m.row(r) * D);
     }
 #pragma unroll
@@ -339,34 +400,58 @@ __global__ __launch_bounds__(kGatherThreads) void scatter_rows_kernel(const uint
   }
 }
 
-template <typename Map, bool POOL>
-void launch_gather_t(const GatherArgs& a, const Map& m, int dtype, int D, dim3 grid, hipStream_t stream) {
-  if (dtype == PRISM_BF16) {
-    if (D == 128) gather_pool_kernel<128, uint16_t, Map, POOL><<<grid, kGatherThreads, 0, stream>>>(a, m);
-    else gather_pool_kernel<64, uint16_t, Map, POOL><<<grid, kGatherThreads, 0, stream>>>(a, m);
+// Rows per wave and wave instructions in flight.  Launches that fill the GPU
+// hide the latency with other waves: 128 rows, 2 instructions with pooling (2:
+// 0.256 ms, 4: 0.283, 8: 0.326 averaged over a step's launches at 302,400 tokens
+// x 5 heads), else 4.  Launches of few units leave about a wave per SIMD: there
+// a wave takes 64 rows (32 without pooling) and keeps them all in flight.  The
+// lines lie where both sides cost the same (bf16, D = 128, us at 280 / 540 /
+// 1,215 units x heads, few and many rows per wave): pooling 28 / 45 / 105 and
+// 32 / 51 / 61, gather 14 / 24 / 59 and 26 / 45 / 55, scatter 14 / 43 / 91 and
+// 22 / 38 / 59.
+constexpr int64_t kFewPools = 768, kFewGathers = 1024, kFewScatters = 400;
+
+template <int D, typename T, typename Map>
+void launch_gather_t(const GatherArgs& a, const Map& m, dim3 grid, hipStream_t stream) {
+  const bool pool = a.block_mean != nullptr || a.block_count != nullptr || a.tile_count != nullptr;
+  if ((int64_t)grid.x * grid.y < (pool ? kFewPools : kFewGathers)) {
+    if (pool) gather_pool_kernel<D, T, Map, true, D / 8, 64><<<dim3(2 * grid.x, grid.y), kGatherThreads, 0, stream>>>(a, m);
+    else gather_pool_kernel<D, T, Map, false, D / 16, 32><<<dim3(4 * grid.x, grid.y), kGatherThreads, 0, stream>>>(a, m);
   } else {
-    if (D == 128) gather_pool_kernel<128, float, Map, POOL><<<grid, kGatherThreads, 0, stream>>>(a, m);
-    else gather_pool_kernel<64, float, Map, POOL><<<grid, kGatherThreads, 0, stream>>>(a, m);
+    if (pool) gather_pool_kernel<D, T, Map, true, 2, 128><<<grid, kGatherThreads, 0, stream>>>(a, m);
+    else gather_pool_kernel<D, T, Map, false, 4, 128><<<grid, kGatherThreads, 0, stream>>>(a, m);
   }
 }
 template <typename Map>
 void launch_gather(const GatherArgs& a, const Map& m, int dtype, int D, dim3 grid, hipStream_t stream) {
-  if (a.block_mean != nullptr || a.block_count != nullptr || a.tile_count != nullptr)
-    launch_gather_t<Map, true>(a, m, dtype, D, grid, stream);
-  else
-    launch_gather_t<Map, false>(a, m, dtype, D, grid, stream);
+  if (dtype == PRISM_BF16) {
+    if (D == 128) launch_gather_t<128, uint16_t>(a, m, grid, stream);
+    else launch_gather_t<64, uint16_t>(a, m, grid, stream);
+  } else {
+    if (D == 128) launch_gather_t<128, float>(a, m, grid, stream);
+    else launch_gather_t<64, float>(a, m, grid, stream);
+  }
 }
 
+template <int D, typename TO, typename Map>
+void launch_scatter_t(const uint16_t* in, int64_t S_in, int64_t S_out, const Map& m, TO* out, dim3 grid,
+                      hipStream_t stream) {
+  if ((int64_t)grid.x * grid.y < kFewScatters)
+    scatter_rows_kernel<D, TO, Map, D / 16, 32><<<dim3(4 * grid.x, grid.y), kGatherThreads, 0, stream>>>(in, S_in,
+                                                                                                       S_out, m, out);
+  else
+    scatter_rows_kernel<D, TO, Map, 4, 128><<<grid, kGatherThreads, 0, stream>>>(in, S_in, S_out, m, out);
+}
 template <typename Map>
 void launch_scatter(const void* in_rows, int64_t S_in, int64_t S_out, const Map& m, void* out, int out_dtype, int D,
                     dim3 grid, hipStream_t stream) {
   const uint16_t* in = (const uint16_t*)in_rows;
   if (out_dtype == PRISM_BF16) {
-    if (D == 128) scatter_rows_kernel<128, uint16_t, Map><<<grid, kGatherThreads, 0, stream>>>(in, S_in, S_out, m, (uint16_t*)out);
-    else scatter_rows_kernel<64, uint16_t, Map><<<grid, kGatherThreads, 0, stream>>>(in, S_in, S_out, m, (uint16_t*)out);
+    if (D == 128) launch_scatter_t<128>(in, S_in, S_out, m, (uint16_t*)out, grid, stream);
+    else launch_scatter_t<64>(in, S_in, S_out, m, (uint16_t*)out, grid, stream);
   } else {
-    if (D == 128) scatter_rows_kernel<128, float, Map><<<grid, kGatherThreads, 0, stream>>>(in, S_in, S_out, m, (float*)out);
-    else scatter_rows_kernel<64, float, Map><<<grid, kGatherThreads, 0, stream>>>(in, S_in, S_out, m, (float*)out);
+    if (D == 128) launch_scatter_t<128>(in, S_in, S_out, m, (float*)out, grid, stream);
+    else launch_scatter_t<64>(in, S_in, S_out, m, (float*)out, grid, stream);
   }
 }
 
@@ -388,8 +473,10 @@ int chunk_map(int T, int Hg, int Wg, int Tp, int Hp, int Wp, int ct, int ch, int
   const int64_t Sp = (int64_t)Tp * Hp * Wp;
   PRISM_REQUIRE(S_out >= Sp && S_out % 128 == 0, "%s: rows per head must be a multiple of 128 and >= T*H*W padded",
                 who);
+  PRISM_REQUIRE(Sp / bsz < (1ll << 31), "%s: too many chunks", who);
   *m = ChunkMap{};
-  m->T = T; m->Hg = Hg; m->Wg = Wg; m->ct = ct; m->ch = ch; m->cw = cw; m->Nh = Hp / ch; m->Nw = Wp / cw;
+  m->g.T = T; m->g.H = Hg; m->g.W = Wg; m->g.lb = __builtin_ctz(bsz); m->g.lh = __builtin_ctz(ch);
+  m->g.lw = __builtin_ctz(cw); m->ct = ct; m->ch = ch; m->cw = cw; m->Nh = Hp / ch; m->Nw = Wp / cw;
   m->Sp = Sp; m->S_out = S_out; m->bsz = bsz;
   return PRISM_OK;
 }
