@@ -29,6 +29,7 @@ __device__ __forceinline__ f32x16 f32x16_zero() {
 }
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 // round-to-nearest-even bf16 pair (one v_cvt_pk_bf16_f32)
 __device__ __forceinline__ uint32_t pack_bf16(float a, float b) {
   const f32x2 v = {a, b};

@@ -18,25 +18,37 @@
 //                          bf16(y)^2 (the squares of the stored values)
 //   rownorm_finish_kernel  norms[m] = sqrt(sum_t partial[m][t]), t ascending
 //
-// MI355X design: one 256 x 256 output tile per workgroup of four waves (one
-// per SIMD), each wave 128 x 128 = 4 x 4 blocks of v_mfma_f32_32x32x16_bf16
-// (256 accumulator registers; the tile computes C^T = W x^T, so each lane owns
-// one output row and four consecutive columns per register quad).  K steps of
-// 64, double-buffered: the x and W tiles of step k + 1 (2 x 32 KB) are copied
-// HBM -> LDS by global_load_lds_dwordx4 while step k is multiplied, the copy
-// instructions spread between the step's MFMA groups.  LDS rows are 128
-// bytes, unpadded, with the 16-byte chunks of row r XOR-swizzled by
-// (r >> 1) & 7, so the row-operand reads (16 consecutive rows, one chunk
-// each, per 16 lanes) hit distinct bank groups.  Workgroup
-// ids are ordered so that each XCD (own L2) works on about 8 x 4 neighbouring
-// output tiles at a time, which share their k-slices of x and W in its L2.
-// Deterministic (no atomics).
+// MI355X design: persistent workgroups of four waves (one per SIMD), one 256 x
+// 256 output tile at a time, each wave 128 x 128 = 8 x 8 blocks of
+// v_mfma_f32_16x16x32_bf16 (256 accumulator AGPRs; the tile computes C^T = W
+// x^T, so each lane owns one output row and four consecutive columns per
+// block).  Stages of 64 columns of K: a ring of five 32 KB slots (all of the
+// 160 KB) takes x and W tiles in turn by global_load_lds_dwordx4, three tiles
+// ahead of the stage being read.  A stage is two steps of 64 MFMAs; each step
+// reads the next one's fragments (two ds_read_b128 per eight MFMAs) and issues
+// one copy per eight MFMAs; the one barrier of a stage stands between its
+// steps, when all of the stage's fragments are in registers, so the MFMAs go on
+// right behind it.  The stages run on over the end of an output tile: its
+// epilogue works while the next tile's first 96 KB land, turning the
+// accumulators through the one free slot so that y is stored in rows of 256
+// bytes.  LDS rows are 128 bytes, unpadded, with the 16-byte chunks of row r
+// XOR-swizzled by (r >> 1) & 7, so the row-operand reads (16 consecutive rows,
+// one chunk each, per 16 lanes) hit distinct bank groups.  Tiles are ordered so
+// that each XCD (own L2) works on about 8 x 4 neighbouring output tiles at a
+// time, which share their k-slices of x and W in its L2.  Deterministic (no
+// atomics).
 //
-// Measured at the config-4 shape (M = 302,400, N = K = 5,120): 15.3-16.7 ms,
-// 1.0 PFLOP/s.  The kernel is bound by streaming its tiles from L2 into LDS:
-// a copies-only variant (no MFMAs) takes 11.4 ms (124 GB of tile copies at
-// 10.9 TB/s), an MFMA-only variant (no copies) 13 ms; torch's F.linear
-// (hipBLASLt) plus prism_a2v_norms takes 11.0 ms for the same outputs.
+// Measured at M = 75,600, N = K = 5,120 (3.96 TFLOP): 3.93 -> 2.89 ms, 1,009 ->
+// 1,369 TFLOP/s, against 2.80 ms of torch's F.linear (hipBLASLt) without the
+// norms.  What the time was: an epilogue of 24 us per tile (16-byte pieces of y
+// and a branch per rounded element; K = 64, 5,120 tiles: 475 -> 199 us, now the
+// write of y), the copies' latency at each stage's end, and 32 x 32 x 16 MFMAs
+// with bursts of fragment reads (as few cycles, but a lower clock: 2.68 against
+// 2.39 ms at M = 65,536).
+// Stages of 32 columns with four in flight were slower (3.81 ms): rows of 64
+// bytes double the L2 requests.  Now bound by the matrix cores at the clock
+// that their power leaves (about 1.7 GHz; with x = 0, M = 65,536 takes 2.03
+// instead of 2.39 ms) and by the last round of tiles (24 for 23.1).
 #include "common.h"
 #include "mfma.h"
 #include "tile_dma.h"
@@ -44,13 +56,11 @@
 namespace {
 
 constexpr int kBM = 256, kBN = 256, kBK = 64;
-constexpr int kStages = 2;                         // the copies of step k + 1 run while step k is multiplied
+constexpr int kSlots = 5;                          // ring of x and W tiles in turn (160 KB)
 constexpr int kRowBytes = kBK * 2;                 // 128
 constexpr int kTileBytes = kBM * kRowBytes;        // 32 KB (x or W tile of one stage)
-constexpr int kStageBytes = 2 * kTileBytes;        // 64 KB
 constexpr int kOprojThreads = 256;                 // 4 waves
-constexpr int kTileKB = kTileBytes / 1024;         // 32
-constexpr int kCopiesPerWave = kStageBytes / 1024 / 4;  // 16 KB-instructions per wave and stage
+constexpr int kCopies = kTileBytes / 1024 / 4;     // 8 KB-instructions per wave and tile
 constexpr int kGroupM = 4;                         // output-tile rows per group of the launch order
 
 struct OprojArgs {
@@ -60,6 +70,7 @@ struct OprojArgs {
   int64_t M;
   int N, K;
   int mtiles, ntiles;    // ceil(M / 256), N / 256
+  int total;             // output tiles
   uint16_t* y;           // [M, N]
   float* partial;        // [M, ntiles]
 };
@@ -70,11 +81,18 @@ struct OprojArgs {
 // 256-byte bank line: (r & 1, (r >> 1) & 7) differ for 16 consecutive rows)
 __device__ __forceinline__ uint32_t swz(int r, int c) { return (uint32_t)(r * kRowBytes + 16 * (c ^ ((r >> 1) & 7))); }
 
-__global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojArgs a) {
-  __shared__ __align__(16) uint8_t smem[kStages * kStageBytes];
-  __shared__ float sNorm[2][kBM];  // the two n-halves' row partials
+// an accumulator element, moved out of its AGPR here (left to the compiler, all
+// 256 are moved at once and the copies' offsets spill)
+__device__ __forceinline__ float acc_read(float a) {
+  float v;
+  asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(v) : "a"(a));
+  return v;
+}
 
-  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, l32 = lane & 31;
+__global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojArgs a) {
+  __shared__ __align__(1024) uint8_t smem[kSlots * kTileBytes];
+
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, l16 = lane & 15;
   const int w = (int)uniform_u32((uint32_t)tid >> 6);
   const int mh = w & 1, nh = w >> 1;
 
@@ -84,153 +102,221 @@ __global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojA
   // once cover about 4 x 8 tiles and share each k-slice of x (8 ways) and W
   // (4 ways) in that XCD's L2 (4-row groups measured 4% faster than 8-row
   // groups; plain row order was within 1%).
-  const int nwg = (int)gridDim.x;
-  const int b = (int)blockIdx.x;
-  const int per = nwg / 8;
-  const int lid = b < per * 8 ? (b & 7) * per + (b >> 3) : b;
-  const int gsize = kGroupM * a.ntiles;
-  const int grp = lid / gsize, first_m = grp * kGroupM;
-  const int gm = a.mtiles - first_m < kGroupM ? a.mtiles - first_m : kGroupM;
-  const int inner = lid - grp * gsize;
-  const int mt = first_m + inner % gm, nt = inner / gm;
-  const int64_t m0 = (int64_t)mt * kBM;
-  const int n0 = nt * kBN;
-
-  // DMA plan: KB-instruction i of a stage covers tile bytes [1024 i', 1024 i' + 1024)
-  // of the x tile (i < 32, i' = i) or the W tile (i' = i - 32); lane L of it
-  // writes 16 bytes at 16 L: row (1024 i' + 16 L) / 128, stored chunk L % 8,
-  // logical chunk (L % 8) ^ ((row >> 1) & 7).  Wave w issues i = w + 4 s.
-  uint32_t voff0[kCopiesPerWave];  // byte offset of this lane's 16 bytes at k = 0, from the tensor's base
-#pragma unroll
-  for (int s = 0; s < kCopiesPerWave; ++s) {
-    const int i = w + 4 * s;
-    const int tb = (i % kTileKB) * 1024 + 16 * lane;
-    const int row = tb / kRowBytes, sc = (tb % kRowBytes) / 16;
-    const int c = sc ^ ((row >> 1) & 7);
-    int64_t grow;
-    if (i < kTileKB) {
-      grow = m0 + row;
-      if (grow >= a.M) grow = a.M - 1;  // rows past M re-read the last row (never stored)
-    } else {
-      grow = n0 + row;
-    }
-    voff0[s] = (uint32_t)((grow * a.K + 8 * c) * 2);
-  }
-  const uint32_t lds0 = lds_addr(smem);
-  const void* xb = uniform_ptr(a.x);
-  const void* wb = uniform_ptr(a.w);
-  // copies [q0, q1) of this wave for k-step kstep into stage st
-  auto issue = [&](int kstep, int st, int q0, int q1) {
-    const uint32_t base = lds0 + (uint32_t)(st * kStageBytes);
-    const uint32_t kb = (uint32_t)kstep * (uint32_t)kRowBytes;
-#pragma unroll
-    for (int s = 0; s < kCopiesPerWave; ++s) {
-      if (s < q0 || s >= q1) continue;
-      const int i = w + 4 * s;
-      dma_b128(voff0[s] + kb, i < kTileKB ? xb : wb, base + (uint32_t)i * 1024u);
-    }
+  const int nwg = (int)gridDim.x, per = a.total / 8;
+  auto tile_of = [&](int b, int& mt, int& nt) {
+    const int lid = b < per * 8 ? (b & 7) * per + (b >> 3) : b;
+    const int gsize = kGroupM * a.ntiles;
+    const int grp = lid / gsize, first_m = grp * kGroupM;
+    const int gm = a.mtiles - first_m < kGroupM ? a.mtiles - first_m : kGroupM;
+    const int inner = lid - grp * gsize;
+    mt = first_m + inner % gm;
+    nt = inner / gm;
   };
 
-  f32x16 acc[4][4];
+  // DMA plan: KB-instruction i of a tile covers its bytes [1024 i, 1024 i + 1024);
+  // lane L writes 16 bytes at 16 L: row 8 i + L / 8, stored chunk L % 8, logical
+  // chunk (L % 8) ^ ((row >> 1) & 7).  Wave w issues i = w + 4 c.
+  uint32_t xoff[kCopies], woff[kCopies];  // byte offsets of this lane's 16 bytes at k = 0
+  const uint32_t last = (uint32_t)a.M - 1, ld = (uint32_t)a.K * 2;  // M < 2^25 (x below 4 GiB)
+  auto x_tile = [&](int v) {
+    int mt, nt;
+    tile_of(v, mt, nt);
+    const int t = opaque_thread_id(), row = 8 * w + (t & 63) / 8;  // (not kept across the tile)
+    const uint32_t chunk = 16u * ((t % 8) ^ ((row >> 1) & 7));  // the same for rows 32 apart
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
+    for (int c = 0; c < kCopies; ++c) {
+      const uint32_t m = (uint32_t)(mt * kBM + row + 32 * c);
+      xoff[c] = (m < last ? m : last) * ld + chunk;  // rows past M re-read the last row (never stored)
+    }
+  };
+  auto w_tile = [&](int v) {
+    int mt, nt;
+    tile_of(v, mt, nt);
+    const int t = opaque_thread_id(), row = 8 * w + (t & 63) / 8;
+    const uint32_t chunk = 16u * ((t % 8) ^ ((row >> 1) & 7));
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x16_zero();
-
+    for (int c = 0; c < kCopies; ++c) woff[c] = (uint32_t)(nt * kBN + row + 32 * c) * ld + chunk;
+  };
   const int nsteps = a.K / kBK;
-  // operand fragments of k-step s: A = W rows 128 nh + 32 i + l32, B = x rows
-  // 128 mh + 32 i + l32, logical chunk 2 s + g; chunk 2 s + g of row r sits at
-  // the offset of chunk g XOR 32 s (the swizzle XORs the chunk index, and 2 s
-  // only touches its upper bit)
-  uint32_t offA[4], offB[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    offA[i] = (uint32_t)kTileBytes + swz(nh * 128 + 32 * i + l32, g);
-    offB[i] = swz(mh * 128 + 32 * i + l32, g);
-  }
-  auto load_ops = [&](const uint8_t* st, int s, bf16x8* av, bf16x8* bv) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      av[i] = *reinterpret_cast<const bf16x8*>(st + (offA[i] ^ (uint32_t)(32 * s)));
-      bv[i] = *reinterpret_cast<const bf16x8*>(st + (offB[i] ^ (uint32_t)(32 * s)));
+  const uint32_t lds0 = lds_addr(smem) + 1024u * (uint32_t)w;
+  const uint8_t* const xb = (const uint8_t*)uniform_ptr(a.x);
+  const uint8_t* const wb = (const uint8_t*)uniform_ptr(a.w);
+  // the tiles to copy next: output tile, k offset, slot.  The copies run on
+  // into the workgroup's next output tile (after its last one, into that one
+  // again: slots that nothing reads any more, so every stage issues and waits
+  // alike)
+  const uint32_t kend = (uint32_t)nsteps * kRowBytes;
+  uint32_t kx = 0, kw = 0, put = 0;
+  int vx = (int)blockIdx.x, vw = vx;
+  auto next_slot = [&](uint32_t s) { return s + kTileBytes == kSlots * kTileBytes ? 0u : s + kTileBytes; };
+  auto copy_x = [&](int c) { dma_b128(xoff[c], xb + kx, lds0 + put + 4096u * (uint32_t)c); };
+  auto copy_w = [&](int c) { dma_b128(woff[c], wb + kw, lds0 + put + 4096u * (uint32_t)c); };
+  auto copied_x = [&] {
+    kx += kRowBytes;
+    put = next_slot(put);
+    if (kx == kend) {
+      kx = 0;
+      if (vx + nwg < a.total) x_tile(vx += nwg);
     }
   };
-  constexpr int KS = kBK / 16;                  // k-steps per stage
-  constexpr int QC = kCopiesPerWave / KS;       // copies issued after each k-step's MFMAs
-  issue(0, 0, 0, kCopiesPerWave);
-  for (int ks = 0; ks < nsteps; ++ks) {
-    dma_wait_all();
-    __syncthreads();
-    const bool more = ks + 1 < nsteps;
-    const uint8_t* sp = smem + (ks & 1) * kStageBytes;
-    // software pipeline over the stage's k-steps: the fragments of step s + 1
-    // are read while the sixteen MFMAs of step s run, and a quarter of the
-    // next stage's copies is issued after each step's MFMAs (a wave stalls
-    // while its copy instructions queue; spread out, they hide behind MFMAs)
-    bf16x8 av[2][4], bv[2][4];
-    load_ops(sp, 0, av[0], bv[0]);
-#pragma unroll
-    for (int s = 0; s < KS; ++s) {
-      if (s + 1 < KS) load_ops(sp, s + 1, av[(s + 1) & 1], bv[(s + 1) & 1]);
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(av[s & 1][i], bv[s & 1][j], acc[i][j], 0, 0, 0);
-      if (s == 0) __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);  // step 0 reads first
-      if (s + 1 < KS) __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      if (more) issue(ks + 1, (ks + 1) & 1, s * QC, s * QC + QC);
-      __builtin_amdgcn_sched_barrier(0);
+  auto copied_w = [&] {
+    kw += kRowBytes;
+    put = next_slot(put);
+    if (kw == kend) {
+      kw = 0;
+      if (vw + nwg < a.total) w_tile(vw += nwg);
     }
-  }
+  };
+  x_tile(vx);
+  w_tile(vw);
 
-  // epilogue: acc[i][j] register r holds C^T[n][m] with
-  // n = n0 + 128 nh + 32 i + 8 (r >> 2) + 4 g + (r & 3), m = m0 + 128 mh + 32 j + l32
-  float ss[4];  // squares of the stored values of this lane's row, per m block
+  f32x4 acc[8][8];
+
+  // operand fragments of k-step s (32 wide): A = W rows 128 nh + 16 i + l16, B =
+  // x rows 128 mh + 16 j + l16, logical chunk 4 s + g: the offset of chunk g
+  // XOR 64 s (4 s only touches the top bit of the chunk), rows 16 i an immediate
+  const uint32_t offA = swz(nh * 128 + l16, g), offB = swz(mh * 128 + l16, g);
+  bf16x8 av[2][8], bv[2][8];
+  uint32_t get = 0;  // slot of the stage's x tile; its W tile is in the next one
+  uint32_t pA = 0, pB = 0;
+  auto stage_at = [&] {
+    pB = get + offB;
+    get = next_slot(get);
+    pA = get + offA;
+    get = next_slot(get);
+  };
+  auto load = [&](int s, int i) {
+    bv[s][i] = *reinterpret_cast<const bf16x8*>(smem + (pB ^ (64u * s)) + 16 * kRowBytes * i);
+    av[s][i] = *reinterpret_cast<const bf16x8*>(smem + (pA ^ (64u * s)) + 16 * kRowBytes * i);
+  };
+  auto mul = [&](int s, int i) {
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) ss[j] = 0.0f;
+    for (int j = 0; j < 8; ++j)
+      asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(av[s][i]), "v"(bv[s][j]));
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // both tiles of the next stage have landed (the x tile after them may still
+  // be in flight) and every wave has its fragments of this one
+  auto landed = [&] {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kCopies));
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int c = 0; c < kCopies; ++c) copy_x(c);
+  copied_x();
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int n = n0 + 128 * nh + 32 * i + 8 * q + 4 * g;
-      float bb[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (a.bias) {
-        const uint2 u = *reinterpret_cast<const uint2*>(a.bias + n);
-        bb[0] = __uint_as_float(u.x << 16); bb[1] = __uint_as_float(u.x & 0xffff0000u);
-        bb[2] = __uint_as_float(u.y << 16); bb[3] = __uint_as_float(u.y & 0xffff0000u);
+  for (int c = 0; c < kCopies; ++c) copy_w(c);
+  copied_w();
+#pragma unroll
+  for (int c = 0; c < kCopies; ++c) copy_x(c);
+  copied_x();
+  landed();
+  stage_at();
+#pragma unroll
+  for (int i = 0; i < 8; ++i) load(0, i);
+#pragma unroll
+  for (int c = 0; c < kCopies; ++c) copy_w(c);
+  copied_w();
+  for (int v = (int)blockIdx.x; v < a.total; v += nwg) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    asm volatile("s_nop 7");  // before inline assembly reads them
+    for (int ks = 0; ks < nsteps; ++ks) {
+      // 64 MFMAs of step 0 while step 1's fragments are read and an x tile is copied
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        load(1, i);
+        mul(0, i);
+        copy_x(i);
       }
+      copied_x();
+      landed();
+      stage_at();
+      // step 1, with the next stage's first fragments and a W tile
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int64_t m = m0 + 128 * mh + 32 * j + l32;
-        float v[4];
+      for (int i = 0; i < 8; ++i) {
+        load(0, i);
+        mul(1, i);
+        copy_w(i);
+      }
+      copied_w();
+    }
+
+    // epilogue, while the next output tile's first copies land: acc[i][j]
+    // element e holds C^T[n][m] with n = n0 + 16 i + 4 g + e, m = m0 + 16 j +
+    // l16.  The wave turns 32 rows of 128 columns at a time through 8 KB of the
+    // slot that the next x tile is copied to after the last barrier, chunk c of
+    // row r at c ^ (r & 15), and stores rows of 256 bytes.
+    int mt, nt;
+    tile_of(v, mt, nt);
+    const int m0 = mt * kBM + 128 * mh, n0 = nt * kBN + 128 * nh, M = (int)a.M;
+    const int lane = opaque_thread_id() & 63, g = lane >> 4, l16 = lane & 15;
+    uint8_t* const stage = smem + put + 8192u * (uint32_t)w;
+    asm volatile("s_nop 15\n\ts_nop 15");  // the last MFMAs' results, read by inline assembly below
+    uint2 bias[8];  // of columns 16 i + 4 g .. + 3
 #pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = round_bf(acc[i][j][4 * q + e] + bb[e]);
+    for (int i = 0; i < 8; ++i)
+      bias[i] = a.bias ? *reinterpret_cast<const uint2*>(a.bias + n0 + 16 * i + 4 * g) : uint2{0u, 0u};
+    float ss[8];  // squares of the stored values of this lane's row, per m block
 #pragma unroll
-        for (int e = 0; e < 4; ++e) ss[j] = __builtin_fmaf(v[e], v[e], ss[j]);
-        if (m < a.M) {
-          uint2 o;
-          o.x = pack_bf16(v[0], v[1]);
-          o.y = pack_bf16(v[2], v[3]);
-          *reinterpret_cast<uint2*>(a.y + m * a.N + n) = o;
+    for (int j = 0; j < 8; ++j) {
+      ss[j] = 0.0f;
+      const int row = 16 * (j & 1) + l16;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        uint2 u = bias[i];
+        asm volatile("" : "+v"(u.x), "+v"(u.y));  // (unpacked here, not kept as floats for all j)
+        const float bb[4] = {__uint_as_float(u.x << 16), __uint_as_float(u.x & 0xffff0000u),
+                             __uint_as_float(u.y << 16), __uint_as_float(u.y & 0xffff0000u)};
+        uint2 o;  // (v_cvt_pk_bf16_f32: round to nearest even, as the scalar helper without its branch)
+        o.x = pack_bf16(acc_read(acc[i][j][0]) + bb[0], acc_read(acc[i][j][1]) + bb[1]);
+        o.y = pack_bf16(acc_read(acc[i][j][2]) + bb[2], acc_read(acc[i][j][3]) + bb[3]);
+        const float t[4] = {__uint_as_float(o.x << 16), __uint_as_float(o.x & 0xffff0000u),
+                            __uint_as_float(o.y << 16), __uint_as_float(o.y & 0xffff0000u)};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) ss[j] = __builtin_fmaf(t[e], t[e], ss[j]);
+        *reinterpret_cast<uint2*>(stage + 256 * row + 16 * ((2 * i + (g >> 1)) ^ l16) + 8 * (g & 1)) = o;
+        if (i & 1) __builtin_amdgcn_sched_barrier(0);
+      }
+      if (j & 1) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) {
+          const int row = 4 * r + (lane >> 4);
+          const uint4 o = *reinterpret_cast<const uint4*>(stage + 256 * row + 16 * ((lane & 15) ^ (row & 15)));
+          const int m = m0 + 16 * (j - 1) + row;
+          if (m < M) *reinterpret_cast<uint4*>(a.y + (int64_t)m * a.N + n0 + 8 * (lane & 15)) = o;
         }
       }
     }
-  }
-  // row partial of this wave (its 128 columns): the two lane halves hold
-  // different columns of the same row
+    // row partial of this wave (its 128 columns): the four lane groups hold
+    // different columns of the same row; then the two waves of a row
+    float* const part = reinterpret_cast<float*>(stage);
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const float t = xor32_add(ss[j]);
-    if (g == 0) sNorm[nh][128 * mh + 32 * j + l32] = t;
+    for (int j = 0; j < 8; ++j) {
+      const float t = xor32_add(ss[j] + __shfl_xor(ss[j], 16));
+      if (g == 0) part[16 * j + l16] = t;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+    if (nh == 0) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int m = m0 + 64 * h + lane;
+        if (m < M) a.partial[(int64_t)m * a.ntiles + nt] = part[64 * h + lane] + part[2 * 2048 + 64 * h + lane];
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();  // the x tile copied there next stays off what other waves read
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
   }
-  __syncthreads();
-  for (int r = tid; r < kBM; r += kOprojThreads) {
-    const int64_t m = m0 + r;
-    if (m < a.M) a.partial[m * a.ntiles + nt] = sNorm[0][r] + sNorm[1][r];
-  }
+  dma_wait_all();
 }
 
 template <typename TO>
@@ -264,8 +350,9 @@ int prism_linear_rownorm(const void* x, const void* w, const void* bias, int64_t
   PRISM_REQUIRE(mtiles * ntiles < (1ll << 31), "prism_linear_rownorm: grid too large");
   OprojArgs a;
   a.x = (const uint16_t*)x; a.w = (const uint16_t*)w; a.bias = (const uint16_t*)bias;
-  a.M = M; a.N = N; a.K = K; a.mtiles = (int)mtiles; a.ntiles = ntiles; a.y = (uint16_t*)y; a.partial = partial;
-  linear_rownorm_kernel<<<(unsigned)(mtiles * ntiles), kOprojThreads, 0, stream>>>(a);
+  a.M = M; a.N = N; a.K = K; a.mtiles = (int)mtiles; a.ntiles = ntiles; a.total = (int)(mtiles * ntiles); a.y = (uint16_t*)y; a.partial = partial;
+  const int resident = resident_workgroups<linear_rownorm_kernel>(kOprojThreads);
+  linear_rownorm_kernel<<<(unsigned)(a.total < resident ? a.total : resident), kOprojThreads, 0, stream>>>(a);
   const unsigned fb = (unsigned)((M + 255) / 256);
   if (norms_dtype == PRISM_BF16) rownorm_finish_kernel<uint16_t><<<fb, 256, 0, stream>>>(partial, M, ntiles, (uint16_t*)norms);
   else rownorm_finish_kernel<float><<<fb, 256, 0, stream>>>(partial, M, ntiles, (float*)norms);

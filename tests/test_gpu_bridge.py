@@ -57,6 +57,17 @@ def test_linear_rownorm_small(M, N, K, bias):
     assert float(((ops.a2v_norms(y.float()).double() - n32.double()).abs() / n32.double()).max()) <= 1e-5
 
 
+@pytest.mark.parametrize("M,N,K,bias", [(33000, 768, 64, True), (16897, 1280, 128, False), (17151, 1280, 192, True),
+                                        (1, 256, 64, True), (255, 512, 128, True), (257, 256, 2560, False)], ids=str)
+def test_linear_rownorm_tile_streams(M, N, K, bias):
+    """Several output tiles per workgroup with one, two and three stages each
+    (the copies of a tile start up to two tiles before it), partial last tiles."""
+    from prism_amd import ops
+    x, w, b = _inputs(M, N, K, bias, seed=M)
+    y, n32 = ops.linear_rownorm(x, w, b, torch.float32)
+    _check_rows(x, w, b, y, n32, torch.arange(M, device=DEV))
+
+
 def test_bridge_projection_api_batch0():
     from prism_amd import a2v_bridge_projection, a2v_token_norms
     x, w, b = _inputs(2 * 300, 256, 128)
