@@ -19,7 +19,8 @@
 //   rownorm_finish_kernel  norms[m] = sqrt(sum_t partial[m][t]), t ascending
 //
 // MI355X design: persistent workgroups of four waves (one per SIMD), one 256 x
-// 256 output tile at a time, each wave 128 x 128 = 8 x 8 blocks of
+// 256 output tile at a time (fewer tiles than CUs, or a nearly empty last
+// round: 128 or 64 rows), each wave 128 x 128 = 8 x 8 blocks of
 // v_mfma_f32_16x16x32_bf16 (256 accumulator AGPRs; the tile computes C^T = W
 // x^T, so each lane owns one output row and four consecutive columns per
 // block).  Stages of 64 columns of K: a ring of five 32 KB slots (all of the
@@ -55,12 +56,12 @@
 
 namespace {
 
-constexpr int kBM = 256, kBN = 256, kBK = 64;
+constexpr int kBN = 256, kBK = 64;
 constexpr int kSlots = 5;                          // ring of x and W tiles in turn (160 KB)
 constexpr int kRowBytes = kBK * 2;                 // 128
-constexpr int kTileBytes = kBM * kRowBytes;        // 32 KB (x or W tile of one stage)
+constexpr int kTileBytes = kBN * kRowBytes;        // 32 KB: the W tile of a stage (the x tile: at most that)
 constexpr int kOprojThreads = 256;                 // 4 waves
-constexpr int kCopies = kTileBytes / 1024 / 4;     // 8 KB-instructions per wave and tile
+constexpr int kCopies = kTileBytes / 1024 / 4;     // 8 KB-instructions per wave and W tile
 constexpr int kGroupM = 4;                         // output-tile rows per group of the launch order
 
 struct OprojArgs {
@@ -69,7 +70,7 @@ struct OprojArgs {
   const uint16_t* bias;  // [N] or null
   int64_t M;
   int N, K;
-  int mtiles, ntiles;    // ceil(M / 256), N / 256
+  int mtiles, ntiles;    // ceil(M / (32 R)), N / 256
   int total;             // output tiles
   uint16_t* y;           // [M, N]
   float* partial;        // [M, ntiles]
@@ -89,7 +90,11 @@ __device__ __forceinline__ float acc_read(float a) {
   return v;
 }
 
+// R: blocks of 16 rows per wave (output tiles of 32 R rows)
+template <int R>
 __global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojArgs a) {
+  static_assert(R == 8 || R == 4 || R == 2, "R copies of x per wave and stage");
+  constexpr int kBM = 32 * R;
   __shared__ __align__(1024) uint8_t smem[kSlots * kTileBytes];
 
   const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, l16 = lane & 15;
@@ -116,7 +121,7 @@ __global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojA
   // DMA plan: KB-instruction i of a tile covers its bytes [1024 i, 1024 i + 1024);
   // lane L writes 16 bytes at 16 L: row 8 i + L / 8, stored chunk L % 8, logical
   // chunk (L % 8) ^ ((row >> 1) & 7).  Wave w issues i = w + 4 c.
-  uint32_t xoff[kCopies], woff[kCopies];  // byte offsets of this lane's 16 bytes at k = 0
+  uint32_t xoff[R], woff[kCopies];  // byte offsets of this lane's 16 bytes at k = 0
   const uint32_t last = (uint32_t)a.M - 1, ld = (uint32_t)a.K * 2;  // M < 2^25 (x below 4 GiB)
   auto x_tile = [&](int v) {
     int mt, nt;
@@ -124,7 +129,7 @@ __global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojA
     const int t = opaque_thread_id(), row = 8 * w + (t & 63) / 8;  // (not kept across the tile)
     const uint32_t chunk = 16u * ((t % 8) ^ ((row >> 1) & 7));  // the same for rows 32 apart
 #pragma unroll
-    for (int c = 0; c < kCopies; ++c) {
+    for (int c = 0; c < R; ++c) {
       const uint32_t m = (uint32_t)(mt * kBM + row + 32 * c);
       xoff[c] = (m < last ? m : last) * ld + chunk;  // rows past M re-read the last row (never stored)
     }
@@ -170,13 +175,13 @@ __global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojA
   x_tile(vx);
   w_tile(vw);
 
-  f32x4 acc[8][8];
+  f32x4 acc[8][R];
 
   // operand fragments of k-step s (32 wide): A = W rows 128 nh + 16 i + l16, B =
-  // x rows 128 mh + 16 j + l16, logical chunk 4 s + g: the offset of chunk g
+  // x rows 16 R mh + 16 j + l16, logical chunk 4 s + g: the offset of chunk g
   // XOR 64 s (4 s only touches the top bit of the chunk), rows 16 i an immediate
-  const uint32_t offA = swz(nh * 128 + l16, g), offB = swz(mh * 128 + l16, g);
-  bf16x8 av[2][8], bv[2][8];
+  const uint32_t offA = swz(nh * 128 + l16, g), offB = swz(mh * 16 * R + l16, g);
+  bf16x8 av[2][8], bv[2][R];
   uint32_t get = 0;  // slot of the stage's x tile; its W tile is in the next one
   uint32_t pA = 0, pB = 0;
   auto stage_at = [&] {
@@ -186,33 +191,33 @@ __global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojA
     get = next_slot(get);
   };
   auto load = [&](int s, int i) {
-    bv[s][i] = *reinterpret_cast<const bf16x8*>(smem + (pB ^ (64u * s)) + 16 * kRowBytes * i);
+    if (i < R) bv[s][i] = *reinterpret_cast<const bf16x8*>(smem + (pB ^ (64u * s)) + 16 * kRowBytes * i);
     av[s][i] = *reinterpret_cast<const bf16x8*>(smem + (pA ^ (64u * s)) + 16 * kRowBytes * i);
   };
   auto mul = [&](int s, int i) {
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < 8; ++j)
+    for (int j = 0; j < R; ++j)
       asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc[i][j]) : "v"(av[s][i]), "v"(bv[s][j]));
     __builtin_amdgcn_sched_barrier(0);
   };
   // both tiles of the next stage have landed (the x tile after them may still
   // be in flight) and every wave has its fragments of this one
   auto landed = [&] {
-    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kCopies));
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(R));
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
   };
 
 #pragma unroll
-  for (int c = 0; c < kCopies; ++c) copy_x(c);
+  for (int c = 0; c < R; ++c) copy_x(c);
   copied_x();
 #pragma unroll
   for (int c = 0; c < kCopies; ++c) copy_w(c);
   copied_w();
 #pragma unroll
-  for (int c = 0; c < kCopies; ++c) copy_x(c);
+  for (int c = 0; c < R; ++c) copy_x(c);
   copied_x();
   landed();
   stage_at();
@@ -225,7 +230,7 @@ __global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojA
 #pragma unroll
     for (int i = 0; i < 8; ++i)
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+      for (int j = 0; j < R; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     asm volatile("s_nop 7");  // before inline assembly reads them
     for (int ks = 0; ks < nsteps; ++ks) {
       // 64 MFMAs of step 0 while step 1's fragments are read and an x tile is copied
@@ -233,7 +238,7 @@ __global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojA
       for (int i = 0; i < 8; ++i) {
         load(1, i);
         mul(0, i);
-        copy_x(i);
+        if (i < R) copy_x(i);
       }
       copied_x();
       landed();
@@ -255,7 +260,7 @@ __global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojA
     // row r at c ^ (r & 15), and stores rows of 256 bytes.
     int mt, nt;
     tile_of(v, mt, nt);
-    const int m0 = mt * kBM + 128 * mh, n0 = nt * kBN + 128 * nh, M = (int)a.M;
+    const int m0 = mt * kBM + 16 * R * mh, n0 = nt * kBN + 128 * nh, M = (int)a.M;
     const int lane = opaque_thread_id() & 63, g = lane >> 4, l16 = lane & 15;
     uint8_t* const stage = smem + put + 8192u * (uint32_t)w;
     asm volatile("s_nop 15\n\ts_nop 15");  // the last MFMAs' results, read by inline assembly below
@@ -263,9 +268,9 @@ __global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojA
 #pragma unroll
     for (int i = 0; i < 8; ++i)
       bias[i] = a.bias ? *reinterpret_cast<const uint2*>(a.bias + n0 + 16 * i + 4 * g) : uint2{0u, 0u};
-    float ss[8];  // squares of the stored values of this lane's row, per m block
+    float ss[R];  // squares of the stored values of this lane's row, per m block
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < R; ++j) {
       ss[j] = 0.0f;
       const int row = 16 * (j & 1) + l16;
 #pragma unroll
@@ -298,7 +303,7 @@ __global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojA
     // different columns of the same row; then the two waves of a row
     float* const part = reinterpret_cast<float*>(stage);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
+    for (int j = 0; j < R; ++j) {
       const float t = xor32_add(ss[j] + __shfl_xor(ss[j], 16));
       if (g == 0) part[16 * j + l16] = t;
     }
@@ -307,9 +312,10 @@ __global__ __launch_bounds__(kOprojThreads, 1) void linear_rownorm_kernel(OprojA
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
     if (nh == 0) {
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
+      for (int h = 0; h < (R + 3) / 4; ++h) {
         const int m = m0 + 64 * h + lane;
-        if (m < M) a.partial[(int64_t)m * a.ntiles + nt] = part[64 * h + lane] + part[2 * 2048 + 64 * h + lane];
+        if (m < M && 64 * h + lane < 16 * R)
+          a.partial[(int64_t)m * a.ntiles + nt] = part[64 * h + lane] + part[2 * 2048 + 64 * h + lane];
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
@@ -331,6 +337,32 @@ __global__ __launch_bounds__(256) void rownorm_finish_kernel(const float* __rest
   else reinterpret_cast<float*>(norms)[m] = r;
 }
 
+template <int R>
+void launch_rows(OprojArgs a, int cus, hipStream_t stream) {
+  a.mtiles = (int)((a.M + 32 * R - 1) / (32 * R));
+  a.total = a.mtiles * a.ntiles;
+  linear_rownorm_kernel<R><<<(unsigned)(a.total < cus ? a.total : cus), kOprojThreads, 0, stream>>>(a);
+}
+
+// Rows per output tile: the height whose rounds of tiles cost least.  A round of
+// 256, 128 and 64 rows takes 118, 67 and 59 us at K = 5,120 (the lower tiles
+// wait for the copies of W, not for the matrix cores), in much the same ratios
+// at other K.  Measured, 256 against 128 against 64 rows (N = K): 200 x 5,120 98
+// / 64 / 60 us; 700 x 1,536 39 / 24 / 18; 1,000 x 5,120 103 / 68 / 119; 4,000 x
+// 5,120 213 / 207 / 301; 6,528 x 5,120 323 / 291 / 469; 8,000 x 1,536 45 / 54 /
+// 60; 12,000 x 5,120 483 / 544 / 852.
+void launch_rownorm(const OprojArgs& a, hipStream_t stream) {
+  const int cus = resident_workgroups<linear_rownorm_kernel<8>>(kOprojThreads);
+  auto cost = [&](int rows, int64_t us) {
+    const int64_t tiles = (a.M + rows - 1) / rows * a.ntiles;
+    return (tiles + cus - 1) / cus * us;
+  };
+  const int64_t c8 = cost(256, 118), c4 = cost(128, 67), c2 = cost(64, 59);
+  if (c8 <= c4 && c8 <= c2) launch_rows<8>(a, cus, stream);
+  else if (c4 <= c2) launch_rows<4>(a, cus, stream);
+  else launch_rows<2>(a, cus, stream);
+}
+
 }  // namespace
 
 extern "C" {
@@ -345,14 +377,12 @@ int prism_linear_rownorm(const void* x, const void* w, const void* bias, int64_t
   // per-lane source offsets are 32-bit byte offsets from the tensors' bases
   PRISM_REQUIRE(M * (int64_t)K * 2 < (1ll << 32) && (int64_t)N * K * 2 < (1ll << 32),
                 "prism_linear_rownorm: x and W must each be smaller than 4 GiB");
-  const int64_t mtiles = (M + kBM - 1) / kBM;
   const int ntiles = N / kBN;
-  PRISM_REQUIRE(mtiles * ntiles < (1ll << 31), "prism_linear_rownorm: grid too large");
+  PRISM_REQUIRE((M + 63) / 64 * ntiles < (1ll << 31), "prism_linear_rownorm: grid too large");
   OprojArgs a;
   a.x = (const uint16_t*)x; a.w = (const uint16_t*)w; a.bias = (const uint16_t*)bias;
-  a.M = M; a.N = N; a.K = K; a.mtiles = (int)mtiles; a.ntiles = ntiles; a.total = (int)(mtiles * ntiles); a.y = (uint16_t*)y; a.partial = partial;
-  const int resident = resident_workgroups<linear_rownorm_kernel>(kOprojThreads);
-  linear_rownorm_kernel<<<(unsigned)(a.total < resident ? a.total : resident), kOprojThreads, 0, stream>>>(a);
+  a.M = M; a.N = N; a.K = K; a.ntiles = ntiles; a.y = (uint16_t*)y; a.partial = partial;
+  launch_rownorm(a, stream);
   const unsigned fb = (unsigned)((M + 255) / 256);
   if (norms_dtype == PRISM_BF16) rownorm_finish_kernel<uint16_t><<<fb, 256, 0, stream>>>(partial, M, ntiles, (uint16_t*)norms);
   else rownorm_finish_kernel<float><<<fb, 256, 0, stream>>>(partial, M, ntiles, (float*)norms);

@@ -58,10 +58,11 @@ def test_linear_rownorm_small(M, N, K, bias):
 
 
 @pytest.mark.parametrize("M,N,K,bias", [(33000, 768, 64, True), (16897, 1280, 128, False), (17151, 1280, 192, True),
-                                        (1, 256, 64, True), (255, 512, 128, True), (257, 256, 2560, False)], ids=str)
+                                        (1, 256, 64, True), (255, 512, 128, True), (257, 256, 2560, False), (65, 1024, 64, True)], ids=str)
 def test_linear_rownorm_tile_streams(M, N, K, bias):
     """Several output tiles per workgroup with one, two and three stages each
-    (the copies of a tile start up to two tiles before it), partial last tiles."""
+    (the copies of a tile start up to two tiles before it), partial last tiles;
+    tiles of 256 rows (33,000 x 768), 128 (17,000 x 1,280) and 64 (below)."""
     from prism_amd import ops
     x, w, b = _inputs(M, N, K, bias, seed=M)
     y, n32 = ops.linear_rownorm(x, w, b, torch.float32)
