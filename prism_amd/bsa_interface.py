@@ -74,6 +74,43 @@ def _check_chunks(chunk_size_q, chunk_size_k):
                          f"chunk_size_k={chunk_size_k})")
 
 
+def _forward_route(pairs: int, Ntq: int, width: int, D: int) -> str:
+    """How attn_fwd_bsa_varlen walks `pairs` pairs of query tiles (Ntq tiles a
+    head) whose lists hold up to `width` entries:
+
+      tiles   one workgroup per query tile (at most ops.TILE_PAIRS pairs)
+      plain   neighbouring tiles paired, no launch order
+      sorted  tiles paired by overlap, all pairs longest first
+      tail    neighbouring tiles paired, the last ones launched longest first
+      quads   four tiles per workgroup, paired by overlap
+
+    Pairing by overlap costs 23-27 us, an order 6-19 us, and a sorted run mixes
+    the heads, which then share no K and V tile in the L2s: lists of up to 64
+    entries, or one round of pairs (512 workgroups), do not earn that back.
+    Long lists do, in their order's even end: sorted up to 2.5 rounds at D = 64
+    and two at D = 128, the tail alone beyond.  Measured, us of the whole call
+    over lists half of whose entries are near the diagonal, quads / sorted /
+    plain / tail: 512 pairs, width 16, D = 128: 98 / 124 / 83 / 89 (106 paired
+    by overlap without an order); 1,024 pairs, width 128, D = 64: 483 / 379 /
+    401 / 386; 1,536 pairs, width 256, D = 128: 1,468 / 1,500 / 1,574 / 1,502;
+    3,840 pairs, width 32, D = 128: 618 / 706 / 541 / 564.
+    Quads prefetch deeper, which short lists of small tiles need where they come
+    in two half-full rounds of pairs (768 pairs, width 6, D = 64: 79 us against
+    96 plain).  From ops.SPLIT_PAIRS on, quads share the tile copies."""
+    if pairs <= ops.TILE_PAIRS:
+        return "tiles"
+    quads = ops.QUADS and Ntq % 4 == 0
+    if pairs >= ops.SPLIT_PAIRS:
+        return "quads" if quads else "plain"
+    if quads and D == 64 and 640 <= pairs <= 1024 and width <= 16:
+        return "quads"
+    if pairs <= 512 or width <= 64:
+        return "plain"
+    if pairs <= (1280 if D == 64 else 1024):
+        return "sorted"
+    return "tail" if width > 128 else "plain"
+
+
 def attn_fwd_bsa_varlen(q, k, v, sm_scale, block_indices, block_indices_lens, chunk_size_q=64, chunk_size_k=64,
                         sparsity=None, kv_valid_mask: Optional[torch.Tensor] = None):
     """Block-sparse attention forward over per-query-tile key-tile lists
@@ -84,21 +121,23 @@ def attn_fwd_bsa_varlen(q, k, v, sm_scale, block_indices, block_indices_lens, ch
     qstart, qlen, qcols = _lists_from_dense(block_indices, block_indices_lens)
     Ntq, Ntk = q.shape[2] // 64, k.shape[2] // 64
     tm = ops.tile_masks(ops._u8(kv_valid_mask))
-    pairs = q.shape[0] * q.shape[1] * Ntq // 2
-    if pairs <= ops.TILE_PAIRS:
+    route = _forward_route(q.shape[0] * q.shape[1] * Ntq // 2, Ntq, block_indices.shape[-1], q.shape[-1])
+    if route == "tiles":
         return ops.bsa_fwd_tile(q, k, v, tm, ops.tile_lists(qstart, qlen, qcols, Ntq, tm, Ntk), sm_scale)
-    if pairs < ops.SPLIT_PAIRS:
-        qpair = ops.pair_tiles(qstart, qlen, qcols, Ntq, Ntk)
-        qunion = ops.pair_union(qstart, qlen, qcols, Ntq, tm, col_tiles=Ntk, pairmap=qpair)
-        return ops.bsa_fwd(q, k, v, tm, qunion, sm_scale, qpair, ops.items_order(qunion[1], 64))
-    if ops.QUADS and Ntq % 4 == 0:
+    if route == "quads":
         # four query tiles per staged K / V tile (two overlap pairs of each
         # group of 8), the same outputs bit for bit
         qpair = ops.pair_tiles(qstart, qlen, qcols, Ntq, Ntk)
         quad = ops.quad_union(qstart, qlen, qcols, Ntq, tm, col_tiles=Ntk, pairmap=qpair)
         return ops.bsa_fwd_quad(q, k, v, tm, quad, sm_scale, qpair, ops.pair_order(quad[1], 32))
-    qunion = ops.pair_union(qstart, qlen, qcols, Ntq, tm, col_tiles=Ntk)
-    return ops.bsa_fwd(q, k, v, tm, qunion, sm_scale)
+    qpair = ops.pair_tiles(qstart, qlen, qcols, Ntq, Ntk) if route == "sorted" else None
+    qunion = ops.pair_union(qstart, qlen, qcols, Ntq, tm, col_tiles=Ntk, pairmap=qpair)
+    order = None
+    if route == "sorted":
+        order = ops.launch_order(qunion[1], 1, 0)[0]
+    elif route == "tail":
+        order = ops.pair_order(qunion[1], 64)
+    return ops.bsa_fwd(q, k, v, tm, qunion, sm_scale, qpair, order)
 
 
 def create_indices_k_from_indices_q_varlen(block_indices: torch.Tensor, N_cols_mask: int):

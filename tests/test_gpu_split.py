@@ -53,6 +53,55 @@ def test_tile_forward_equals_pair_forward(shape):
     assert bits_equal(host(o1), host(o2)) and bits_equal(host(l1), host(l2))
 
 
+def called(monkeypatch):
+    """The names of the operators that run from here on."""
+    from prism_amd import ops
+    names, run = [], ops._op
+    monkeypatch.setattr(ops, "_op", lambda name, *args: (names.append(name), run(name, *args))[1])
+    return names
+
+
+# (BH, Nt, width, D, operators after tile_masks): both sides of every line of
+# the rule that picks the forward of given lists
+ROUTES = [(2, 128, 9, 64, ["tile_lists", "bsa_fwd_tile"]),
+          (2, 130, 9, 128, ["pair_union", "bsa_fwd"]),
+          (4, 256, 70, 64, ["pair_union", "bsa_fwd"]),
+          (2, 640, 16, 64, ["pair_tiles", "quad_union", "pair_order", "bsa_fwd_quad"]),
+          (2, 642, 16, 64, ["pair_union", "bsa_fwd"]),
+          (2, 640, 16, 128, ["pair_union", "bsa_fwd"]),
+          (2, 636, 16, 64, ["pair_union", "bsa_fwd"]),
+          (2, 640, 17, 64, ["pair_union", "bsa_fwd"]),
+          (2, 514, 64, 64, ["pair_union", "bsa_fwd"]),
+          (2, 514, 65, 64, ["pair_tiles", "pair_union", "launch_order", "bsa_fwd"]),
+          (2, 1026, 129, 128, ["pair_union", "pair_order", "bsa_fwd"]),
+          (2, 1026, 128, 128, ["pair_union", "bsa_fwd"]),
+          (2, 1282, 130, 64, ["pair_union", "pair_order", "bsa_fwd"]),
+          (16, 512, 5, 64, ["pair_tiles", "quad_union", "pair_order", "bsa_fwd_quad"]),
+          (64, 130, 5, 64, ["pair_union", "bsa_fwd"])]
+
+
+@pytest.mark.parametrize("shape", ROUTES, ids=str)
+def test_given_lists_forward_routes(shape, monkeypatch):
+    """attn_fwd_bsa_varlen: the kernels and launch orders of the rule, and the
+    bits of the pair forward over neighbouring pairs whichever it takes (empty
+    lists, unsorted rows, key masks)."""
+    from prism_amd import bsa_interface, ops
+    BH, Nt, W, D, want = shape
+    say("forward route", shape)
+    g = torch.Generator(device="cuda").manual_seed(W)
+    q, k, v = (torch.randn((1, BH, Nt * 64, D), device="cuda", generator=g).to(torch.bfloat16) for _ in range(3))
+    idx = torch.sort(torch.rand((1, BH, Nt, Nt), device="cuda", generator=g), -1).indices[..., :W].contiguous()
+    lens = torch.randint(0, W + 1, (1, BH, Nt), device="cuda", generator=g, dtype=torch.int32)
+    valid = torch.rand((Nt * 64,), device="cuda", generator=g) < 0.8
+    tm, sm = ops.tile_masks(valid), 1.0 / math.sqrt(D)
+    union = ops.pair_union(*bsa_interface._lists_from_dense(idx, lens), Nt, tm, col_tiles=Nt)
+    ref = ops.bsa_fwd(q, k, v, tm, union, sm)
+    names = called(monkeypatch)
+    got = bsa_interface.attn_fwd_bsa_varlen(q, k, v, sm, idx, lens, kv_valid_mask=valid)
+    assert [n for n in names if n != "tile_masks"] == want
+    assert all(bits_equal(host(a), host(b)) for a, b in zip(ref, got))
+
+
 # (whole, splits): every pair split, some, none
 @pytest.mark.parametrize("shape", [(1, 2, 2, 64, 2, False, 0, 2), (3, 6, 10, 64, 6, True, 3, 3),
                                    (2, 10, 40, 128, 40, True, 4, 5), (2, 16, 24, 128, 24, False, 16, 1),
