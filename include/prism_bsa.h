@@ -394,6 +394,9 @@ int prism_bsa_fwd_tile(const void* q, const void* k, const void* v, int BH, int6
  * unsplit entry points'.  With n = whole + (pairs - whole) * splits items,
  * ustart / ulen / ucols are prism_part_union's n rows (entries as
  * prism_pair_union's) and order (or NULL) is a permutation of [0, n).
+ * prism_part_union's rows are ucap entries apart, those of split pairs only as
+ * many as such a row can hold: with c = min(col_tiles, 8 * ceil(col_tiles / (8 *
+ * splits))), ucols holds whole * ucap + (pairs - whole) * splits * c.
  * prism_split_plan chooses whole and splits on the host for `heads` x
  * pairs_per_head pairs (Sq/128 per head; for dK/dV Sk/128) whose lists hold up
  * to max_entries entries (Sk/64; for dK/dV Sq/64); kernel: 1 dQ, 2 dK/dV.

@@ -225,9 +225,10 @@ def _register_fakes():
 
     @reg("prism::part_union")
     def _(start, length, cols, row_tiles, col_tiles, pairmap, tile_masks, whole, splits):
-        items = whole + (start.numel() // 2 - whole) * splits
+        rest = start.numel() // 2 - whole
+        items, cap = whole + rest * splits, min(col_tiles, -(-col_tiles // (8 * splits)) * 8)
         return (_empty(start, (items,), i64), _empty(start, (items,), i32),
-                _empty(start, (max(items * col_tiles, 1),), i32))
+                _empty(start, (max(whole * col_tiles + rest * splits * cap, 1),), i32))
 
     @reg("prism::tile_lists")
     def _(start, length, cols, row_tiles, col_tiles, tile_masks):

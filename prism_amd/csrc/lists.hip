@@ -34,7 +34,8 @@ constexpr int kUnionWin = 8192;  // tiles per LDS bitmap window (256 words)
 // member bits (bit k: row k lists the tile).
 // SPLIT (R = 2): row b is work item b of a split launch (split.h): a whole
 // pair, or the entries of a pair whose tile t has (t / 8) mod splits equal to
-// the item's number within its pair.
+// the item's number within its pair.  Rows are ucap entries apart, those of
+// split pairs split_item_cap (<= ucap).
 template <int R, bool SPLIT>
 __global__ __launch_bounds__(256) void pair_union_kernel(const int64_t* __restrict__ start,
                                                     const int32_t* __restrict__ len,
@@ -59,7 +60,8 @@ __global__ __launch_bounds__(256) void pair_union_kernel(const int64_t* __restri
     nl[k] = len[r];
   }
   // list entries index column tiles inside one head (0 .. Nc-1), as does tile_masks
-  int32_t* out = ucols + row * ucap;
+  const int64_t first = SPLIT && item.slot >= 0 ? whole * ucap + item.slot * split_item_cap(Nc, splits) : row * ucap;
+  int32_t* out = ucols + first;
   int count = 0;
   for (int64_t w0 = 0; w0 < Nc; w0 += kUnionWin) {
 #pragma unroll
@@ -114,7 +116,7 @@ __global__ __launch_bounds__(256) void pair_union_kernel(const int64_t* __restri
     __syncthreads();
   }
   if (tid == 0) {
-    ustart[row] = row * ucap;
+    ustart[row] = first;
     ulen[row] = count;
   }
 }

@@ -43,6 +43,14 @@ __host__ __device__ __forceinline__ SplitItem split_item(int whole, int splits, 
   return SplitItem{whole + (it - whole) / splits, it - whole};
 }
 
+// Entries that an item of a split pair can hold: its groups of eight of the
+// col_tiles listed tiles.  (The pairs' items together: little more than the
+// pair's own row, not `splits` rows.)
+__host__ __device__ __forceinline__ int64_t split_item_cap(int64_t col_tiles, int splits) {
+  const int64_t cap = (col_tiles + 8 * splits - 1) / (8 * splits) * 8;
+  return cap < col_tiles ? cap : col_tiles;
+}
+
 // Which pairs to split, and into how many items, for heads * per_head pairs on
 // `slots` workgroups.  Launches of eight rounds or more keep whole lists: the
 // work queue already ends them within an eighth of their time, usually much

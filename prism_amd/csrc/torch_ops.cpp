@@ -478,7 +478,9 @@ std::tuple<Tensor, Tensor, Tensor> part_union(const Tensor& s_, const Tensor& l_
   const int64_t items = whole + (pairs - whole) * splits;
   Tensor ustart = at::empty({items}, opts(s, at::kLong));
   Tensor ulen = at::empty({items}, opts(s, at::kInt));
-  Tensor ucols = at::empty({std::max<int64_t>(items * col_tiles, 1)}, opts(s, at::kInt));
+  const int64_t cap = std::min(col_tiles, (col_tiles + 8 * splits - 1) / (8 * splits) * 8);  // of a split pair's item
+  Tensor ucols =
+      at::empty({std::max<int64_t>(whole * col_tiles + (pairs - whole) * splits * cap, 1)}, opts(s, at::kInt));
   PRISM_TORCH_CALL(prism_part_union, s.data_ptr<int64_t>(), l.data_ptr<int32_t>(), c.data_ptr<int32_t>(), rows,
                    row_tiles, col_tiles, (const int32_t*)p(pairmap), (const uint64_t*)p(masks), whole, (int)splits, col_tiles,
                    ustart.data_ptr<int64_t>(), ulen.data_ptr<int32_t>(), ucols.data_ptr<int32_t>(), stream_of(s));

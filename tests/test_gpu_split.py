@@ -124,6 +124,8 @@ def test_split_backward(shape):
         us, ul, uc = (host(t) for t in un)
         s, n, c = (host(t) for t in it)
         assert n.size == w + (ul.size - w) * splits
+        # the items of a pair take little more than the pair's own row
+        assert c.size <= uc.size + 8 * (n.size - w)
         for i in range(n.size):
             p, part = (i, -1) if i < w else (w + (i - w) // splits, (i - w) % splits)
             e = uc[us[p]: us[p] + ul[p]]

@@ -110,3 +110,15 @@ def test_fake_split_csr(prism):
         # no entries: still a one-element buffer (a valid pointer for the kernels)
         ent = prism.lists_csr_fill(_t((100,), torch.int64), _t((100,), torch.int32), _t((5000,), torch.int32), off, 0)
         assert ent.shape == (1,)
+
+
+def test_fake_part_union_rows(prism):
+    """A split pair's items share its row's room: eight entries more at most
+    per item, whatever the number of items."""
+    lists = [(s, d) for s, d in (((200,), torch.int64), ((200,), torch.int32), ((900,), torch.int32))]
+    with FakeTensorMode():
+        for whole, splits, tiles in ((0, 7, 8000), (60, 16, 515), (100, 1, 9), (0, 1, 9), (3, 64, 520)):
+            us, ul, uc = prism.part_union(*(_t(s, d) for s, d in lists), 200, tiles, None, None, whole, splits)
+            items = whole + (100 - whole) * splits
+            assert us.shape == ul.shape == (items,)
+            assert 100 * tiles <= uc.numel() <= 100 * tiles + 8 * (items - whole)
