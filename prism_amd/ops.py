@@ -440,9 +440,9 @@ class DeferredCompaction:
     """Compaction of several (start, len, cols) lists into CSR with one host
     read for all of them.  add() launches a list's offsets on the current
     stream and copies its nnz into pinned host memory without waiting;
-    finish() waits for those copies (their events, not the streams: work
+    fill() waits for those copies (their events, not the streams: work
     queued after them, such as an attention kernel, is not waited for), then
-    fills every list's CSR entries on the current stream.  The entries and
+    fills a list's CSR entries on the current stream.  The entries and
     their order are the source lists'."""
 
     def __init__(self, n: int):
@@ -471,10 +471,6 @@ class DeferredCompaction:
         if self.offsets[i] is None:
             return lists
         return (*csr_lists(self.offsets[i]), csr_fill(*lists, self.offsets[i], self.sizes()[i]))
-
-    def finish(self, lists_seq):
-        """fill of every list: lists_seq[i] was added as i."""
-        return [self.fill(i, lists) for i, lists in enumerate(lists_seq)]
 
 
 def csr_lists(offsets: torch.Tensor):
@@ -603,8 +599,10 @@ def bsa_fwd(q, k, v, tmasks, qunion, sm_scale: float, qpair: Optional[torch.Tens
 # TILE_PAIRS (one tile per CU) walk single tiles.
 SPLIT_PAIRS = 4096
 TILE_PAIRS = 128
-# A side of a few rounds keeps up to this much of dense lists to the backward:
-# compact ones would cost a host read of their size and launches of their own.
+# A side of a few rounds whose per-tile lists and whose pair unions, twice over,
+# fit this keeps what its backward walks (pair unions or split items: at most
+# half of it) as dense rows: compact ones would cost a host read of their size
+# and launches of their own.
 KEEP_DENSE_BYTES = 64 << 20
 
 

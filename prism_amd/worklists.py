@@ -18,12 +18,12 @@ class _Side:
     dK/dV), built when first asked for."""
 
     def __init__(self, source, rows, cols, BH, D, keys, tmasks):
-        self.source = source      # the per-tile lists (start, len, cols)
+        self.source = source      # the per-tile lists (start, len, cols), until release()
         self.rows, self.cols, self.BH, self.D, self.keys, self.tmasks = rows, cols, BH, D, keys, tmasks
         self.group = 32 if keys else 64
         pairs = BH * (rows // 2)
-        # a side of a few rounds of workgroups: its dense lists are kept as
-        # they are (at most ops.KEEP_DENSE_BYTES)
+        # a side of a few rounds of workgroups whose lists take little room:
+        # what its backward walks is kept dense (ops.KEEP_DENSE_BYTES)
         self.small = (pairs < 8 * 8 * self.group
                       and 4 * max(2 * pairs * cols, source[2].numel()) <= ops.KEEP_DENSE_BYTES)
         self._pairmap = self._pairs = self._items = None
@@ -38,25 +38,19 @@ class _Side:
             self._pairmap = ops.pair_tiles(*self.source, self.rows, self.cols)
         return self._pairmap
 
-    def union(self):
-        return ops.pair_union(*self.source, self.rows, self.tmasks, col_tiles=self.cols, pairmap=self.pairmap)
-
     @property
     def pairs(self):
-        """Pair unions."""
-        if self._pairs is None:
-            self._pairs = self.union()
+        """Pair unions (None once a split side is released)."""
+        if self._pairs is None and self.source is not None:
+            self._pairs = ops.pair_union(*self.source, self.rows, self.tmasks, col_tiles=self.cols,
+                                         pairmap=self.pairmap)
         return self._pairs
-
-    @pairs.setter
-    def pairs(self, value):
-        self._pairs = value
 
     @property
     def items(self):
         """The backward's lists: the work items of a split launch where a
         launch over the pairs would leave the GPU partly idle, else the pairs."""
-        if self._items is None and self.small:
+        if self._items is None and self.small and self.source is not None:
             whole, splits = ops.split_plan(2 if self.keys else 1, self.BH, self.rows // 2, self.cols, self.D)
             if splits > 1:
                 self.split = (whole, splits)
@@ -71,6 +65,28 @@ class _Side:
             self._orders[key] = ops.items_order(lists[1], self.group, self.BH, self.cache_bytes)
         return self._orders[key]
 
+    def release(self, walked=True):
+        """Keep the backward's lists, their order (if it walks them) and the
+        pairing alone."""
+        items = self.items
+        if walked:
+            self.order(items)
+        if self._items is not None:
+            self._pairs = None
+            self._orders.pop("pairs", None)
+        self.source = None
+
+    def compact(self, pairs):
+        """The pair unions as CSR: the same rows and entries."""
+        self._pairs = pairs
+
+    def tensors(self):
+        """Every list, pairing and order that the side holds."""
+        for lists in (self.source, self._pairs, self._items):
+            yield from lists or ()
+        yield self._pairmap
+        yield from self._orders.values()
+
     @property
     def cache_bytes(self):
         """bf16 operand rows that the lists index (K and V, or Q and dO)."""
@@ -81,9 +97,11 @@ class WorkLists:
     """Base of the plans.  A plan sets qstart, qlen, qcols (its per-query-tile
     key lists) and calls _build_query_lists.
 
-    A query side of fewer than eight rounds of workgroups walks pairs (its
-    forward single tiles when there are few), whatever the quad switches say; a
-    larger one walks pairs or quads, as the switches and the lists say."""
+    A side of fewer than eight rounds of workgroups whose lists fit
+    ops.KEEP_DENSE_BYTES is small: its backward walks pairs, split where that
+    fills the GPU, its forward pairs or, when there are few, single tiles,
+    whatever the quad switches say.  A larger one walks pairs or quads, as the
+    switches and the lists say."""
 
     def _build_query_lists(self, BH, Ntq, Ntk, D, tmasks, compact, dq_quads):
         self._BH, self._Ntq, self._Ntk, self._D = BH, Ntq, Ntk, D
@@ -97,43 +115,28 @@ class WorkLists:
         self._k = None
         self._few = self._q.small and BH * Ntq // 2 <= ops.TILE_PAIRS
         # quad unions (two pairs of a group per workgroup: four query tiles per
-        # staged K / V tile); quads: the call may walk them, dq_quads: dQ too
+        # staged K / V tile) of a large side; quads: the switches and tile
+        # counts allow them, dq_quads: for dQ too
         self.quads = ops.QUADS and Ntq % 4 == 0
         self.dq_quads = self.quads and dq_quads
-        self._qquad = self._qquad_order = self._qquad_total = None
-        self._shown = {}
+        self.qquad = self.qquad_order = self._qquad_total = None
         if self.quads and not self._q.small:
-            self._qquad = self._query_quads()
-            self._qquad_order, self._qquad_total = ops.launch_order(self._qquad[1], BH, self._q.cache_bytes)
+            self.qquad = ops.quad_union(*self._q.source, Ntq, tmasks, col_tiles=Ntk, pairmap=self.qpair)
+            self.qquad_order, self._qquad_total = ops.launch_order(self.qquad[1], BH, self._q.cache_bytes)
         self.klists = None
         self.keys_ready = None  # event of a key-list build on the side stream
 
-    def _query_quads(self):
-        return ops.quad_union(*self._q.source, self._Ntq, self.tmasks, col_tiles=self._Ntk, pairmap=self.qpair)
-
-    # ------------------------------------------------ the lists, for inspection
-    def _union_of(self, name, side):
-        """A side's pair unions.  A small side's kernels may walk other lists,
-        and keep them dense: its unions are built when asked for, as CSR once a
-        compact plan has settled."""
-        if side is None or not side.small:
-            return None if side is None else side.pairs
-        if name not in self._shown:
-            u = side.union()
-            if self._settled and self.compact:
-                u = (*ops.csr_lists(ops.csr_offsets(u[1])[0]), ops.lists_to_csr(*u)[1])
-            self._shown[name] = u
-        return self._shown[name]
-
+    # ------------------------------------------------ the lists, for callers that launch the kernels themselves
     @property
     def qunion(self):
-        """Query-side pair unions (CSR once a compact plan has settled)."""
-        return self._union_of("q", self._q)
+        """Query-side pair unions (CSR once a compact plan of a large side has
+        settled; None once a split side has)."""
+        return self._q.pairs
 
     @property
     def kunion(self):
         """Key-side pair unions, once build_key_lists has run."""
-        return self._union_of("k", self._k)
+        return None if self._k is None else self._k.pairs
 
     @property
     def qpair(self):
@@ -145,34 +148,12 @@ class WorkLists:
 
     @property
     def qorder(self):
-        """A launch order of the pair kernels over qunion."""
-        if "qorder" not in self._shown:
-            self._shown["qorder"] = ops.pair_order(self.qunion[1], 64)
-        return self._shown["qorder"]
+        """A launch order over qunion (launches that all run at once go without one)."""
+        return ops.launch_order(self.qunion[1], self._BH, self._q.cache_bytes)[0]
 
     @property
     def korder(self):
-        if "korder" not in self._shown and self._k is not None:
-            self._shown["korder"] = ops.pair_order(self.kunion[1], 32)
-        return self._shown.get("korder")
-
-    @property
-    def qquadmap(self):
-        return self.qpair if self.quads else None
-
-    @property
-    def qquad(self):
-        """Quad unions (None where the call cannot walk them or has released
-        them); a small query side builds them when asked."""
-        if self._qquad is None and self._q.small and (self.dq_quads if self._settled else self.quads):
-            self._qquad = self._query_quads()
-        return self._qquad
-
-    @property
-    def qquad_order(self):
-        if self._qquad_order is None and self.qquad is not None:
-            self._qquad_order = ops.pair_order(self._qquad[1], 32)
-        return self._qquad_order
+        return None if self._k is None else ops.launch_order(self.kunion[1], self._BH, self._k.cache_bytes)[0]
 
     # ------------------------------------------------ key-side lists
     def build_key_lists_side(self):
@@ -219,53 +200,48 @@ class WorkLists:
             if not self._q.small:
                 self._csr.add(0, self._q.pairs)
                 if self.dq_quads:
-                    self._csr.add(2, self._qquad)
+                    self._csr.add(2, self.qquad)
             if self._k is not None and not self._k.small:
                 self._csr.add(1, self._k.pairs)
 
     def settle(self):
-        """Keep only what the backward reads: each side's lists (a large
-        side's pair unions, and the quad unions when dQ walks them, as CSR when
-        the plan is compact, with one batched host read of their sizes),
-        pairings and launch orders.  A large side's per-tile lists (1.0 GB
-        query-side and 0.66 GB key-side at a 21 x 90 x 160 grid with 5 heads)
-        and the forward-only quad unions are released."""
+        """Keep only what the backward reads: each side's lists, their launch
+        order and the pairing.  A large side's are its pair unions (or, where dQ
+        walks them, the quad unions beside them), as CSR when the plan is
+        compact, with one batched host read of their sizes; a small side's its
+        pair unions or split items.  The per-tile lists (1.0 GB query-side and
+        0.66 GB key-side at a 21 x 90 x 160 grid with 5 heads) and the
+        forward-only quad unions are released."""
         if self._settled:
             return
         self.build_key_lists()
         self._start_compaction()
-        if self.dq_quads and not self._q.small and ops.DQ_QUADS is None:
+        if self.qquad is not None and self.dq_quads and ops.DQ_QUADS is None:
             sizes = None if self._csr is None else self._csr.sizes()
             self.dq_quads = sizes is not None and sizes[0] >= ops.DQ_QUAD_RATIO * sizes[2]
-        if not self.dq_quads and not self._q.small:
-            self._qquad = None
+        if not self.dq_quads:  # not walked by the backward
+            self.qquad = self.qquad_order = None
         if self._csr is not None:
-            self._q._pairs, self._k._pairs = self._csr.finish([self._q._pairs, self._k._pairs])
-            if self._qquad is not None:
-                self._qquad = self._csr.fill(2, self._qquad)
+            for i, side in enumerate((self._q, self._k)):
+                if not side.small:
+                    side.compact(self._csr.fill(i, side.pairs))
+            if self.qquad is not None:
+                self.qquad = self._csr.fill(2, self.qquad)
             self._csr = None
-        if not self.dq_quads or self._q.small:  # not walked by the backward
-            self._qquad = self._qquad_order = None
-        for side in (self._q, self._k):
-            if not side.small:
-                side.source = None
-        self._shown.pop("q", None)
-        self._shown.pop("k", None)
+        self._q.release(walked=self.qquad is None)
+        self._k.release()
         self.qcols = None
         self.klists = None
         self.sel = {key: val for key, val in self.sel.items() if key != "tiles"}
         self._settled = True
 
     def list_bytes(self) -> int:
-        """Bytes of the work lists that the plan holds (small sides: of the
-        pair unions that stand for theirs)."""
-        ts = [*self.qunion, self.qstart, self.qlen]
-        for lists in (self._qquad, self.kunion, self.klists):
-            if lists is not None:
-                ts += list(lists)
-        if self.qcols is not None:
-            ts.append(self.qcols)
-        return sum(t.numel() * t.element_size() for t in ts)
+        """Bytes of the work lists, pairings and launch orders that the plan holds."""
+        held = [self.qstart, self.qlen, self.qcols, self.qquad_order, *(self.qquad or ()), *(self.klists or ())]
+        for side in (self._q, self._k):
+            if side is not None:
+                held += side.tensors()
+        return sum({id(t): t.numel() * t.element_size() for t in held if t is not None}.values())
 
     def sum_lens(self) -> int:
         """Executed (query tile, key tile) pairs (host sync)."""
@@ -288,7 +264,7 @@ class WorkLists:
             out = ops.bsa_fwd_tile(*qkv, ops.tile_lists(*q.source, self._Ntq, self.tmasks, self._Ntk), sm_scale)
         elif self.quads and not q.small:
             order, total = ops.launch_order(q.pairs[1], self._BH, q.cache_bytes, ops.FWD_CHUNK)
-            out = ops.bsa_fwd_either(*qkv, q.pairs, order, total, self._qquad, self._qquad_order, self._qquad_total,
+            out = ops.bsa_fwd_either(*qkv, q.pairs, order, total, self.qquad, self.qquad_order, self._qquad_total,
                                      sm_scale, q.pairmap)
         else:
             out = ops.bsa_fwd(*qkv, q.pairs, sm_scale, q.pairmap, q.order(q.pairs))
@@ -301,11 +277,11 @@ class WorkLists:
         """dq, dk, dv in tile order."""
         self.build_key_lists()
         q, k = self._q, self._k
-        quads = self.dq_quads and not q.small
-        qlists, klists = self._qquad if quads else q.items, k.items
+        quads = self.qquad is not None
+        qlists, klists = self.qquad if quads else q.items, k.items
         return ops.bsa_bwd(self.q_re, self.k_re, self.v_re, do_re, ops.lse_to_m2(lse), delta, self.kv_valid,
                            self.tmasks, qlists, klists, sm_scale, q.pairmap, k.pairmap,
-                           self._qquad_order if quads else q.order(qlists), k.order(klists), after_dkdv=after_dkdv,
+                           self.qquad_order if quads else q.order(qlists), k.order(klists), after_dkdv=after_dkdv,
                            q_quads=quads, q_split=q.split, k_split=k.split)
 
 

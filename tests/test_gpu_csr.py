@@ -87,9 +87,10 @@ def test_select_and_transpose_csr_bitexact(plan_case):
         assert np.array_equal(kq_h[koff_h[r]: koff_h[r + 1]], ref_c[r, : ref_l[r]]), r
 
 
-def test_compact_plan_identical_and_smaller(plan_case):
-    from prism_amd import flash_attn_bsa_3d_dynamic, plan_dynamic
+def test_compact_plan_identical_and_smaller(plan_case, monkeypatch):
+    from prism_amd import flash_attn_bsa_3d_dynamic, ops, plan_dynamic
     c = plan_case
+    monkeypatch.setattr(ops, "KEEP_DENSE_BYTES", -1)  # every launch keeps its lists as a large one does
     outs = []
     for compact in (False, True):
         say("compact_lists", compact)
@@ -129,11 +130,13 @@ def test_compact_plan_identical_and_smaller(plan_case):
     assert sizes[1] < sizes[0]
 
 
-def test_compact_uniform_identical(plan_case):
+def test_compact_uniform_identical(plan_case, monkeypatch):
     """The uniform-shape branch (run_bsa_uniform) with compact lists: same
     output and gradients as with the dense lists."""
+    from prism_amd import ops
     from prism_amd.adapter import run_bsa_uniform
     c = plan_case
+    monkeypatch.setattr(ops, "KEEP_DENSE_BYTES", -1)
     outs = []
     for compact in (False, True):
         say("uniform compact_lists", compact)
@@ -146,18 +149,45 @@ def test_compact_uniform_identical(plan_case):
         assert np.array_equal(a, b)
 
 
-def test_autograd_forward_keeps_only_compact_unions(plan_case):
-    """Through autograd (flash_attn_bsa_3d_dynamic with gradients), the plan
-    the backward holds has released its per-tile lists and keeps the two pair
-    unions as CSR (each entry buffer exactly the union sizes), by default."""
-    from prism_amd import flash_attn_bsa_3d_dynamic
+def _held(plan):
+    """The tensors that hang on the plan's work lists, by walking its
+    attributes (shared ones once)."""
+    seen, todo = {}, [plan._q, plan._k, plan.qquad, plan.qquad_order, plan.klists, plan.qcols, plan.qstart, plan.qlen]
+    while todo:
+        x = todo.pop()
+        if isinstance(x, torch.Tensor):
+            seen[id(x)] = x
+        elif isinstance(x, (tuple, list)):
+            todo += x
+        elif isinstance(x, dict):
+            todo += x.values()
+        elif hasattr(x, "__dict__"):
+            todo += [v for k, v in vars(x).items() if k != "tmasks"]
+    return list(seen.values())
+
+
+@pytest.mark.parametrize("keep", [-1, 64 << 20], ids=["large", "small"])
+def test_autograd_forward_keeps_only_the_backwards_lists(plan_case, keep, monkeypatch):
+    """Through autograd (flash_attn_bsa_3d_dynamic with gradients, compact
+    lists by default): the plan that the backward holds has released its
+    per-tile lists.  A large launch keeps its unions as CSR (each entry buffer
+    exactly the union's size), a small one the dense unions of each side, and
+    list_bytes() is the sum of what hangs on the plan."""
+    from prism_amd import flash_attn_bsa_3d_dynamic, ops
+    monkeypatch.setattr(ops, "KEEP_DENSE_BYTES", keep)
     c = plan_case
     q, k, v = (dev(bf16(c[n])).requires_grad_(True) for n in ("q", "k", "v"))
     o = flash_attn_bsa_3d_dynamic(q, k, v, c["grid"], method="ivpq", sparsity=0.75, cdf_threshold=0.9,
                                   audio_token_norms=dev(c["norms"]), valid_mask=dev(c["valid"]).bool())
     plan = o.grad_fn.plan
+    assert plan._q.small == plan._k.small == (keep > 0)
     assert plan.qcols is None and plan.klists is None and "tiles" not in plan.sel
+    assert plan._q.source is None and plan._k.source is None
+    rows = plan.qstart.numel() // 2
     for u in (plan.qunion, plan.kunion):
-        assert u[2].numel() == int(u[1].sum().item())
+        assert u[0].numel() == rows
+        assert u[2].numel() == (int(u[1].sum().item()) if keep < 0 else rows * plan.lay.Nt)
+    assert plan.list_bytes() == sum(t.numel() * t.element_size() for t in _held(plan))
     o.backward(torch.ones_like(o))
     assert all(bool(torch.isfinite(t.grad).all()) for t in (q, k, v))
+    assert plan.list_bytes() == sum(t.numel() * t.element_size() for t in _held(plan))

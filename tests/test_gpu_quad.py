@@ -14,6 +14,7 @@ import torch
 
 from oracle import oracle as O
 from tests.test_gpu_parity import CASES, bits_equal, dev, host, make, say
+from tests.test_gpu_split import called
 
 pytestmark = pytest.mark.gpu
 
@@ -101,8 +102,28 @@ def test_quad_forward_bitexact_fullsize(cfg):
 
 
 # (ops.QUADS, ops.DQ_QUADS); None: the path's default (dQ on quads on the
-# dynamic-shape path, on pairs on the uniform and cross paths)
+# dynamic-shape path where the lists favour them, on pairs on the uniform and
+# cross paths)
 SWITCHES = ((False, False), (True, False), (True, True), (True, None))
+
+
+def _switched(monkeypatch, quads, dq_quads):
+    """Sets the switches for a launch that takes the large path whatever its
+    size; returns the names of the operators that run from here on."""
+    from prism_amd import ops
+    monkeypatch.undo()
+    monkeypatch.setattr(ops, "KEEP_DENSE_BYTES", -1)
+    monkeypatch.setattr(ops, "QUADS", quads)
+    monkeypatch.setattr(ops, "DQ_QUADS", dq_quads)
+    return called(monkeypatch)
+
+
+def _walked(names, quads, dq_quads):
+    """The attention kernels that ran are those of the switches."""
+    fwd = "bsa_fwd_either" if quads else "bsa_fwd"
+    dq = "bsa_bwd_dq_quad" if dq_quads else "bsa_bwd_dq"
+    attention = [n for n in names if n.startswith("bsa_")]
+    assert attention == [fwd, "bsa_bwd_dkdv", dq], attention
 
 
 @pytest.mark.parametrize("case", [CASES[0], CASES[-1]], ids=[CASES[0][0], CASES[-1][0]])
@@ -115,18 +136,20 @@ def test_quads_autograd_identical(case, monkeypatch):
     say("quads autograd", case)
     valid = dev(c["valid"]).bool() if c["pad"] else None
     outs = []
-    for quads, dq_quads in SWITCHES:
-        monkeypatch.setattr(ops, "QUADS", quads)
-        monkeypatch.setattr(ops, "DQ_QUADS", dq_quads)
+    # the ratio of the default, below and above that of these lists, last
+    for quads, dq_quads, ratio in (*((*s, 2.0) for s in SWITCHES[:3]), (True, None, 3.0), (True, None, 1.0)):
+        names = _switched(monkeypatch, quads, dq_quads)
+        monkeypatch.setattr(ops, "DQ_QUAD_RATIO", ratio)
         q, k, v = (dev(c[n]).requires_grad_(True) for n in ("qh", "kh", "vh"))
         o = flash_attn_bsa_3d_dynamic(q, k, v, c["grid"], method="ivpq", sparsity=0.6, cdf_threshold=0.9,
                                       valid_mask=valid)
         plan = o.grad_fn.plan
-        want_dq = quads and dq_quads is not False
+        want_dq = quads and (dq_quads is True or dq_quads is None and ratio == 1.0)
         assert plan.lay.Nt % 4 == 0 and plan.quads == quads and plan.dq_quads == want_dq
         assert (plan.qquad is not None) == want_dq  # kept for the backward only when dQ walks it
         o.backward(torch.randn(o.shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(3))
                    .to(o.dtype))
+        _walked(names, quads, want_dq)
         outs.append([host(t) for t in (o, q.grad, k.grad, v.grad)])
     for other in outs[1:]:
         for name, a, b in zip(("O", "dQ", "dK", "dV"), outs[0], other):
@@ -158,13 +181,13 @@ def test_quads_uniform_and_cross_identical(monkeypatch):
         outs = []
         for quads, dq_quads in SWITCHES:
             say("quads", name, quads, dq_quads)
-            monkeypatch.setattr(ops, "QUADS", quads)
-            monkeypatch.setattr(ops, "DQ_QUADS", dq_quads)
+            names = _switched(monkeypatch, quads, dq_quads)
             q, k, v = (dev(a).requires_grad_(True) for a in arrays)
             o = fn(q, k, v)
             assert o.grad_fn.plan.quads == quads and o.grad_fn.plan.dq_quads == (quads and dq_quads is True), name
             o.backward(torch.randn(o.shape, device="cuda", generator=torch.Generator(device="cuda").manual_seed(4))
                        .to(o.dtype))
+            _walked(names, quads, quads and dq_quads is True)
             outs.append([host(t) for t in (o, q.grad, k.grad, v.grad)])
         for other in outs[1:]:
             for what, a, b in zip(("O", "dQ", "dK", "dV"), outs[0], other):
