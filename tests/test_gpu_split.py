@@ -149,6 +149,120 @@ def test_split_backward(shape):
             assert bits_equal(host(a), host(b)), name
 
 
+def _close(x, y, name):
+    """The same float32 products in another order of summation: as in
+    test_split_backward."""
+    x, y = x.float(), y.float()
+    assert bool(((x - y).abs() <= 2.0 ** -7 * x.abs() + 2.0 ** -10 * x.pow(2).mean().sqrt()).all()), name
+
+
+def _call(kind):
+    """(function of q, k, v; their tokens; sides that are split): a clip of 576
+    tiles, attended by itself, by 300 audio tokens, and attending to them."""
+    from prism_amd import flash_attn_bsa_3d_dynamic, flash_attn_bsa_cross
+    grid = (16, 32, 72)
+    S = grid[0] * grid[1] * grid[2]
+    if kind == "self":
+        return (lambda q, k, v: flash_attn_bsa_3d_dynamic(q, k, v, grid, method="ivpq", sparsity=0.9)), S, S, "qk"
+    if kind == "audio_queries":
+        return (lambda q, k, v: flash_attn_bsa_cross(q, k, v, "1d", "3d", k_grid_size=grid, sparsity=0.75)), 300, S, "q"
+    return (lambda q, k, v: flash_attn_bsa_cross(q, k, v, "3d", "1d", q_grid_size=grid, sparsity=0.5)), S, 300, "k"
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("kind", ["self", "audio_queries", "audio_keys"])
+def test_split_through_the_layers(kind, D, monkeypatch):
+    """A training step whose dQ and / or dK/dV is split, key lists beside the
+    forward or before it: the gradients of whole lists to the order of
+    summation, the same bits from both overlap settings, the forward's bits
+    untouched."""
+    from prism_amd import ops
+    fn, Sq, Sk, sides = _call(kind)
+    say("split layer", kind, D)
+    g = torch.Generator(device="cuda").manual_seed(11)
+    make_t = lambda S: torch.randn((1, 2, S, D), device="cuda", generator=g).to(torch.bfloat16)
+    q, k, v, do = make_t(Sq), make_t(Sk), make_t(Sk), make_t(Sq)
+
+    def step(overlap, split):
+        monkeypatch.undo()
+        monkeypatch.setattr(ops, "OVERLAP_SIDE_WORK", overlap)
+        if not split:
+            monkeypatch.setattr(ops, "split_plan", lambda kernel, heads, per_head, entries, D: (heads * per_head, 1))
+        names = called(monkeypatch)
+        x = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        o = fn(*x)
+        plan = o.grad_fn.plan
+        assert (plan._q.split is not None) == (split and "q" in sides)
+        assert (plan._k.split is not None) == (split and "k" in sides)
+        assert plan._q.source is None and plan._k.source is None
+        o.backward(do)
+        assert ("bsa_bwd_dq_split" in names) == (split and "q" in sides)
+        assert ("bsa_bwd_dkdv_split" in names) == (split and "k" in sides)
+        return [o.detach()] + [t.grad for t in x]
+
+    whole, apart, beside = step(True, False), step(False, True), step(True, True)
+    assert bits_equal(host(whole[0]), host(beside[0]))
+    for name, w, a, b in zip(("O", "dQ", "dK", "dV"), whole, apart, beside):
+        assert bits_equal(host(a), host(b)), name
+        _close(w, b, name)
+
+
+@pytest.mark.parametrize("D", [64, 128])
+def test_split_given_lists(D, monkeypatch):
+    """attn_bwd_bsa_varlen over lists long enough to be split, with key masks."""
+    from prism_amd import bsa_interface, ops
+    BH, Nt, W = 2, 514, 70
+    say("split given lists", D)
+    g = torch.Generator(device="cuda").manual_seed(12)
+    q, k, v, do = (torch.randn((1, BH, Nt * 64, D), device="cuda", generator=g).to(torch.bfloat16) for _ in range(4))
+    idx = torch.sort(torch.rand((1, BH, Nt, Nt), device="cuda", generator=g), -1).indices[..., :W]
+    idx, lens = torch.sort(idx, -1).values, torch.randint(0, W + 1, (1, BH, Nt), device="cuda", generator=g, dtype=torch.int32)
+    valid = torch.rand((Nt * 64,), device="cuda", generator=g) < 0.8
+    o, lse = bsa_interface.attn_fwd_bsa_varlen(q, k, v, 0.1, idx, lens, kv_valid_mask=valid)
+
+    def back():
+        out = [torch.empty_like(t) for t in (q, k, v)]
+        return bsa_interface.attn_bwd_bsa_varlen(do, q, k, v, o, *out, 0.1, lse, idx, lens, kv_valid_mask=valid)
+
+    names = called(monkeypatch)
+    split = back()
+    assert "bsa_bwd_dq_split" in names and "bsa_bwd_dkdv_split" in names
+    monkeypatch.setattr(ops, "split_plan", lambda kernel, heads, per_head, entries, D: (heads * per_head, 1))
+    names.clear()
+    for name, w, x in zip(("dQ", "dK", "dV"), back(), split):
+        _close(w, x, name)
+    assert "bsa_bwd_dq" in names and "bsa_bwd_dkdv" in names
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("grid,audio", [((7, 16, 16), 0), ((9, 30, 52), 0), ((7, 20, 24), 460)], ids=str)
+def test_small_and_large_launches_agree(grid, audio, D, monkeypatch):
+    """Single tiles and dense lists of small launches against pairs or quads
+    and compact or dense lists of large ones: the same output and gradients,
+    bit for bit (lists too short to be split)."""
+    from prism_amd import flash_attn_bsa_cross, ops
+    from prism_amd.adapter import run_bsa_uniform
+    S = grid[0] * grid[1] * grid[2]
+    say("small and large", grid, audio, D)
+    g = torch.Generator(device="cuda").manual_seed(13)
+    make_t = lambda n: torch.randn((1, 2, n, D), device="cuda", generator=g).to(torch.bfloat16)
+    q, k, v, do = make_t(audio or S), make_t(S), make_t(S), make_t(audio or S)
+    outs = []
+    for keep, compact in ((ops.KEEP_DENSE_BYTES, True), (-1, True), (-1, False)):
+        monkeypatch.setattr(ops, "KEEP_DENSE_BYTES", keep)
+        x = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        if audio:
+            o = flash_attn_bsa_cross(*x, "1d", "3d", k_grid_size=grid, sparsity=0.75)
+        else:
+            o = run_bsa_uniform(*x, grid, {"sparsity": 0.75, "cdf_threshold": 0.9, "compact_lists": compact})
+        assert o.grad_fn.plan._q.small == (keep > 0)
+        o.backward(do)
+        outs.append([host(t) for t in (o, *(t.grad for t in x))])
+    for other in outs[1:]:
+        for name, a, b in zip(("O", "dQ", "dK", "dV"), outs[0], other):
+            assert bits_equal(a, b), name
+
+
 def test_split_plan_covers_the_gpu():
     """split_plan cuts only launches of a few rounds over long lists, at a
     group boundary, and never makes more items than it has workgroups for
