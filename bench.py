@@ -387,35 +387,50 @@ def summarize_counters(fetch_csv, write_csv, calib_fetch_csv, calib_write_csv):
     print(json.dumps(out), flush=True)
 
 
-def staged_tile_bytes(plan, D: int) -> dict:
+def union_entries(plan) -> dict:
+    """Entries of the unions that the plan's kernels can walk, before settle():
+    query-side pairs and quads (None: the plan builds none), key-side pairs."""
+    count = lambda u: None if u is None else int(u[1].sum().item())
+    return {"pair": count(plan.qunion), "quad": count(plan.qquad), "key": count(plan.kunion)}
+
+
+def walked_unions(launched, entries: dict) -> dict:
+    """Which query-side unions the forward and dQ walked, by the entry points
+    that were launched; prism_bsa_fwd_either decides by the entries."""
+    fwd = {"prism_bsa_fwd": "pair", "prism_bsa_fwd_tile": "tile", "prism_bsa_fwd_quad": "quad",
+           "prism_bsa_fwd_either": "quad" if 2 * entries["pair"] >= 3 * (entries["quad"] or 0) else "pair"}
+    dq = {"prism_bsa_bwd_dq": "pair", "prism_bsa_bwd_dq_split": "split pair", "prism_bsa_bwd_dq_quad": "quad"}
+    one = lambda kinds: next((kind for name, kind in kinds.items() if name in launched), None)
+    return {"forward": one(fwd), "dq": one(dq)}
+
+
+def staged_tile_bytes(entries: dict, walked: dict, sum_lens: int, D: int) -> dict:
     """Bytes the attention kernels copy into LDS per launch: one 64 x D bf16
     tile of each operand per union entry (forward and dQ: K and V over the
-    query-side pair or quad unions; dK/dV: Q and dO plus the m2 and delta rows
-    over the key-side unions), whether the copy hits in L2 or not."""
+    query-side pair or quad unions, single tiles their own lists; dK/dV: Q and
+    dO plus the m2 and delta rows over the key-side unions), whether the copy
+    hits in L2 or not.  (Split launches stage their pairs' entries.)"""
     tile = 64 * D * 2
-    q_entries = int(plan.qunion[1].sum().item())
-    out = {"prism_bsa_fwd": 2 * tile * q_entries, "prism_bsa_bwd_dq": 2 * tile * q_entries}
-    quad = getattr(plan, "qquad", None)
-    if quad is not None:
-        quad_entries = int(quad[1].sum().item())
-        out.update({"prism_bsa_fwd_quad": 2 * tile * quad_entries, "prism_bsa_bwd_dq_quad": 2 * tile * quad_entries})
-    if plan.kunion is not None:
-        out["prism_bsa_bwd_dkdv"] = (2 * tile + 2 * 64 * 4) * int(plan.kunion[1].sum().item())
+    by_kind = {"pair": entries["pair"], "split pair": entries["pair"], "quad": entries["quad"], "tile": sum_lens}
+    out = {}
+    for names, kind in ((("prism_bsa_fwd", "prism_bsa_fwd_tile", "prism_bsa_fwd_quad", "prism_bsa_fwd_either"), "forward"),
+                        (("prism_bsa_bwd_dq", "prism_bsa_bwd_dq_split", "prism_bsa_bwd_dq_quad"), "dq")):
+        if walked[kind] is not None:
+            out.update({n: 2 * tile * by_kind[walked[kind]] for n in names})
+    if entries["key"] is not None:
+        out.update({n: (2 * tile + 2 * 64 * 4) * entries["key"] for n in ("prism_bsa_bwd_dkdv", "prism_bsa_bwd_dkdv_split")})
     return out
 
 
-def slot_efficiency(plan, sum_lens: int) -> dict:
+def slot_efficiency(entries: dict, walked: dict, sum_lens: int) -> dict:
     """Fraction of the wave-tile slots of the forward and dQ kernels that do
     math: Σlens over (tiles per union) x (union entries), for the pair unions
     and, when the plan has them, the quad unions; and which unions the
-    forward and dQ launches of the plan walk."""
-    pair = sum_lens / max(1, 2 * int(plan.qunion[1].sum().item()))
-    quad = getattr(plan, "qquad", None)
-    qeff = None if quad is None else sum_lens / max(1, 4 * int(quad[1].sum().item()))
-    walk = {"forward": "quad" if getattr(plan, "quads", False) else "pair",
-            "dq": "quad" if getattr(plan, "dq_quads", False) else "pair"}
-    return {"union_slot_efficiency": round(pair, 4),
-            "quad_union_slot_efficiency": None if qeff is None else round(qeff, 4), "query_unions": walk}
+    forward and dQ launches walked."""
+    quad = entries["quad"]
+    return {"union_slot_efficiency": round(sum_lens / max(1, 2 * entries["pair"]), 4),
+            "quad_union_slot_efficiency": None if quad is None else round(sum_lens / max(1, 4 * quad), 4),
+            "query_unions": walked}
 
 
 def measured_traffic(kernel: str):
@@ -531,7 +546,8 @@ def measured_ceilings():
         "copy_GBps": round(2 * nbytes / (c_ms * 1e-3) / 1e9, 1), "copy": "prism_copy_peak, 4 GiB read + 4 GiB written",
         "tile_stream_TBps": round(stream_cache, 2), "tile_stream_hbm_TBps": round(stream_hbm, 2),
         "tile_stream": "prism_tile_stream_peak: 32 KB stages of two random 16 KB tiles into LDS, the forward's copy "
-                       "plan, no math; over 189 MB (Infinity Cache) and over 4 GiB (HBM)",
+                       "plan, no math; over 189 MB (Infinity Cache) and over 4 GiB (HBM); a yardstick, no ceiling: "
+                       "tiles that several workgroups list at one time come from the L2",
         "cus": cus,
     }
 
@@ -668,8 +684,8 @@ def main():
                             compact_lists=compact, keep_scores=True)
         plan.build_key_lists()
     # bytes of work lists at their peak (all lists of the call) and those the
-    # step keeps from its forward to its backward (the two pair unions, after
-    # the forward's settle(), as _DynBSA.forward does)
+    # step keeps from its forward to its backward (after the forward's settle(),
+    # as _DynBSA.forward does): unions, pairings and launch orders
     list_bytes_peak = plan.list_bytes()
     sum_lens = plan.sum_lens()
     Nt, Nb, Sp = plan.lay.Nt, plan.lay.N_b, plan.S
@@ -689,8 +705,10 @@ def main():
     X = B * H * Sp * D * 2   # one bf16 [B,H,S_p,D] tile-order tensor (zone grid)
     Xin = B * H * S * D * 2  # one bf16 [B,H,S,D] THW tensor (input grid)
     nnz_tiles = int(plan.sel["ntiles"].sum().item())
-    slots = slot_efficiency(plan, sum_lens)
-    staged = staged_tile_bytes(plan, D)
+    entries = union_entries(plan)
+    walked = walked_unions(kt, entries)
+    slots = slot_efficiency(entries, walked, sum_lens)
+    staged = staged_tile_bytes(entries, walked, sum_lens, D)
     with torch.no_grad():
         plan.settle()
     list_bytes = plan.list_bytes()
@@ -1050,10 +1068,12 @@ def run_uniform(args, inp):
         plan = plan_chunked(q.detach(), k.detach(), v.detach(), lq, lq, sparsity=sparsity, cdf_threshold=cdf,
                             sm_scale=1 / math.sqrt(D))
     sum_lens = plan.sum_lens()
-    slots = slot_efficiency(plan, sum_lens)
     with torch.no_grad():
         plan.key_lists()
-    staged = staged_tile_bytes(plan, D)
+    entries = union_entries(plan)
+    walked = walked_unions(kt, entries)
+    slots = slot_efficiency(entries, walked, sum_lens)
+    staged = staged_tile_bytes(entries, walked, sum_lens, D)
     fl = 64 * 64 * D * sum_lens
     kept_flops = 14 * fl
     attn = {"prism_bsa_fwd": (4 * fl, 4 * fl), "prism_bsa_bwd_dkdv": (8 * fl, 8 * fl),
