@@ -405,16 +405,22 @@ __global__ __launch_bounds__(kGatherThreads) void scatter_rows_kernel(const uint
 // 0.256 ms, 4: 0.283, 8: 0.326 averaged over a step's launches at 302,400 tokens
 // x 5 heads), else 4.  Launches of few units leave about a wave per SIMD: there
 // a wave takes 64 rows (32 without pooling) and keeps them all in flight.  The
-// lines lie where both sides cost the same (bf16, D = 128, us at 280 / 540 /
-// 1,215 units x heads, few and many rows per wave): pooling 28 / 45 / 105 and
-// 32 / 51 / 61, gather 14 / 24 / 59 and 26 / 45 / 55, scatter 14 / 43 / 91 and
-// 22 / 38 / 59.
-constexpr int64_t kFewPools = 768, kFewGathers = 1024, kFewScatters = 400;
+// lines lie where both sides cost the same with bf16 rows of D = 128 (us at 280
+// / 360 / 480 / 810 / 1,215 units x heads, few and many rows per wave): pooling
+// 27 / 32 / 36 / 59 / 110 and 30 / 31 / 32 / 40 / 65, gather 13 / 19 / 23 / 35 / 66
+// and 25 / 27 / 29 / 36 / 62, scatter 14 / 28 / 39 / 71 / 101 and 28 / 30 / 32 / 38
+// / 66.  Pooling at D = 64 crosses at 720 (bf16 23 and 23, fp32 28 and 27) and
+// with fp32 rows of D = 128 at 360 (32 and 31).  Elsewhere few rows are no slower
+// on either side of the line (fp32 gathers at 1,215: 92 and 99, with row dots 125
+// and 133; fp32 scatters at 480: 30 and 32, at D = 64 18 and 19).
+template <int D>
+constexpr int64_t kFewPools = D == 128 ? 360 : 720;
+constexpr int64_t kFewGathers = 1024, kFewScatters = 400;
 
 template <int D, typename T, typename Map>
 void launch_gather_t(const GatherArgs& a, const Map& m, dim3 grid, hipStream_t stream) {
   const bool pool = a.block_mean != nullptr || a.block_count != nullptr || a.tile_count != nullptr;
-  if ((int64_t)grid.x * grid.y < (pool ? kFewPools : kFewGathers)) {
+  if ((int64_t)grid.x * grid.y < (pool ? kFewPools<D> : kFewGathers)) {
     if (pool) gather_pool_kernel<D, T, Map, true, D / 8, 64><<<dim3(2 * grid.x, grid.y), kGatherThreads, 0, stream>>>(a, m);
     else gather_pool_kernel<D, T, Map, false, D / 16, 32><<<dim3(4 * grid.x, grid.y), kGatherThreads, 0, stream>>>(a, m);
   } else {
