@@ -628,10 +628,12 @@ def part_union(start: torch.Tensor, length: torch.Tensor, cols: torch.Tensor, Nt
 
 
 def launch_order(ulen: torch.Tensor, heads: int, cache_bytes: int, chunk: int = 1):
-    """(order int32 [n], total int64 [1]) of an attention launch over the lists
-    of `heads` heads: each head's lists longest first, or all heads' together
-    when the operands they read (cache_bytes) fit the Infinity Cache; total is
-    the sum of the lengths (prism_launch_order)."""
+    """(order int32 [n], total int64 [1]) of an attention launch over the n
+    lists of `heads` heads: runs of ceil(n / heads) consecutive lists (a head's;
+    of a split launch, whose heads may differ in items, about a head's) longest
+    first, or all of them as one run when the operands that they read
+    (cache_bytes) fit the Infinity Cache; total is the sum of the lengths
+    (prism_launch_order)."""
     _cuda(ulen)
     n = ulen.numel()
     seg = n if n <= SEGMENT_MAX and cache_bytes <= CACHE_BYTES else -(-n // heads)
@@ -643,9 +645,16 @@ def launch_order(ulen: torch.Tensor, heads: int, cache_bytes: int, chunk: int = 
 # ranks per XCD run of the pair forward's launch order
 FWD_CHUNK = 64
 SEGMENT_MAX = 16384
-# 256 MB of Infinity Cache; the launches' padded tiles are never read, so a
-# little more than that may pass (171,360 tokens of 3 heads, 318 MB with the
-# padding and 263 without, gain from one sorted run)
+# About the Infinity Cache (256 MB; padded tiles are never read).  One run over
+# all heads against one per head, dQ over pairs, ms, at 270 / 304 / 360 / 405 /
+# 540 / 900 MB of K and V: lists of a cumulative threshold (lengths vary widely)
+# 6.58, 7.30 / 12.8, 14.0 / 24.1, 24.8 / 17.4, 18.4 / 36.1, 35.4 / 64.2, 59.0;
+# top-k lists (lengths nearly equal) 3.51, 3.45 / 8.61, 8.34 / 18.6, 18.0 /
+# 11.9, 11.0 / 29.3, 26.9 / 51.4, 44.5: the line lies where the one kind gains
+# what the other loses.  The pair forward, whose runs are dealt in chunks, has it
+# lower for top-k lists (2.0, 1.9 at 180 MB, 7.6, 7.1 at 304) and about here for
+# the others (4.0, 4.0 at 180; 11.5, 11.6 at 304, and 11.3, 12.4 with audio
+# norms; 15.5, 14.3 at 405).
 CACHE_BYTES = 320 << 20
 
 
