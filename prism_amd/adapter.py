@@ -78,9 +78,9 @@ class DynamicBlockSparseAttention:
     """State the reference keeps on SelfAttention for the dynamic path: the
     bsa_params dict, the method switch and the per-pass shape cache
     (wan_video_dit.py:22-33, :401-427).  One key beyond the reference's:
-    bsa_params["compact_lists"] (default True) keeps the work lists in
-    compact CSR form until the backward (O(nnz) memory; identical results;
-    False: dense buffers)."""
+    bsa_params["compact_lists"] (default True) keeps the work lists of a long
+    launch in compact CSR form until the backward (O(nnz) memory; identical
+    results; False: dense buffers, as a short launch's always are)."""
 
     def __init__(self, method: str = "ivpq", bsa_params: Optional[dict] = None):
         if method not in ("ivpq", "penalty"):

@@ -21,6 +21,10 @@
 // 490 us, dK/dV of 80 pairs of 180 entries 659 -> 255 us, dQ of 2,160 pairs of
 // 180 entries 2,002 -> 1,875 us.
 //
+// The workspace lives for the two launches: items x 128 x D floats for dQ, twice
+// that for dK/dV; by the rule below at most 237 MB at D = 128 (the last 514 of
+// 4,095 pairs of dQ, 258 of 1,791 of dK/dV, in seven items each).
+//
 // The forward is not split: its O would differ in its last bits, and delta =
 // rowsum(O dO) carries such a bit into a whole row of dQ.
 #pragma once

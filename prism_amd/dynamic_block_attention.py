@@ -206,11 +206,12 @@ def flash_attn_bsa_3d_dynamic(
     kernels; the result equals padding first and slicing after, bit for bit.
 
     When gradients are needed, the forward releases the per-tile lists once
-    the backward's pair unions exist.  compact_lists (not in the reference's
-    signature; default True) keeps those unions in compact CSR form until
-    the backward (O(nnz) memory, one host read of their sizes made while the
-    forward kernel runs); False keeps them as dense pairs x Nt buffers.
-    Results are identical either way."""
+    the backward's lists exist.  compact_lists (not in the reference's
+    signature; default True) keeps those of a long launch in compact CSR form
+    until the backward (O(nnz) memory, one host read of their sizes made while
+    the forward kernel runs); False keeps them as dense pairs x Nt buffers.  A
+    short launch's (fewer than eight rounds of workgroups) are kept dense either
+    way, about 32 MB a side at most.  Results are identical either way."""
     plan = plan_dynamic(q, k, v, grid_padded, method=method, sparsity=sparsity, cdf_threshold=cdf_threshold,
                         audio_token_norms=audio_token_norms, valid_mask=valid_mask, lambda_a=lambda_a,
                         tau_128=tau_128, lambda_128=lambda_128, shape_ids=shape_ids,

@@ -593,10 +593,14 @@ def bsa_fwd(q, k, v, tmasks, qunion, sm_scale: float, qpair: Optional[torch.Tens
     return _op("bsa_fwd", q, k, v, tmasks, ustart, ulen, ucols, qpair, qorder, float(sm_scale))
 
 
-# Query-side launches of fewer pairs than SPLIT_PAIRS (eight rounds of the 512
-# workgroups that the pair forward and dQ kernels keep resident) walk pairs, dQ
-# and dK/dV with split lists where they pay; forward launches of at most
-# TILE_PAIRS (one tile per CU) walk single tiles.
+# A launch of fewer pairs than SPLIT_PAIRS (eight rounds of the 512 workgroups
+# that the pair forward and dQ kernels keep resident; dK/dV keeps 256) is short:
+# the forwards of at most TILE_PAIRS pairs (one tile per CU) walk single tiles,
+# and dQ and dK/dV split lists where split_plan says so.  Over given lists the
+# number of pairs decides alone; a plan also asks that a short side's lists be
+# small (KEEP_DENSE_BYTES), and treats it as a long one otherwise: one head at
+# 369,000 padded tokens has 2,880 pairs and 133 MB of lists, walks pairs or quads
+# and splits nothing.
 SPLIT_PAIRS = 4096
 TILE_PAIRS = 128
 # A side of a few rounds whose per-tile lists and whose pair unions, twice over,
@@ -740,9 +744,10 @@ OVERLAP_DKDV_SCATTER = False
 # quad unions (bsa_bwd_dq_quad, bit-identical to bsa_bwd_dq; the plan then
 # keeps them for the backward): DQ_QUADS None (the default) takes it on the
 # dynamic-shape path where the pair unions hold at least DQ_QUAD_RATIO times
-# the quad unions' entries (known on the host when a compact plan settles),
-# and not on the uniform and cross paths; True / False (PRISM_DQ_QUADS=1 / 0)
-# force it on launches of eight rounds.  Pair over quad entries, dQ on pairs
+# the quad unions' entries (known on the host when a compact plan settles; a plan
+# of dense lists keeps dQ on pairs, whole steps within 0.5% of the choice on
+# every kind of list tried), and not on the uniform and cross paths; True / False
+# (PRISM_DQ_QUADS=1 / 0) force it on long launches.  Pair over quad entries, dQ on pairs
 # and quads (ms): 1.20: 55.5, 62.3; 1.39: 31.9, 33.2; 1.65: 60.6, 60.9; 1.72:
 # 79.2, 76.8.
 DQ_QUAD_RATIO = 1.68

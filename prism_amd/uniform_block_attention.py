@@ -133,8 +133,8 @@ def plan_chunked(q, k, v, lq: ops.ChunkLayout, lk: ops.ChunkLayout, *, sparsity,
                  compact_lists=False) -> _ChunkPlan:
     """Selection half of the uniform path (no attention).  keep_scores keeps
     the fp32 chunk scores on the plan (plan.scores) for inspection;
-    compact_lists makes plan.settle() keep the pair unions in compact CSR
-    form (O(nnz) memory)."""
+    compact_lists makes plan.settle() keep the pair unions of a long launch in
+    compact CSR form (O(nnz) memory)."""
     if sparsity is None and cdf_threshold is None:
         raise ValueError("Either sparsity or cdf_threshold must be provided")
     with torch.no_grad():
