@@ -362,7 +362,7 @@ def summarize_counters(fetch_csv, write_csv, calib_fetch_csv, calib_write_csv):
     COPY_BYTES reads and writes exactly COPY_BYTES."""
     names = {"bsa_fwd_kernel": "prism_bsa_fwd", "bsa_bwd_dkdv_kernel": "prism_bsa_bwd_dkdv",
              "bsa_bwd_dq_kernel": "prism_bsa_bwd_dq", "bsa_fwd_quad_kernel": "prism_bsa_fwd_quad",
-             "bsa_bwd_dq_quad_kernel": "prism_bsa_bwd_dq_quad", "select_kernel": "prism_select_tiles",
+             "bsa_bwd_dq_quad_kernel": "prism_bsa_bwd_dq_quad", "select_rows_kernel": "prism_select_tiles",
              "gather_pool_kernel": "prism_gather_pool", "scatter_rows_kernel": "prism_scatter_rows",
              "block_scores_kernel": "prism_block_scores", "a2v_norms_kernel": "prism_a2v_norms",
              "zone_stats_kernel": "prism_zone_stats", "pair_union_kernel": "prism_pair_union"}
@@ -379,6 +379,8 @@ def summarize_counters(fetch_csv, write_csv, calib_fetch_csv, calib_write_csv):
         if entry is None or k not in write:
             continue
         fb, wb = fv * 1024.0 * f_scale, write[k] * 1024.0 * w_scale
+        if fb + wb < 1e6:
+            continue  # the kernel of prism_bsa_fwd_either that returned at once
         out["kernels"][entry] = {"fetch_bytes": round(fb), "write_bytes": round(wb),
                                  "hbm_bytes_per_launch": round(fb + wb)}
     os.makedirs(os.path.dirname(TRAFFIC_FILE), exist_ok=True)
