@@ -416,6 +416,14 @@ __global__ __launch_bounds__(kGatherThreads) void scatter_rows_kernel(const uint
 template <int D>
 constexpr int64_t kFewPools = D == 128 ? 360 : 720;
 constexpr int64_t kFewGathers = 1024, kFewScatters = 400;
+// LDS that a launch with row dots of more than one round asks for and does not
+// use: it reads two streams and writes a third, and seven workgroups of a CU (71
+// VGPRs) disturb each other's lines where six do not (bf16, D = 128, 302,400 tokens
+// x 5 heads: 315 -> 295 us; 2,025 to 4,320 units x heads, both types and D: 0 to 7%
+// faster; a launch that seven hold at once, 1,620 units x heads, would take 165 us
+// for 136)
+constexpr unsigned kDotLds = 26 * 1024;
+constexpr int64_t kDotRound = 7 * 256;
 
 template <int D, typename T, typename Map>
 void launch_gather_t(const GatherArgs& a, const Map& m, dim3 grid, hipStream_t stream) {
@@ -425,7 +433,10 @@ void launch_gather_t(const GatherArgs& a, const Map& m, dim3 grid, hipStream_t s
     else gather_pool_kernel<D, T, Map, false, D / 16, 32><<<dim3(4 * grid.x, grid.y), kGatherThreads, 0, stream>>>(a, m);
   } else {
     if (pool) gather_pool_kernel<D, T, Map, true, 2, 128><<<grid, kGatherThreads, 0, stream>>>(a, m);
-    else gather_pool_kernel<D, T, Map, false, 4, 128><<<grid, kGatherThreads, 0, stream>>>(a, m);
+    else {
+      const unsigned lds = a.rowdot && (int64_t)grid.x * grid.y > kDotRound ? kDotLds : 0;
+      gather_pool_kernel<D, T, Map, false, 4, 128><<<grid, kGatherThreads, lds, stream>>>(a, m);
+    }
   }
 }
 template <typename Map>

@@ -288,8 +288,9 @@ __global__ __launch_bounds__(1024) void pair_order_kernel(const int32_t* __restr
 // quarter sorted), 302,400 tokens, 5 heads: pair forward 54.0 -> 51.7 ms, dQ
 // 58.0 -> 55.5, quad forward 52.5 -> 51.8; 171,360 tokens, 3 heads: 12.4 ->
 // 11.4, 13.9 -> 13.2, 12.7 -> 11.4 ms.  Sorting all heads together takes
-// another 7% off dQ there but costs 10% and more once the heads' K and V
-// outgrow the Infinity Cache (the caller picks seg).
+// another 7% off dQ there (lists of a cumulative threshold; top-k lists, nearly
+// of one length, lose 3%) but costs 10% and more once the heads' K and V outgrow
+// the Infinity Cache (the caller picks seg).
 // With chunk > 1, runs of `chunk` consecutive ranks go to one XCD (launch
 // position b runs on XCD b mod 8), every second round of XCDs in reverse so
 // that no XCD gets all the long lists: the workgroups of one L2 then walk
