@@ -350,72 +350,78 @@ __global__ __launch_bounds__(kGatherThreads) void gather_pool_kernel(GatherArgs 
   }
 }
 
-// grid (units x 128 / RPW, B*H): tile-order bf16 rows (S_out per head) -> THW
-// rows of dtype TO (S_in per head); padding rows are dropped.  Each lane moves
-// 16 bytes (8 channels): a wave instruction covers 64 / (D / 8) rows, NB
-// instructions are in flight per wave, and a wave takes RPW rows.
-template <int D, typename TO, typename Map, int NB, int RPW>
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+// grid (units x 4, B*H): tile-order bf16 rows (S_out per head) -> THW rows of
+// dtype TO (S_in per head); padding rows are dropped.  Each lane moves 16 bytes (8
+// channels): a wave instruction covers 64 / (D / 8) rows, and a wave takes 32 rows
+// with all their loads in flight.  HBM bounds it, and short launches the latency
+// of one load and one store.  A lane whose row is padding loads the head's row 0:
+// under a branch, or as uint4 (a class type), the compiler keeps bf16 rows in
+// flight in LDS (16 KB per workgroup), in scratch or in up to 256 VGPRs; loaded by
+// all lanes they take 30 to 60.  us at 64 / 360 / 1,215 / 2,025 / 3,240 units x
+// heads, bf16, D = 128: 7.1 / 28.9 / 64 / 114 / 178 with the rows in LDS or scratch,
+// 6.1 / 15.1 / 55 / 96 / 152 so.  128 rows per wave, 4 instructions in flight, take
+// 8.6 / 15.9 / 57 / 105 / 166 and are no faster with fp32 outputs (109 and 97 at
+// 1,215) or D = 64 (26 and 25) either; they win by 3% at most (fp32, D = 128, 240
+// units x heads: 17.2 and 17.8).
+template <int D, typename TO, typename Map>
 __global__ __launch_bounds__(kGatherThreads) void scatter_rows_kernel(const uint16_t* __restrict__ in, int64_t S_in,
                                                                       int64_t S_out, Map m, TO* __restrict__ out) {
   constexpr int LPR = D / 8;     // lanes per row
   constexpr int RPI = 64 / LPR;  // rows per wave instruction
-  constexpr int RB = RPI * NB;   // rows per batch
-  static_assert(64 % RB == 0 && RPW % RB == 0, "batches must not straddle blocks");
+  constexpr int NB = 32 / RPI;   // wave instructions in flight
   const int bh = blockIdx.y;
   const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int sub = lane / LPR, c8 = (lane % LPR) * 8;
-  constexpr int SUBS = 128 / RPW;  // workgroups per unit
-  m.init(blockIdx.x / SUBS);
-  const int r0 = (int)(blockIdx.x % SUBS) * 4 * RPW + wid * RPW;
+  m.init(blockIdx.x / 4);
+  const int r0 = (int)(blockIdx.x % 4) * 128 + wid * 32;
   if (!m.live(r0)) return;
   const uint16_t* inh = in + (int64_t)bh * S_out * D + c8;
   TO* outh = out + (int64_t)bh * S_in * D + c8;
-  for (int o0 = 0; o0 < RPW; o0 += RB) {
-    uint4 v[NB];
-    int64_t tok[NB];
-    if (RPW < 128 || (o0 & 63) == 0) m.group((r0 + o0) & ~63);
+  u32x4 v[NB];
+  int64_t tok[NB];
+  m.group(r0 & ~63);
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      const int r = r0 + o0 + b * RPI + sub;
-      tok[b] = m.g.token(r & 63);
-      if (tok[b] >= 0) v[b] = *reinterpret_cast<const uint4*>(inh + m.row(r) * D);
-    }
+  for (int b = 0; b < NB; ++b) {
+    const int r = r0 + b * RPI + sub;
+    tok[b] = m.g.token(r & 63);
+    v[b] = *reinterpret_cast<const u32x4*>(inh + (tok[b] < 0 ? 0 : m.row(r)) * D);
+  }
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-      if (tok[b] < 0) continue;
-      TO* dst = outh + tok[b] * D;
-      if (sizeof(TO) == 2) {
-        *reinterpret_cast<uint4*>(dst) = v[b];
-      } else {
-        const uint32_t w[4] = {v[b].x, v[b].y, v[b].z, v[b].w};
-        float4 lo, hi;
-        lo.x = __uint_as_float(w[0] << 16); lo.y = __uint_as_float(w[0] & 0xffff0000u);
-        lo.z = __uint_as_float(w[1] << 16); lo.w = __uint_as_float(w[1] & 0xffff0000u);
-        hi.x = __uint_as_float(w[2] << 16); hi.y = __uint_as_float(w[2] & 0xffff0000u);
-        hi.z = __uint_as_float(w[3] << 16); hi.w = __uint_as_float(w[3] & 0xffff0000u);
-        reinterpret_cast<float4*>(dst)[0] = lo;
-        reinterpret_cast<float4*>(dst)[1] = hi;
-      }
+  for (int b = 0; b < NB; ++b) {
+    if (tok[b] < 0) continue;
+    TO* dst = outh + tok[b] * D;
+    if (sizeof(TO) == 2) {
+      *reinterpret_cast<u32x4*>(dst) = v[b];
+    } else {
+      const uint32_t w[4] = {v[b].x, v[b].y, v[b].z, v[b].w};
+      float4 lo, hi;
+      lo.x = __uint_as_float(w[0] << 16); lo.y = __uint_as_float(w[0] & 0xffff0000u);
+      lo.z = __uint_as_float(w[1] << 16); lo.w = __uint_as_float(w[1] & 0xffff0000u);
+      hi.x = __uint_as_float(w[2] << 16); hi.y = __uint_as_float(w[2] & 0xffff0000u);
+      hi.z = __uint_as_float(w[3] << 16); hi.w = __uint_as_float(w[3] & 0xffff0000u);
+      reinterpret_cast<float4*>(dst)[0] = lo;
+      reinterpret_cast<float4*>(dst)[1] = hi;
     }
   }
 }
 
-// Rows per wave and wave instructions in flight.  Launches that fill the GPU
-// hide the latency with other waves: 128 rows, 2 instructions with pooling (2:
+// The gathers' rows per wave and wave instructions in flight.  Launches that fill
+// the GPU hide the latency with other waves: 128 rows, 2 instructions with pooling (2:
 // 0.256 ms, 4: 0.283, 8: 0.326 averaged over a step's launches at 302,400 tokens
 // x 5 heads), else 4.  Launches of few units leave about a wave per SIMD: there
 // a wave takes 64 rows (32 without pooling) and keeps them all in flight.  The
 // lines lie where both sides cost the same with bf16 rows of D = 128 (us at 280
 // / 360 / 480 / 810 / 1,215 units x heads, few and many rows per wave): pooling
 // 27 / 32 / 36 / 59 / 110 and 30 / 31 / 32 / 40 / 65, gather 13 / 19 / 23 / 35 / 66
-// and 25 / 27 / 29 / 36 / 62, scatter 14 / 28 / 39 / 71 / 101 and 28 / 30 / 32 / 38
-// / 66.  Pooling at D = 64 crosses at 720 (bf16 23 and 23, fp32 28 and 27) and
-// with fp32 rows of D = 128 at 360 (32 and 31).  Elsewhere few rows are no slower
-// on either side of the line (fp32 gathers at 1,215: 92 and 99, with row dots 125
-// and 133; fp32 scatters at 480: 30 and 32, at D = 64 18 and 19).
+// and 25 / 27 / 29 / 36 / 62.  Pooling at D = 64 crosses at 720 (bf16 23 and 23,
+// fp32 28 and 27) and with fp32 rows of D = 128 at 360 (32 and 31).  Elsewhere few
+// rows are no slower on either side of the line (fp32 gathers at 1,215: 92 and 99,
+// with row dots 125 and 133).
 template <int D>
 constexpr int64_t kFewPools = D == 128 ? 360 : 720;
-constexpr int64_t kFewGathers = 1024, kFewScatters = 400;
+constexpr int64_t kFewGathers = 1024;
 // LDS that a launch with row dots of more than one round asks for and does not
 // use: it reads two streams and writes a third, and seven workgroups of a CU (71
 // VGPRs) disturb each other's lines where six do not (bf16, D = 128, 302,400 tokens
@@ -450,25 +456,17 @@ void launch_gather(const GatherArgs& a, const Map& m, int dtype, int D, dim3 gri
   }
 }
 
-template <int D, typename TO, typename Map>
-void launch_scatter_t(const uint16_t* in, int64_t S_in, int64_t S_out, const Map& m, TO* out, dim3 grid,
-                      hipStream_t stream) {
-  if ((int64_t)grid.x * grid.y < kFewScatters)
-    scatter_rows_kernel<D, TO, Map, D / 16, 32><<<dim3(4 * grid.x, grid.y), kGatherThreads, 0, stream>>>(in, S_in,
-                                                                                                       S_out, m, out);
-  else
-    scatter_rows_kernel<D, TO, Map, 4, 128><<<grid, kGatherThreads, 0, stream>>>(in, S_in, S_out, m, out);
-}
 template <typename Map>
 void launch_scatter(const void* in_rows, int64_t S_in, int64_t S_out, const Map& m, void* out, int out_dtype, int D,
                     dim3 grid, hipStream_t stream) {
   const uint16_t* in = (const uint16_t*)in_rows;
+  grid.x *= 4;
   if (out_dtype == PRISM_BF16) {
-    if (D == 128) launch_scatter_t<128>(in, S_in, S_out, m, (uint16_t*)out, grid, stream);
-    else launch_scatter_t<64>(in, S_in, S_out, m, (uint16_t*)out, grid, stream);
+    if (D == 128) scatter_rows_kernel<128, uint16_t><<<grid, kGatherThreads, 0, stream>>>(in, S_in, S_out, m, (uint16_t*)out);
+    else scatter_rows_kernel<64, uint16_t><<<grid, kGatherThreads, 0, stream>>>(in, S_in, S_out, m, (uint16_t*)out);
   } else {
-    if (D == 128) launch_scatter_t<128>(in, S_in, S_out, m, (float*)out, grid, stream);
-    else launch_scatter_t<64>(in, S_in, S_out, m, (float*)out, grid, stream);
+    if (D == 128) scatter_rows_kernel<128, float><<<grid, kGatherThreads, 0, stream>>>(in, S_in, S_out, m, (float*)out);
+    else scatter_rows_kernel<64, float><<<grid, kGatherThreads, 0, stream>>>(in, S_in, S_out, m, (float*)out);
   }
 }
 

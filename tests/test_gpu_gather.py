@@ -1,6 +1,7 @@
-"""The gathers and scatters of launches of few workgroups (64 or 32 rows per
-wave) against those that fill the GPU (128 rows per wave): the same heads once
-a few at a time and once repeated past the line between the two, bit for bit.
+"""The gathers of launches of few workgroups (64 or 32 rows per wave) against
+those that fill the GPU (128 rows per wave), and the scatters (32 rows per wave) of
+both: the same heads once a few at a time and once repeated past the line between
+the two, bit for bit.
 Every candidate shape, grids with padding, a valid mask, chunks of 64 and 128
 tokens with row padding (an odd number of 64-row tiles)."""
 import numpy as np
